@@ -88,7 +88,7 @@ def draw(rng):
         more.update(rheology=rng.choice(("maxwell", "powerlaw", "powerlaw", "burgers", "afterslip")),
                     patches=rng.randint(1, 23), steps=rng.randint(3, 12), dt=0.005)
         if more["rheology"] == "afterslip":
-            more.update(patches=1, dt=0.002)
+            more.update(patches=1, dt=0.002, dx2=dx)
         more["steps"] = max(1, min(more["steps"], 2 ** 27 // (n1 * n2 * n3)))
     elif kind == "request":
         more.update(rheology=rng.choice(("maxwell", "powerlaw")), patches=rng.randint(1, 9), steps=rng.randint(3, 19))
@@ -152,11 +152,12 @@ def spec(c, seed, member=0):
     else:
         # a creeping plane down dip of a thrust rupture
         s["nonlinear"] = [(lid, workloads.gdot0(1e18, 3.5), 3.5, 0.0, 0.6, 0.0)]
-        dip, width = 20.0, 0.25 * deep
+        dip, width = 20.0, round(0.125 * c["n3"]) * dx
+        long = 2 * round(0.15 * half / dx) * dx
         down = width * math.sin(math.radians(dip)), width * math.cos(math.radians(dip))
-        s["deck"] = [(rng.uniform(0.1e-3, 0.5e-3), -0.25 * half, 0.0, 0.0, 0.5 * half, width, 0.0, dip, 90.0)]
-        s["planes"] = [dict(x=-0.5 * half, y=-down[1], z=down[0], length=half, width=2 * width, strike=0.0, dip=dip,
-                            rake=90.0)]
+        s["deck"] = [(rng.uniform(3e-5, 1.2e-4) * width, -0.25 * half, 0.0, 0.0, 0.5 * half, width, 0.0, dip, 90.0)]
+        s["planes"] = [dict(x=-long / 2, y=-down[1], z=down[0], length=long, width=width, strike=0.0, dip=dip,
+                            rake=-90.0)]
         s["friction"] = [(0.0, 1e-3, 1.0, 0.0, 0.6, 0.0)]
     # observation points on grid points of the top half
     i = np.stack([rng.integers(0, n, POINTS) for n in (c["n1"], c["n2"], c["n3"] // 2)], 1)
