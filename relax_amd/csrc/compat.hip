@@ -8,7 +8,9 @@
 #include <algorithm>
 #include <functional>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -442,15 +444,40 @@ int fftn_padded(float* d, int n1, int n2, int nz, double dx1, double dx2, double
 }
 
 // host <-> device copies between the reference layout (padded rows of n1+2 or
-// packed rows of n1) and the device's padded layout
+// packed rows of n1) and the device's padded layout.  Packed rows go through
+// blocks of at most 4 MB that the host repacks: a pitched copy of pageable
+// memory goes row by row in the runtime, 7 us each.
+size_t block_rows(int n1, long rows) {
+  return (size_t)std::max(1L, std::min(rows, (4L << 20) / (long)((n1 + 2) * sizeof(float))));
+}
 int put_real(float* dev, const float* host, int n1, long rows, int align) {
-  if (align) HIP_TRY(hipMemcpy(dev, host, (size_t)(n1 + 2) * rows * 4, hipMemcpyHostToDevice));
-  else HIP_TRY(hipMemcpy2D(dev, (n1 + 2) * 4, host, n1 * 4, n1 * 4, rows, hipMemcpyHostToDevice));
+  if (align) {
+    HIP_TRY(hipMemcpy(dev, host, (size_t)(n1 + 2) * rows * 4, hipMemcpyHostToDevice));
+    return RELAX_OK;
+  }
+  const size_t ld = n1 + 2, nb = block_rows(n1, rows);
+  std::unique_ptr<float[]> block(new (std::nothrow) float[nb * ld]());
+  if (!block) return RELAX_ERR_NOMEM;
+  for (size_t r0 = 0; r0 < (size_t)rows; r0 += nb) {
+    const size_t n = std::min(nb, (size_t)rows - r0);
+    for (size_t r = 0; r < n; ++r) std::memcpy(block.get() + r * ld, host + (r0 + r) * n1, (size_t)n1 * 4);
+    HIP_TRY(hipMemcpy(dev + r0 * ld, block.get(), n * ld * 4, hipMemcpyHostToDevice));
+  }
   return RELAX_OK;
 }
 int get_real(float* host, const float* dev, int n1, long rows, int align) {
-  if (align) HIP_TRY(hipMemcpy(host, dev, (size_t)(n1 + 2) * rows * 4, hipMemcpyDeviceToHost));
-  else HIP_TRY(hipMemcpy2D(host, n1 * 4, dev, (n1 + 2) * 4, n1 * 4, rows, hipMemcpyDeviceToHost));
+  if (align) {
+    HIP_TRY(hipMemcpy(host, dev, (size_t)(n1 + 2) * rows * 4, hipMemcpyDeviceToHost));
+    return RELAX_OK;
+  }
+  const size_t ld = n1 + 2, nb = block_rows(n1, rows);
+  std::unique_ptr<float[]> block(new (std::nothrow) float[nb * ld]);
+  if (!block) return RELAX_ERR_NOMEM;
+  for (size_t r0 = 0; r0 < (size_t)rows; r0 += nb) {
+    const size_t n = std::min(nb, (size_t)rows - r0);
+    HIP_TRY(hipMemcpy(block.get(), dev + r0 * ld, n * ld * 4, hipMemcpyDeviceToHost));
+    for (size_t r = 0; r < n; ++r) std::memcpy(host + (r0 + r) * n1, block.get() + r * ld, (size_t)n1 * 4);
+  }
   return RELAX_OK;
 }
 

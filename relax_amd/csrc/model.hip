@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -788,12 +789,60 @@ int relax_model_get_patches(relax_model_t* m, relax_slippatch_t* patches) {
   return RELAX_OK;
 }
 
-static int copy_field(float* dst, const float* src, const Grid& g, int align, bool to_dev, hipStream_t st) {
-  const size_t hp = (size_t)(align ? g.n1 + 2 : g.n1) * 4, dp = (size_t)g.n1 * 4;
+// Fields between the host's rows (n1 floats, pitch n1 + 2 with align) and the
+// device's packed rows.  A pitched copy (hipMemcpy2DAsync) of pageable memory
+// goes row by row in the runtime, 7 us each: 10.3 ms for the surface of a
+// 512x512 grid (3 x 512 rows), 0.46 s for the four fields of 256x256x128.  So
+// only whole blocks are copied: packed host rows directly (the surface: 0.2 ms),
+// padded ones through a block of at most 4 MB that the host unpacks row by row
+// (the caller's padding is left alone), and an upload's padded rows as they
+// stand into the work field, where a kernel packs them.
+static const size_t COPY_BLOCK = 4u << 20;
+
+// rows of the padded host layout (host -> device), staged in tmp (device, rows
+// (n1 + 2) floats)
+__global__ void k_pack_rows(float* __restrict__ dst, const float* __restrict__ src, int n1, long n) {
+  const long o = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  if (o >= n) return;
+  const long r = o / n1;
+  dst[o] = src[o + 2 * r];
+}
+
+static int put_field(float* dst, const float* src, const Grid& g, int align, float* tmp, hipStream_t st) {
+  if (!align) {
+    HIP_TRY(hipMemcpyAsync(dst, src, (size_t)g.H * 4, hipMemcpyHostToDevice, st));
+    return RELAX_OK;
+  }
+  // the last row's padding is not read
   const size_t rows = (size_t)g.n2 * g.h3;
-  if (to_dev) HIP_TRY(hipMemcpy2DAsync(dst, dp, src, hp, dp, rows, hipMemcpyHostToDevice, st));
-  else HIP_TRY(hipMemcpy2DAsync(dst, hp, src, dp, dp, rows, hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipMemcpyAsync(tmp, src, (rows * (g.n1 + 2) - 2) * 4, hipMemcpyHostToDevice, st));
+  k_pack_rows<<<(unsigned)((g.H + 255) / 256), 256, 0, st>>>(dst, tmp, g.n1, g.H);
+  HIP_TRY(hipGetLastError());
   return RELAX_OK;
+}
+
+// rows consecutive rows of a device field into the host layout; the caller
+// waits for st
+static int get_rows(float* dst, const float* src, int n1, size_t rows, int align, hipStream_t st) {
+  const size_t row = (size_t)n1 * 4;
+  if (!align) {
+    HIP_TRY(hipMemcpyAsync(dst, src, row * rows, hipMemcpyDeviceToHost, st));
+    return RELAX_OK;
+  }
+  const size_t nb = std::max<size_t>(1, std::min(rows, COPY_BLOCK / row));
+  std::unique_ptr<char[]> block(new (std::nothrow) char[nb * row]);
+  if (!block) return RELAX_ERR_NOMEM;
+  for (size_t r0 = 0; r0 < rows; r0 += nb) {
+    const size_t n = std::min(nb, rows - r0);
+    HIP_TRY(hipMemcpyAsync(block.get(), src + r0 * n1, n * row, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    for (size_t r = 0; r < n; ++r) std::memcpy(dst + (r0 + r) * (n1 + 2), block.get() + r * row, row);
+  }
+  return RELAX_OK;
+}
+
+static int get_field(float* dst, const float* src, const Grid& g, int align, hipStream_t st) {
+  return get_rows(dst, src, g.n1, (size_t)g.n2 * g.h3, align, st);
 }
 
 int relax_model_upload(relax_model_t* m, const float* u1, const float* u2, const float* u3,
@@ -804,10 +853,11 @@ int relax_model_upload(relax_model_t* m, const float* u1, const float* u2, const
   const Grid& g = m->g;
   const long H = g.H;
   int rc;
-  if ((rc = copy_field(m->u, u1, g, align_data, true, m->stream))) return rc;
-  if ((rc = copy_field(m->u + H, u2, g, align_data, true, m->stream))) return rc;
-  if ((rc = copy_field(m->u + 2 * H, u3, g, align_data, true, m->stream))) return rc;
-  if (gamma) { if ((rc = copy_field(m->gam, gamma, g, align_data, true, m->stream))) return rc; }
+  // padded rows are staged in the work field (3H floats, scratch between steps)
+  if ((rc = put_field(m->u, u1, g, align_data, m->W, m->stream))) return rc;
+  if ((rc = put_field(m->u + H, u2, g, align_data, m->W, m->stream))) return rc;
+  if ((rc = put_field(m->u + 2 * H, u3, g, align_data, m->W, m->stream))) return rc;
+  if (gamma) { if ((rc = put_field(m->gam, gamma, g, align_data, m->W, m->stream))) return rc; }
   else HIP_TRY(hipMemsetAsync(m->gam, 0, H * 4, m->stream));
   // tensors: stage the AoS copy in the sig buffer's space via a temporary
   float* tmp = nullptr;
@@ -839,10 +889,10 @@ int relax_model_download(relax_model_t* m, float* u1, float* u2, float* u3, rela
   const Grid& g = m->g;
   const long H = g.H;
   int rc;
-  if (u1 && (rc = copy_field(u1, m->u, g, align_data, false, m->stream))) return rc;
-  if (u2 && (rc = copy_field(u2, m->u + H, g, align_data, false, m->stream))) return rc;
-  if (u3 && (rc = copy_field(u3, m->u + 2 * H, g, align_data, false, m->stream))) return rc;
-  if (gamma && (rc = copy_field(gamma, m->gam, g, align_data, false, m->stream))) return rc;
+  if (u1 && (rc = get_field(u1, m->u, g, align_data, m->stream))) return rc;
+  if (u2 && (rc = get_field(u2, m->u + H, g, align_data, m->stream))) return rc;
+  if (u3 && (rc = get_field(u3, m->u + 2 * H, g, align_data, m->stream))) return rc;
+  if (gamma && (rc = get_field(gamma, m->gam, g, align_data, m->stream))) return rc;
   if (tau || sig) {
     float* tmp = nullptr;
     HIP_TRY(rx_malloc(&tmp, 6 * H * 4));
@@ -874,11 +924,10 @@ int relax_model_surface(relax_model_t* m, float* u1, float* u2, float* u3, int a
   if (!m) return RELAX_ERR_ARG;
   if (int rc = wait_batch(m)) return rc;
   const Grid& g = m->g;
-  const size_t hp = (size_t)(align_data ? g.n1 + 2 : g.n1) * 4, dp = (size_t)g.n1 * 4;
   float* dst[3] = {u1, u2, u3};
   for (int c = 0; c < 3; ++c) {
     if (!dst[c]) continue;
-    HIP_TRY(hipMemcpy2DAsync(dst[c], hp, m->u + c * g.H, dp, dp, (size_t)g.n2, hipMemcpyDeviceToHost, m->stream));
+    if (int rc = get_rows(dst[c], m->u + c * g.H, g.n1, (size_t)g.n2, align_data, m->stream)) return rc;
   }
   HIP_TRY(hipStreamSynchronize(m->stream));
   return RELAX_OK;
@@ -1194,8 +1243,11 @@ int relax_model_run(relax_model_t* m, int nsteps, const double* dt_override, rel
   if (!m || nsteps < 0 || m->batch) return RELAX_ERR_ARG;
   int k = 0;
   for (; k < nsteps; ++k) {
-    HIP_TRY(hipMemcpyAsync(m->host_sc, m->sc, sizeof(StepScalars), hipMemcpyDeviceToHost, m->stream));
-    HIP_TRY(hipStreamSynchronize(m->stream));
+    // the scalars before the first step; later steps have left theirs in host_sc
+    if (k == 0) {
+      HIP_TRY(hipMemcpyAsync(m->host_sc, m->sc, sizeof(StepScalars), hipMemcpyDeviceToHost, m->stream));
+      HIP_TRY(hipStreamSynchronize(m->stream));
+    }
     if (m->host_sc->status) { if (done) *done = k; return m->host_sc->status; }
     if (m->host_sc->t >= m->desc.interval) break;
     const int e0 = m->host_sc->e;
