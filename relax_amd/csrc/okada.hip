@@ -30,7 +30,7 @@ namespace {
 struct OkadaSource {
   double x1, x2;          // upper corner at the start of the strike (north, east)
   double csst, ssst;      // cos, sin of the strike
-  double sd, cd;          // DC3D's dip constants (DCCON0)
+  double sd, cd, icd2;    // DC3D's dip constants (DCCON0), 1/cd^2
   float depth, al2, aw1;  // DEPTH, AL2 = length, AW1 = -width (AL1 = AW2 = 0)
   float d1, d2, d3;       // DISL1..3: slip cos(rake), slip sin(rake), opening
 };
@@ -38,135 +38,274 @@ struct OkadaSource {
 constexpr double OK_EPS = 1.0e-6;
 constexpr double OK_PI2 = 6.283185307179586;
 
-// Displacement of one corner: the A part (infinite medium) and, for the
-// image, the B and C parts, each summed over the three dislocation kinds and
-// divided by 2 pi.
-__device__ __forceinline__ void ok_corner(double xi, double et, double q, double z, double sd, double cd, double alpha,
-                                          double U1, double U2, double U3, bool kxi, bool ket, bool image,
-                                          double fA[3], double fB[3], double fC[3]) {
+// Both sections of DC3D (the real source and its image) at one point need
+// Table 6 at the four corners (xi, eta) of the fault, summed with the signs
+// + - - + (Chinnery).  q, the dip and z are the same at the four corners, so
+// the table is linear in a few corner sums and the transcendental terms
+// collapse before they are evaluated:
+//  - the signed sum of ln(R + eta) is one logarithm of a quotient of
+//    products, likewise ln(R + xi) and ln(R + d~);
+//  - the signed sum of four arc tangents is one atan2 of a product of complex
+//    numbers: two of them lie within half a turn of each other, and the signs
+//    of the pairs tell the full turns;
+//  - roots and reciprocals are Newton steps on the hardware's estimates.
+// The kernel is bound by FP64 issue: 129 sources on 256x256x64 points (541 M
+// pairs) take 24.6 ms (about 900 FP64 instructions a pair, 214 VGPRs) against
+// 103 ms with the table evaluated corner by corner (20 logarithms, 12 arc
+// tangents, 18 roots and some 150 divisions a pair).  Held to 3 waves per
+// SIMD (168 VGPRs, 50 spilled) it takes 36 ms, with the two sections in a loop
+// 27 ms.
+struct OkadaSums {
+  double th, le, lx;               // th, ln(R+eta), ln(R+xi)
+  double R1, X, Y, xY, eX;         // 1/R, X11, Y11, xi Y11, eta X11
+  // the image only
+  double lrd, at, xd, yd;          // ln(Rd), 2 atan of I4, xi/Rd, y~/Rd
+  double ed, yd2, xyd2;            // vertical faults: eta/Rd, y~/Rd^2, xi y~/Rd^2
+  double R3, eR3, eeR3;            // 1/R^3 and eta, eta^2 times it
+  double X3, eX3, eeX3;            // X32 and eta, eta^2 times it
+  double Z, xZ, xxZ;               // Z32 and xi, xi^2 times it
+};
+
+// 1/x from the hardware's estimate (better than 2^-26) and two Newton steps;
+// x is normal here, so none of a division's scaling and special cases
+__device__ __forceinline__ double ok_rcp(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+// sqrt(x), x > 0, and 1/sqrt(x): Goldschmidt's iteration from the hardware's
+// estimate
+__device__ __forceinline__ double ok_root(double x, double& inv) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  inv = 2.0 * h;
+  return g;
+}
+// a b and a - b rounded by themselves (no fused multiply-add)
+__device__ __forceinline__ double ok_mul(double a, double b) {
 #pragma clang fp contract(off)
-  const double R2 = xi * xi + et * et + q * q;
-  const double R = sqrt(R2);
-  const double yt = et * cd + q * sd, dt = et * sd - q * cd;
-  const double th = (q == 0.0) ? 0.0 : atan(xi * et / (q * R));
-  double lx, X11, X32, le, Y11, Y32;
-  if (kxi) {
-    lx = -log(R - xi); X11 = 0.0; X32 = 0.0;
-  } else {
-    const double rx = R + xi;
-    lx = log(rx); X11 = 1.0 / (R * rx); X32 = (2.0 * R + xi) / (R * R * R * rx * rx);
-  }
-  if (ket) {
-    le = -log(R - et); Y11 = 0.0; Y32 = 0.0;
-  } else {
-    const double re = R + et;
-    le = log(re); Y11 = 1.0 / (R * re); Y32 = (2.0 * R + et) / (R * R * R * re * re);
-  }
-  const double a = alpha, b = 1.0 - alpha, q2 = q * q;
-  // strike-slip, dip-slip and tensile rows of Table 6, A part
-  {
-    const double s1 = th / 2 + a / 2 * xi * q * Y11, s2 = a / 2 * q / R, s3 = b / 2 * le - a / 2 * q2 * Y11;
-    const double d1 = a / 2 * q / R, d2 = th / 2 + a / 2 * et * q * X11, d3 = b / 2 * lx - a / 2 * q2 * X11;
-    const double t1 = -b / 2 * le - a / 2 * q2 * Y11, t2 = -b / 2 * lx - a / 2 * q2 * X11;
-    const double t3 = th / 2 - a / 2 * q * (et * X11 + xi * Y11);
-    fA[0] = (U1 * s1 + U2 * d1 + U3 * t1) / OK_PI2;
-    fA[1] = (U1 * s2 + U2 * d2 + U3 * t2) / OK_PI2;
-    fA[2] = (U1 * s3 + U2 * d3 + U3 * t3) / OK_PI2;
-  }
-  if (!image) return;
-  const double Rd = R + dt;
-  double I3, I4;
-  if (cd != 0.0) {
-    if (xi == 0.0) {
-      I4 = 0.0;
-    } else {
-      const double X = sqrt(xi * xi + q2);
-      I4 = (xi / Rd * sd * cd + 2.0 * atan((et * (X + q * cd) + X * (R + X) * sd) / (xi * (R + X) * cd))) / (cd * cd);
+  return a * b;
+}
+__device__ __forceinline__ double ok_sub(double a, double b) {
+#pragma clang fp contract(off)
+  return a - b;
+}
+
+// atan2(y0, x0) - atan2(y1, x1) with one atan2: the angle of the product of
+// one number and the other's conjugate, a full turn apart where the
+// difference leaves (-pi, pi)
+__device__ __forceinline__ double ok_angle(double y0, double x0, double y1, double x1) {
+  const double t = atan2(y0 * x1 - y1 * x0, x0 * x1 + y0 * y1);
+  const double turn = (y0 >= 0.0 && y1 < 0.0 && t < 0.0) ? OK_PI2 : (y0 < 0.0 && y1 >= 0.0 && t > 0.0) ? -OK_PI2 : 0.0;
+  return t + turn;
+}
+
+// The sums of one section.  kxi[k], ket[j] mark the negative extensions of the
+// edges (k: eta corner, j: xi corner).
+template <bool IMAGE>
+__device__ __forceinline__ OkadaSums ok_sums(const double xi[2], const double et[2], double q, double z, double sd,
+                                             double cd) {
+  OkadaSums S{};
+  double R[2][2], iR[2][2], re[2][2], rx[2][2], rd[2][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) R[j][k] = ok_root(xi[j] * xi[j] + et[k] * et[k] + q * q, iR[j][k]);
+  const bool kxi[2] = {xi[0] < 0.0 && R[1][0] + xi[1] < OK_EPS, xi[0] < 0.0 && R[1][1] + xi[1] < OK_EPS};
+  const bool ket[2] = {et[0] < 0.0 && R[0][1] + et[1] < OK_EPS, et[0] < 0.0 && R[1][1] + et[1] < OK_EPS};
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    OkadaSums t[2];  // the terms of the two xi corners
+    const double e = et[k];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const double x = xi[j];
+      const double r = R[j][k], i1 = iR[j][k];
+      // the logarithms' arguments, on an extension those of -ln(R - .)
+      rx[j][k] = kxi[k] ? r - x : r + x;
+      re[j][k] = ket[j] ? r - e : r + e;
+      const double X11 = kxi[k] ? 0.0 : ok_mul(i1, ok_rcp(rx[j][k])), Y11 = ket[j] ? 0.0 : ok_mul(i1, ok_rcp(re[j][k]));
+      t[j].R1 = i1;
+      t[j].X = X11;
+      t[j].Y = Y11;
+      t[j].xY = x * Y11;
+      if (IMAGE) {
+        const double yt = e * cd + q * sd, d = r + (e * sd - q * cd), id = ok_rcp(d);
+        rd[j][k] = d;
+        t[j].xd = x * id;
+        t[j].yd = ok_mul(yt, id);
+        if (cd == 0.0) {
+          t[j].ed = ok_mul(e, id);
+          t[j].yd2 = ok_mul(yt * id, id);
+          t[j].xyd2 = x * yt * id * id;
+        }
+        const double i3 = ok_mul(i1 * i1, i1), Y32 = (2.0 * r + e) * i1 * Y11 * Y11;
+        t[j].R3 = i3;
+        const double X32 = (2.0 * r + x) * i1 * X11 * X11;
+        t[j].X3 = X32;
+        const double Z32 = sd * i3 - (q * cd - z) * Y32;
+        t[j].Z = Z32;
+        t[j].xZ = x * Z32;
+        t[j].xxZ = ok_mul(x * x, Z32);
+      }
     }
-    I3 = (yt * cd / Rd - le + sd * log(Rd)) / (cd * cd);
-  } else {
-    I3 = (et / Rd + yt * q / (Rd * Rd) - le) / 2.0;
-    I4 = xi * yt / (Rd * Rd) / 2.0;
-  }
-  const double I1 = -xi / Rd * cd - I4 * sd;
-  const double I2 = log(Rd) + I3 * sd;
-  const double k = b / a;
-  {
-    const double s1 = -xi * q * Y11 - th - k * I1 * sd, s2 = -q / R + k * yt / Rd * sd, s3 = q2 * Y11 - k * I2 * sd;
-    const double d1 = -q / R + k * I3 * sd * cd, d2 = -et * q * X11 - th - k * xi / Rd * sd * cd;
-    const double d3 = q2 * X11 + k * I4 * sd * cd;
-    const double t1 = q2 * Y11 - k * I3 * sd * sd, t2 = q2 * X11 + k * xi / Rd * sd * sd;
-    const double t3 = q * (et * X11 + xi * Y11) - th - k * I4 * sd * sd;
-    fB[0] = (U1 * s1 + U2 * d1 + U3 * t1) / OK_PI2;
-    fB[1] = (U1 * s2 + U2 * d2 + U3 * t2) / OK_PI2;
-    fB[2] = (U1 * s3 + U2 * d3 + U3 * t3) / OK_PI2;
+    // a point midway along the strike has equal terms at the two corners:
+    // their difference is exactly 0, as in the corner-by-corner sum
+    const double sg = k == 0 ? 1.0 : -1.0;
+#define OK_SUM(f) S.f += sg * ok_sub(t[0].f, t[1].f)
+    OK_SUM(R1); OK_SUM(X); OK_SUM(Y); OK_SUM(xY); S.eX += sg * (e * ok_sub(t[0].X, t[1].X));
+    if (IMAGE) {
+      OK_SUM(xd); OK_SUM(yd);
+      if (cd == 0.0) { OK_SUM(ed); OK_SUM(yd2); OK_SUM(xyd2); }
+      const double r3 = sg * ok_sub(t[0].R3, t[1].R3), x3 = sg * ok_sub(t[0].X3, t[1].X3);
+      S.R3 += r3; S.eR3 += e * r3; S.eeR3 += e * e * r3;
+      S.X3 += x3; S.eX3 += e * x3; S.eeX3 += e * e * x3;
+      OK_SUM(Z); OK_SUM(xZ); OK_SUM(xxZ);
+    }
+#undef OK_SUM
   }
   {
-    const double R3 = R * R * R;
-    const double ct = dt + z, h = q * cd - z;
-    const double Z32 = sd / R3 - h * Y32;
-    const double s1 = b * xi * Y11 * cd - a * xi * q * Z32;
-    const double s2 = b * (cd / R + 2.0 * q * Y11 * sd) - a * ct * q / R3;
-    const double s3 = b * q * Y11 * cd - a * (ct * et / R3 - z * Y11 + xi * xi * Z32);
-    const double d1 = b * cd / R - q * Y11 * sd - a * ct * q / R3;
-    const double d2 = b * yt * X11 - a * ct * et * q * X32;
-    const double d3 = -dt * X11 - xi * Y11 * sd - a * ct * (X11 - q2 * X32);
-    const double t1 = -b * (sd / R + q * Y11 * cd) - a * (z * Y11 - q2 * Z32);
-    const double t2 = b * 2.0 * xi * Y11 * sd + dt * X11 - a * ct * (X11 - q2 * X32);
-    const double t3 = b * (yt * X11 + xi * Y11 * cd) + a * q * (ct * et * X32 + xi * Z32);
-    fC[0] = (U1 * s1 + U2 * d1 + U3 * t1) / OK_PI2;
-    fC[1] = (U1 * s2 + U2 * d2 + U3 * t2) / OK_PI2;
-    fC[2] = (U1 * s3 + U2 * d3 + U3 * t3) / OK_PI2;
+    double n = 1.0, d = 1.0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      // + le(0,0) - le(0,1), - le(1,0) + le(1,1); reversed on an extension
+      const double a = re[j][j], b = re[j][1 - j];
+      n *= ket[j] ? b : a;
+      d *= ket[j] ? a : b;
+    }
+    S.le = log(n / d);
   }
+  {
+    double n = 1.0, d = 1.0;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const double a = rx[k][k], b = rx[1 - k][k];
+      n *= kxi[k] ? b : a;
+      d *= kxi[k] ? a : b;
+    }
+    S.lx = log(n / d);
+  }
+  if (q != 0.0) {
+    // the angles of the two xi corners, atan(p0/w0) - atan(p1/w1)
+    const double aq = fabs(q);
+    double y[2], w[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const double p0 = xi[j] * et[0], p1 = xi[j] * et[1], w0 = aq * R[j][0], w1 = aq * R[j][1];
+      y[j] = p0 * w1 - p1 * w0;
+      w[j] = w0 * w1 + p0 * p1;
+    }
+    const double t = ok_angle(y[0], w[0], y[1], w[1]);
+    S.th = q < 0.0 ? -t : t;
+  }
+  if (IMAGE) {
+    S.lrd = log((rd[0][0] * rd[1][1]) / (rd[0][1] * rd[1][0]));
+    if (cd != 0.0) {
+      double y[2], w[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        double i1;
+        const double x = xi[j], X = ok_root(x * x + q * q, i1);
+        const double r0 = R[j][0] + X, r1 = R[j][1] + X, c = fabs(x * cd);
+        const double n0 = et[0] * (X + q * cd) + X * r0 * sd, n1 = et[1] * (X + q * cd) + X * r1 * sd;
+        const double d0 = c * r0, d1 = c * r1, v = n0 * d1 - n1 * d0;
+        y[j] = x * cd < 0.0 ? -v : v;
+        w[j] = d0 * d1 + n0 * n1;
+        if (x == 0.0) { y[j] = 0.0; w[j] = 1.0; }  // I4 = 0 there
+      }
+      S.at = 2.0 * ok_angle(y[0], w[0], y[1], w[1]);
+    }
+  }
+  return S;
 }
 
 // DC3D's displacement at (X, Y, Z) (its single-precision arguments, widened);
 // false at a singular point (on a fault edge).
-__device__ bool ok_dc3d(const OkadaSource& S, double alpha, double x, double y, double z, double u[3]) {
-#pragma clang fp contract(off)
+__device__ __forceinline__ bool ok_dc3d(const OkadaSource& S, double alpha, double x, double y, double z, double u[3]) {
   const double sd = S.sd, cd = S.cd, c = S.depth;
   const double U1 = S.d1, U2 = S.d2, U3 = S.d3;
-  double xi[2] = {x - 0.0, x - (double)S.al2};
-  for (int j = 0; j < 2; ++j)
-    if (fabs(xi[j]) < OK_EPS) xi[j] = 0.0;
   u[0] = u[1] = u[2] = 0.0;
+  const double a = alpha, b = 1.0 - alpha;
+#pragma unroll
   for (int section = 0; section < 2; ++section) {
-    const double d = section == 0 ? c + z : c - z;
-    const double p = y * cd + d * sd;
-    double q = y * sd - d * cd;
-    double et[2] = {p - (double)S.aw1, p - 0.0};
-    if (fabs(q) < OK_EPS) q = 0.0;
-    for (int k = 0; k < 2; ++k)
-      if (fabs(et[k]) < OK_EPS) et[k] = 0.0;
-    if (q == 0.0 && ((xi[0] * xi[1] <= 0.0 && et[0] * et[1] == 0.0) || (et[0] * et[1] <= 0.0 && xi[0] * xi[1] == 0.0)))
-      return false;
-    const double r12 = sqrt(xi[0] * xi[0] + et[1] * et[1] + q * q);
-    const double r21 = sqrt(xi[1] * xi[1] + et[0] * et[0] + q * q);
-    const double r22 = sqrt(xi[1] * xi[1] + et[1] * et[1] + q * q);
-    const bool kxi[2] = {xi[0] < 0.0 && r21 + xi[1] < OK_EPS, xi[0] < 0.0 && r22 + xi[1] < OK_EPS};
-    const bool ket[2] = {et[0] < 0.0 && r12 + et[1] < OK_EPS, et[0] < 0.0 && r22 + et[1] < OK_EPS};
-    for (int kk = 0; kk < 2; ++kk)
-      for (int j = 0; j < 2; ++j) {
-        double fA[3], fB[3] = {0.0, 0.0, 0.0}, fC[3] = {0.0, 0.0, 0.0};
-        ok_corner(xi[j], et[kk], q, z, sd, cd, alpha, U1, U2, U3, kxi[kk], ket[j], section == 1, fA, fB, fC);
-        double du0, du1, du2;
-        if (section == 0) {
-          // the real source: -A (dc3d.f's real-source sum)
-          du0 = -fA[0];
-          du1 = -fA[1] * cd + fA[2] * sd;
-          du2 = -fA[1] * sd - fA[2] * cd;
-        } else {
-          // the image: A + B + z C, the vertical part of C reversed
-          du0 = fA[0] + fB[0] + z * fC[0];
-          du1 = (fA[1] + fB[1] + z * fC[1]) * cd - (fA[2] + fB[2] + z * fC[2]) * sd;
-          du2 = (fA[1] + fB[1] - z * fC[1]) * sd + (fA[2] + fB[2] - z * fC[2]) * cd;
-        }
-        const double sgn = (j + kk == 1) ? -1.0 : 1.0;  // Chinnery's sum
-        u[0] += sgn * du0;
-        u[1] += sgn * du1;
-        u[2] += sgn * du2;
+    double xi[2], et[2], q;
+    {
+      // the decisions below follow DC3D's own rounding
+#pragma clang fp contract(off)
+      xi[0] = x - 0.0;
+      xi[1] = x - (double)S.al2;
+      const double d = section == 0 ? c + z : c - z;
+      const double p = y * cd + d * sd;
+      q = y * sd - d * cd;
+      et[0] = p - (double)S.aw1;
+      et[1] = p - 0.0;
+      if (fabs(q) < OK_EPS) q = 0.0;
+      for (int k = 0; k < 2; ++k) {
+        if (fabs(xi[k]) < OK_EPS) xi[k] = 0.0;
+        if (fabs(et[k]) < OK_EPS) et[k] = 0.0;
       }
+      if (q == 0.0 && ((xi[0] * xi[1] <= 0.0 && et[0] * et[1] == 0.0) || (et[0] * et[1] <= 0.0 && xi[0] * xi[1] == 0.0)))
+        return false;
+    }
+    const OkadaSums T = section == 0 ? ok_sums<false>(xi, et, q, z, sd, cd) : ok_sums<true>(xi, et, q, z, sd, cd);
+    const double q2 = q * q, a2 = a / 2, b2 = b / 2;
+    // the A part (infinite medium): strike-slip, dip-slip and tensile rows
+    double A0 = U1 * (T.th / 2 + a2 * q * T.xY) + U2 * (a2 * q * T.R1);
+    double A1 = U1 * (a2 * q * T.R1) + U2 * (T.th / 2 + a2 * q * T.eX);
+    double A2 = U1 * (b2 * T.le - a2 * q2 * T.Y) + U2 * (b2 * T.lx - a2 * q2 * T.X);
+    if (U3 != 0.0) {
+      A0 += U3 * (-b2 * T.le - a2 * q2 * T.Y);
+      A1 += U3 * (-b2 * T.lx - a2 * q2 * T.X);
+      A2 += U3 * (T.th / 2 - a2 * q * (T.eX + T.xY));
+    }
+    if (section == 0) {
+      // the real source: -A (dc3d.f's real-source sum)
+      u[0] = -A0;
+      u[1] = -A1 * cd + A2 * sd;
+      u[2] = -A1 * sd - A2 * cd;
+      continue;
+    }
+    double I3, I4;
+    if (cd != 0.0) {
+      I4 = (T.xd * sd * cd + T.at) * S.icd2;
+      I3 = (T.yd * cd - T.le + sd * T.lrd) * S.icd2;
+    } else {
+      I3 = (T.ed + q * T.yd2 - T.le) / 2.0;
+      I4 = T.xyd2 / 2.0;
+    }
+    const double I1 = -T.xd * cd - I4 * sd, I2 = T.lrd + I3 * sd, k = b / a;
+    double B0 = U1 * (-q * T.xY - T.th - k * I1 * sd) + U2 * (-q * T.R1 + k * I3 * sd * cd);
+    double B1 = U1 * (-q * T.R1 + k * T.yd * sd) + U2 * (-q * T.eX - T.th - k * T.xd * sd * cd);
+    double B2 = U1 * (q2 * T.Y - k * I2 * sd) + U2 * (q2 * T.X + k * I4 * sd * cd);
+    // c~ = eta sin(dip) - h; y~ and d~ are linear in eta as well
+    const double h = q * cd - z;
+    const double yX = cd * T.eX + q * sd * T.X, dX = sd * T.eX - q * cd * T.X, cX = sd * T.eX - h * T.X;
+    const double cR3 = sd * T.eR3 - h * T.R3, ceR3 = sd * T.eeR3 - h * T.eR3;
+    const double cX3 = sd * T.eX3 - h * T.X3, ceX3 = sd * T.eeX3 - h * T.eX3;
+    double C0 = U1 * (b * cd * T.xY - a * q * T.xZ) + U2 * (b * cd * T.R1 - q * sd * T.Y - a * q * cR3);
+    double C1 = U1 * (b * (cd * T.R1 + 2.0 * q * sd * T.Y) - a * q * cR3) + U2 * (b * yX - a * q * ceX3);
+    double C2 = U1 * (b * q * cd * T.Y - a * (ceR3 - z * T.Y + T.xxZ)) +
+                U2 * (-dX - sd * T.xY - a * (cX - q2 * cX3));
+    if (U3 != 0.0) {
+      B0 += U3 * (q2 * T.Y - k * I3 * sd * sd);
+      B1 += U3 * (q2 * T.X + k * T.xd * sd * sd);
+      B2 += U3 * (q * (T.eX + T.xY) - T.th - k * I4 * sd * sd);
+      C0 += U3 * (-b * (sd * T.R1 + q * cd * T.Y) - a * (z * T.Y - q2 * T.Z));
+      C1 += U3 * (b * 2.0 * sd * T.xY + dX - a * (cX - q2 * cX3));
+      C2 += U3 * (b * (yX + cd * T.xY) + a * q * (ceX3 + T.xZ));
+    }
+    // the image: A + B + z C, the vertical part of C reversed
+    u[0] += A0 + B0 + z * C0;
+    u[1] += (A1 + B1 + z * C1) * cd - (A2 + B2 + z * C2) * sd;
+    u[2] += (A1 + B1 - z * C1) * sd + (A2 + B2 - z * C2) * cd;
   }
+  for (int c3 = 0; c3 < 3; ++c3) u[c3] *= 1.0 / OK_PI2;
   return true;
 }
 
@@ -224,6 +363,7 @@ static OkadaSource okada_source(double slip, double opening, const relax_source_
     S.cd = 0.0;
     S.sd = S.sd > 0.0 ? 1.0 : (S.sd < 0.0 ? -1.0 : S.sd);
   }
+  S.icd2 = S.cd != 0.0 ? 1.0 / (S.cd * S.cd) : 0.0;
   S.depth = (float)s.z;
   S.al2 = (float)s.length;
   S.aw1 = -(float)s.width;
