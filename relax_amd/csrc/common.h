@@ -156,6 +156,9 @@ struct PlaneDev {
   double Wp, Lp, xr, yr, zr;
   double n[3], r[3];
   double minlw;  // min(L,W)/sqrt(dx1*dx3) of the relaxation-time estimate
+  // d_gauss(x, dx1) = gs1 exp(gs2 x^2); d_omega(x, beta) = 1 to om0, 0 from
+  // om1, cos^2(omA |x| + omB) between
+  double iW, iL, gs1, gs2, om0, om1, omA, omB;
 };
 struct FrictionTables {
   // double precision, as LAYER_STRUCT (types.f90:31-34)
@@ -166,6 +169,9 @@ struct FrictionTables {
   const PlaneDev* planes;
   int np;
   int active;
+  // the box of all planes' bands: depths below zmax, nx samples along x1 from
+  // index x0 (periodic), ny along x2 from y0
+  int zmax, x0, nx, y0, ny;
 };
 
 // Device-side scalars of one model's time line.

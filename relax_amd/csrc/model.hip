@@ -312,12 +312,13 @@ static TimeLine timeline(const relax_model_t* m) {
   return tl;
 }
 
-// The kernels a model needs: the extended rheology with weak zones or
-// transient creep, the fault-creep kernels with afterslip planes.
+// The kernels a model needs: the extended rheology with weak zones,
+// transient creep or inter-seismic loading, the fault-creep kernels with
+// afterslip planes.
 static int rheo_class(const relax_model_t* m) {
   const RheoParams& R = m->R;
-  if (R.tr[0].active || R.tr[1].active || R.mech[0].dg || R.mech[1].dg || R.inter) return RHEO_EXT;
-  return (R.fr.active && R.fr.np > 0) ? RHEO_CREEP : RHEO_VISCOUS;
+  const bool ext = R.tr[0].active || R.tr[1].active || R.mech[0].dg || R.mech[1].dg || R.inter;
+  return (ext ? RHEO_EXT : 0) | (R.fr.active && R.fr.np > 0 ? RHEO_CREEP : 0);
 }
 
 // Refresh the model's device record after a change of its rheology, planes
@@ -486,6 +487,8 @@ int relax_model_reset(relax_model_t* m) {
   m->patch_off.assign(1, 0);
   m->R.fr.np = 0;
   m->R.fr.active = 0;
+  m->R.fr.zmax = 0;
+  m->R.fr.x0 = m->R.fr.nx = m->R.fr.y0 = m->R.fr.ny = 0;
   m->R.inter = nullptr;
   m->inter = 0;
   m->md_dirty = true;
@@ -732,6 +735,12 @@ PlaneDev make_plane(const relax_plane_t& p, double beta, double dx1, double dx3)
   P.r[1] = P.cstrike * cr - P.sstrike * P.sdip * sr;
   P.r[2] = P.cdip * sr;
   P.minlw = std::min(p.length, p.width) / std::sqrt(dx1 * dx3);
+  P.iW = 1.0 / P.W; P.iL = 1.0 / P.L;
+  P.gs1 = 1.0 / (std::sqrt(RELAX_PI2) * dx1); P.gs2 = -0.5 / (dx1 * dx1);
+  P.om0 = (1.0 - 2.0 * beta) / (1.0 - beta) / 2.0; P.om1 = 1.0 / (1.0 - beta) / 2.0;
+  // (beta = 0: om0 = om1, the taper is never evaluated)
+  P.omA = beta != 0.0 ? RELAX_PI * (1.0 - beta) / 2.0 / beta : 0.0;
+  P.omB = beta != 0.0 ? RELAX_PI * (beta - 0.5) / 2.0 / beta : 0.0;
   return P;
 }
 
@@ -775,6 +784,28 @@ int relax_model_set_planes(relax_model_t* m, const relax_plane_t* planes, int np
   m->R.fr.planes = m->planes_dev;
   m->R.fr.np = np;
   m->R.fr.active = (np > 0) && m->mech[2];
+  // the box of the planes' bands: their points have x3 <= |z| + Lp and x1, x2
+  // within max(Wp, Lp) of the centre (friction3d.f90:136-148)
+  FrictionTables& F = m->R.fr;
+  double lo[2] = {1e9, 1e9}, hi[3] = {-1e9, -1e9, -1.0};
+  const double d[2] = {m->desc.dx1, m->desc.dx2};
+  for (const PlaneDev& p : m->plane_dev_host) {
+    const double c[2] = {p.x, p.y}, wl = std::max(p.Wp, p.Lp);
+    for (int a = 0; a < 2; ++a) {
+      lo[a] = std::min(lo[a], std::floor((c[a] - wl) / d[a]) - 1.0);
+      hi[a] = std::max(hi[a], std::ceil((c[a] + wl) / d[a]) + 1.0);
+    }
+    hi[2] = std::max(hi[2], (std::fabs(p.z) + p.Lp) / m->desc.dx3);
+  }
+  F.zmax = hi[2] < 0.0 ? 0 : (int)std::min((double)m->g.h3, std::floor(hi[2]) + 2.0);
+  const int n[2] = {m->g.n1, m->g.n2};
+  int x0[2] = {0, 0}, nx[2] = {n[0], n[1]};
+  for (int a = 0; a < 2; ++a)
+    if (lo[a] >= -n[a] && hi[a] < n[a] && hi[a] - lo[a] + 1.0 < n[a]) {
+      x0[a] = ((int)lo[a] + 2 * n[a]) % n[a];
+      nx[a] = (int)(hi[a] - lo[a]) + 1;
+    }
+  F.x0 = x0[0]; F.nx = nx[0]; F.y0 = x0[1]; F.ny = nx[1];
   m->md_dirty = true;
   return RELAX_OK;
 }
@@ -2009,7 +2040,7 @@ static void batch_classes(relax_batch_t* b) {
 
 static int batch_rclass(const relax_batch_t* b) {
   int rc = RHEO_VISCOUS;
-  for (relax_model_t* m : b->models) rc = std::max(rc, rheo_class(m));
+  for (relax_model_t* m : b->models) rc |= rheo_class(m);
   return rc;
 }
 

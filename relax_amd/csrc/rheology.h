@@ -111,6 +111,18 @@ __device__ __forceinline__ float viscous_point(const Mechanism& M, const Prestre
   return 1.f / gd;
 }
 
+// d_omega and d_gauss with the plane's constants: no FP64 divisions
+__device__ __forceinline__ double plane_omega(const PlaneDev& P, double x) {
+  const double ax = fabs(x);
+  if (ax <= P.om0) return 1.0;
+  if (ax < P.om1) {
+    const double c = cos(P.omA * ax + P.omB);
+    return c * c;
+  }
+  return 0.0;
+}
+__device__ __forceinline__ double plane_gauss(const PlaneDev& P, double x) { return P.gs1 * exp(P.gs2 * x * x); }
+
 // Fault-creep contribution of one plane at grid point (i1,i2,i3).
 // Returns the candidate relaxation time (NaN-free: a NaN candidate becomes
 // +inf, as MIN keeps the running value) and sets *status on overflow.
@@ -129,9 +141,9 @@ __device__ __forceinline__ float friction_point(const RheoParams& R, const Plane
   const double x2s = P.sstrike * x1 + P.cstrike * x2;
   const double x3s = P.sdip * x2r + P.cdip * x3;
   const double x3i = -P.sdip * x2r + P.cdip * x3;
-  const double temp2 = d_omega((x2s - P.yr) / P.W, P.beta);
-  const double sourc = d_gauss(x1s - P.xr, dx1) * temp2 * d_omega((x3s - P.zr) / P.L, P.beta);
-  const double image = d_gauss(x1i - P.xr, dx1) * temp2 * d_omega((x3i + P.zr) / P.L, P.beta);
+  const double temp2 = plane_omega(P, (x2s - P.yr) * P.iW);
+  const double sourc = plane_gauss(P, x1s - P.xr) * temp2 * plane_omega(P, (x3s - P.zr) * P.iL);
+  const double image = plane_gauss(P, x1i - P.xr) * temp2 * plane_omega(P, (x3i + P.zr) * P.iL);
   const double impulse = sourc + image;
   const double* n = P.n;
   const double t0 = s.s11 * n[0] + s.s12 * n[1] + s.s13 * n[2];
@@ -144,11 +156,14 @@ __device__ __forceinline__ float friction_point(const RheoParams& R, const Plane
   const double tau = fmax(0.0, taus + fric * taun - coh);
   if ((ts0 * P.r[0] + ts1 * P.r[1] + ts2 * P.r[2]) < 0.0 && fabs(P.rake) < RELAX_PI2 * 1.5)
     return __builtin_inff();
-  const double tauc = R.fr.tauc[i3];
-  if ((tau / tauc) > 20) { *status = RELAX_ERR_FRICTION; return __builtin_inff(); }
-  ts0 /= taus; ts1 /= taus; ts2 /= taus;
-  const double gd = R.fr.v0[i3] * 2.0 * d_my_sinh(tau / tauc);
-  float cand = (float)(tau / (double)R.mu / gd * P.minlw);
+  const double ratio = tau / R.fr.tauc[i3];
+  if (ratio > 20) { *status = RELAX_ERR_FRICTION; return __builtin_inff(); }
+  const double it = 1.0 / taus;
+  ts0 *= it; ts1 *= it; ts2 *= it;
+  // sinh(x) = (e + e/(e+1))/2 with e = exp(x) - 1, clamped as my_sinh
+  const double e = expm1(fmin(ratio, 11.0));
+  const double gd = R.fr.v0[i3] * (e + e / (e + 1.0));
+  float cand = (float)(tau * P.minlw / ((double)R.mu * gd));
   if (cand != cand) cand = __builtin_inff();
   if (vel) *vel = (float)((double)*vel + gd * impulse * sqrt(RELAX_PI2) * dx1);
   const double a = 2.0 * (double)R.mu * impulse * gd;
@@ -160,6 +175,55 @@ __device__ __forceinline__ float friction_point(const RheoParams& R, const Plane
   m.s23 += (float)((ts1 * b2 + ts2 * b1) / 2.0);
   m.s33 += (float)(ts2 * b2);
   return cand;
+}
+
+// The band of a creeping plane: every grid point where friction_point passes
+// its gates, and a little more (7.02 instead of 7.01 dx1).  Kernels with and
+// without the creep code share a model's points by these tests, so no
+// contraction: they round alike wherever they are inlined.
+constexpr double BAND = 7.02;
+
+// whether point (i1,i2,i3) lies in the band of a plane
+__device__ __forceinline__ bool in_band(const RheoParams& R, int i1, int i2, int i3) {
+#pragma clang fp contract(off)
+  if (i3 >= R.fr.zmax) return false;
+  const double x1 = d_shifted(i1, R.n1, R.dx1), x2 = d_shifted(i2, R.n2, R.dx2), x3 = (double)i3 * R.dx3;
+  bool in = false;
+  for (int k = 0; k < R.fr.np; ++k) {
+    const PlaneDev& P = R.fr.planes[k];
+    const double wl = fmax(P.Wp, P.Lp), c = P.cdip * (P.cstrike * x1 - P.sstrike * x2) - P.xr, d = P.sdip * x3;
+    in = in || (x3 <= fabs(P.z) + P.Lp && fabs(x1 - P.x) <= wl && fabs(x2 - P.y) <= wl &&
+                (fabs(c - d) <= BAND * R.dx1 || fabs(c + d) <= BAND * R.dx1));
+  }
+  return in;
+}
+
+// depths [lo, hi] between which the bands of all planes cross column (i1,i2)
+// (lo > hi: none)
+__device__ __forceinline__ void column_band(const RheoParams& R, int i1, int i2, int& lo, int& hi) {
+#pragma clang fp contract(off)
+  lo = R.fr.zmax;
+  hi = -1;
+  const double x1 = d_shifted(i1, R.n1, R.dx1), x2 = d_shifted(i2, R.n2, R.dx2);
+  for (int k = 0; k < R.fr.np; ++k) {
+    const PlaneDev& P = R.fr.planes[k];
+    const double wl = fmax(P.Wp, P.Lp);
+    if (!(fabs(x1 - P.x) <= wl && fabs(x2 - P.y) <= wl)) continue;
+    const double c = P.cdip * (P.cstrike * x1 - P.sstrike * x2) - P.xr, w = BAND * R.dx1, sd = fabs(P.sdip);
+    const double zlim = fabs(P.z) + P.Lp;
+    // |c| - w <= sd x3 <= |c| + w bounds both the plane and its image
+    double za = 0.0, zb = zlim;
+    if (sd * zlim > 1e-9 * R.dx1) {
+      za = fmax(0.0, (fabs(c) - w) / sd);
+      zb = fmin(zlim, (fabs(c) + w) / sd);
+    } else if (fabs(c) > w + 1e-9 * R.dx1) {
+      continue;
+    }
+    if (za > zb + R.dx3) continue;
+    const double r = 1.0 / R.dx3;
+    lo = min(lo, max(0, (int)floor(fmin(za * r, 1e9) - 1e-3)));
+    hi = max(hi, min(R.fr.zmax - 1, (int)ceil(zb * r + 1e-3)));
+  }
 }
 
 // Moment-density rate of all mechanisms at one point (relax.f90:568-612).
@@ -226,7 +290,7 @@ __device__ __forceinline__ float point_fluidity(const Mechanism& M, int i3, long
 // calls, which pass epsilonikdot as both the strain and the rate: the
 // second mechanism reads the first one's rate.  In the predictor both read
 // epsilonik and the second one's rate replaces the first one's.
-template <bool TM, bool CORR>
+template <bool TM, bool CORR, bool FRIC>
 __device__ __forceinline__ T6 rheology_ext(const RheoParams& R, const T6& s, int i1, int i2, int i3, long o,
                                            const T6& e, T6* ed, float* tmin, float* grate_lin, float* grate_nl,
                                            int* status) {
@@ -243,7 +307,7 @@ __device__ __forceinline__ T6 rheology_ext(const RheoParams& R, const T6& s, int
       const float t = viscous_point(M, R.pre, R.mu, i3, g0, gdp, sd, m, k ? grate_nl : grate_lin);
       if (TM) tmin[k] = fminf(tmin[k], t);
     }
-    if (R.fr.active) {
+    if (FRIC && R.fr.active) {
       for (int k = 0; k < R.fr.np; ++k) {
         const float t = friction_point(R, R.fr.planes[k], i1, i2, i3, s, m, nullptr, status);
         if (TM) tmin[2] = fminf(tmin[2], t);
@@ -261,7 +325,7 @@ __device__ __forceinline__ T6 rheology_ext(const RheoParams& R, const T6& s, int
       }
       *ed = r;
     }
-  } else if (R.fr.active) {
+  } else if (FRIC && R.fr.active) {
     for (int k = 0; k < R.fr.np; ++k) {
       const float t = friction_point(R, R.fr.planes[k], i1, i2, i3, s, m, nullptr, status);
       if (TM) tmin[2] = fminf(tmin[2], t);

@@ -9,10 +9,15 @@ enum { STRESS_SET = 0, STRESS_PRED = 1, STRESS_CORR = 2 };
 // k_bodyforce: predictor (rheology + relaxation time), corrector, or the
 // divergence of a given moment density (no rheology)
 enum { BODY_PRED = 0, BODY_CORR = 1, BODY_RAW = 2 };
-// Rheology class of a launch: viscous mechanisms only; with fault creep;
-// extended (also weak zones and transient creep).  A batch takes the
-// largest class of its members.
-enum { RHEO_VISCOUS = 0, RHEO_CREEP = 1, RHEO_EXT = 2 };
+// Rheology class of a launch, a set of bits: viscous mechanisms only, with
+// fault creep, extended (weak zones, transient creep, inter-seismic loading).
+// A batch takes every bit of its members.
+enum { RHEO_VISCOUS = 0, RHEO_CREEP = 1, RHEO_EXT = 2, RHEO_ALL = 3 };
+// The part of a model that a kernel computes: models without creeping planes
+// have one part; with planes, the points in the planes' bands (in_band) go to
+// kernels with the FP64 creep code (165-210 VGPRs) and all others to kernels
+// without it (60-110).
+enum { PART_ALL = 0, PART_OUT = 1, PART_IN = 2 };
 
 struct StencilConst {
   float k1h, k2h, k3h;  // fir1 taps divided by the spacing: 0.5/dx

@@ -12,6 +12,7 @@
 //     differences at the top and bottom planes (stressupdate,
 //     elastic3d.f90:956-1180), Hooke's law, and the stage update of the RK2
 //     loop (relax.f90:679-701, :833-890) in the same pass.
+#include <algorithm>
 #include <atomic>
 
 #include "kernels.h"
@@ -23,18 +24,44 @@
 // rheology tables (read-only) are known not to alias the stores and are
 // read through the scalar cache.
 //
-// RC is the rheology class: RHEO_VISCOUS, RHEO_CREEP (with fault creep) or
-// RHEO_EXT (also weak zones and transient creep, which reads the transient
-// strain E: epsilonik in the predictor, the mid-step strain in the
-// corrector).  TM marks the predictor pass.
-template <int TXB, int TYB, bool TM, bool RAW, int RC>
+// EXT is the extended rheology (also weak zones and transient creep, which
+// reads the transient strain E: epsilonik in the predictor, the mid-step
+// strain in the corrector), PART the part of the model (PART_*).  TM marks the
+// predictor pass.
+
+// The planes [s0, s1) of a tile's output that the creep bands reach: outputs
+// one plane above and below a band take its moments too.  The tile's columns
+// and their halo are tested over the whole depth, so every chunk of the tile
+// and both parts get the same range.  Uniform over the workgroup.
+template <int TXB, int TYB, int NT>
+__device__ __forceinline__ int2 tile_band(const RheoParams& R, const Grid& g, int x0, int y0) {
+  __shared__ int band[2];
+  constexpr int HX = TXB + 2, HP = HX * (TYB + 2);
+  const int tid = threadIdx.x;
+  if (!R.fr.active) return make_int2(0, 0);
+  if (tid == 0) { band[0] = g.h3; band[1] = -1; }
+  __syncthreads();
+  int lo = g.h3, hi = -1;
+  for (int e = tid; e < HP; e += NT) {
+    int a, b;
+    column_band(R, (x0 + e % HX - 1 + g.n1) & (g.n1 - 1), (y0 + e / HX - 1 + g.n2) & (g.n2 - 1), a, b);
+    if (a <= b) { lo = min(lo, a); hi = max(hi, b); }
+  }
+  if (lo <= hi) { atomicMin(&band[0], lo); atomicMax(&band[1], hi); }
+  __syncthreads();
+  lo = band[0]; hi = band[1];
+  __syncthreads();
+  return lo > hi ? make_int2(0, 0) : make_int2(max(0, lo - 1), min(g.h3, hi + 2));
+}
+
+template <int TXB, int TYB, bool TM, bool RAW, bool EXT, int PART>
 __device__ __forceinline__ void bodyforce_tile(const Grid& g, const RheoParams& R, const StencilConst& S,
                                                const float* __restrict__ sig, const float* __restrict__ E,
                                                float* __restrict__ W, float* __restrict__ T, StepScalars* sc,
                                                int bx, int by, int bz, int zc, int gz) {
   constexpr int NT = TXB * TYB;
   constexpr int HX = TXB + 2, HY = TYB + 2, HP = HX * HY;
-  constexpr int NTM = RC == RHEO_EXT ? NMECH : 3;  // mechanisms whose minima are reduced
+  constexpr int NTM = EXT ? NMECH : 3;  // mechanisms whose minima are reduced
   __shared__ float ring[3][6][HP];
   __shared__ float rmin[NTM][NT / 64];
   const int tid = threadIdx.x;
@@ -42,12 +69,20 @@ __device__ __forceinline__ void bodyforce_tile(const Grid& g, const RheoParams& 
   const int n1 = g.n1, n2 = g.n2, h3 = g.h3;
   const long H = g.H;
   const int x0 = bx * TXB, y0 = by * TYB;
-  const int z0 = (bz % gz) * zc, z1 = min(z0 + zc, h3);
+  int z0 = (bz % gz) * zc, z1 = min(z0 + zc, h3);
+  // planes [s0, s1) belong to PART_IN
+  int2 sk = make_int2(0, 0);
+  if (PART != PART_ALL) {
+    if (PART == PART_IN && z0 > R.fr.zmax) return;
+    sk = tile_band<TXB, TYB, NT>(R, g, x0, y0);
+    if (PART == PART_IN) { z0 = max(z0, sk.x); z1 = min(z1, sk.y); }
+    if (z0 >= z1 || (PART == PART_OUT && z0 >= sk.x && z1 <= sk.y)) return;
+  }
   float tmin[NTM];
 #pragma unroll
   for (int k = 0; k < NTM; ++k) tmin[k] = __builtin_inff();
   int status = 0;
-  const bool trans = RC == RHEO_EXT && (R.tr[0].active || R.tr[1].active);
+  const bool trans = EXT && (R.tr[0].active || R.tr[1].active);
   const int e0 = (ty + 1) * HX + (tx + 1);
   const int i1 = x0 + tx, i2 = y0 + ty;
 
@@ -68,6 +103,7 @@ __device__ __forceinline__ void bodyforce_tile(const Grid& g, const RheoParams& 
     const float f1 = (s11[e0 + 1] - s11[e0 - 1]) * S.k1h + (s12[e0 + HX] - s12[e0 - HX]) * S.k2h + v[0];
     const float f2 = (s12[e0 + 1] - s12[e0 - 1]) * S.k1h + (s22[e0 + HX] - s22[e0 - HX]) * S.k2h + v[1];
     const float f3 = (s13[e0 + 1] - s13[e0 - 1]) * S.k1h + (s23[e0 + HX] - s23[e0 - HX]) * S.k2h + v[2];
+    if (PART == PART_OUT && zo >= sk.x && zo < sk.y) return;
     const long o = i1 + (long)n1 * (i2 + (long)n2 * zo);
     gst(W + o, -f1);
     gst(W + H + o, -f2);
@@ -92,14 +128,14 @@ __device__ __forceinline__ void bodyforce_tile(const Grid& g, const RheoParams& 
     pj1[k] = (x0 + hx - 1 + n1) % n1;
     pj2[k] = (y0 + hy - 1 + n2) % n2;
   }
-  T6 pre[KP], pre_e[RC == RHEO_EXT ? KP : 1];
+  T6 pre[KP], pre_e[EXT ? KP : 1];
   auto load_plane = [&](int z) {
 #pragma unroll
     for (int k = 0; k < KP; ++k) {
       if (tid + k * NT < HP) {
         const long o = pj1[k] + (long)n1 * (pj2[k] + (long)n2 * z);
         pre[k] = load_t6(sig, H, o);
-        if (RC == RHEO_EXT) pre_e[k] = trans ? load_t6(E, H, o) : T6{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (EXT) pre_e[k] = trans ? load_t6(E, H, o) : T6{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       }
     }
   };
@@ -107,11 +143,11 @@ __device__ __forceinline__ void bodyforce_tile(const Grid& g, const RheoParams& 
   load_plane(zs);
   for (int z = zs; z <= ze; ++z) {
     float* slot = &ring[z % 3][0][0];
-    T6 cur[KP], cur_e[RC == RHEO_EXT ? KP : 1];
+    T6 cur[KP], cur_e[EXT ? KP : 1];
 #pragma unroll
     for (int k = 0; k < KP; ++k) {
       cur[k] = pre[k];
-      if (RC == RHEO_EXT) cur_e[k] = pre_e[k];
+      if (EXT) cur_e[k] = pre_e[k];
     }
     if (z < ze) load_plane(z + 1);
 #pragma unroll
@@ -121,10 +157,10 @@ __device__ __forceinline__ void bodyforce_tile(const Grid& g, const RheoParams& 
         T6 m;
         if (RAW) {
           m = cur[k];
-        } else if (RC == RHEO_EXT) {
+        } else if (EXT) {
           T6 ed;
           const long o = pj1[k] + (long)n1 * (pj2[k] + (long)n2 * z);
-          m = rheology_ext<TM, !TM>(R, cur[k], pj1[k], pj2[k], z, o, cur_e[RC == RHEO_EXT ? k : 0], &ed, tmin,
+          m = rheology_ext<TM, !TM, PART == PART_IN>(R, cur[k], pj1[k], pj2[k], z, o, cur_e[EXT ? k : 0], &ed, tmin,
                                     nullptr, nullptr, &status);
           // the corrector's moment includes the inter-seismic loading
           if (!TM && R.inter) {
@@ -132,7 +168,7 @@ __device__ __forceinline__ void bodyforce_tile(const Grid& g, const RheoParams& 
             m = T6{m.s11 + a.s11, m.s12 + a.s12, m.s13 + a.s13, m.s22 + a.s22, m.s23 + a.s23, m.s33 + a.s33};
           }
         } else {
-          m = rheology<TM, RC == RHEO_CREEP>(R, cur[k], pj1[k], pj2[k], z, tmin, nullptr, nullptr, &status);
+          m = rheology<TM, PART == PART_IN>(R, cur[k], pj1[k], pj2[k], z, tmin, nullptr, nullptr, &status);
         }
         slot[e] = m.s11; slot[HP + e] = m.s12; slot[2 * HP + e] = m.s13;
         slot[3 * HP + e] = m.s22; slot[4 * HP + e] = m.s23; slot[5 * HP + e] = m.s33;
@@ -172,8 +208,9 @@ __device__ __forceinline__ void bodyforce_tile(const Grid& g, const RheoParams& 
 // that one barrier per plane suffices.  The first 2*(TXB+TYB) threads also
 // evaluate one halo point each, on the tile's output planes only; the planes
 // just above and below the depth chunk need only the tile's own points.
-// Every output is the same expression as in bodyforce_tile.
-template <int TXB, int TYB, bool TM, bool RAW, int RC>
+// Every output is the same expression as in bodyforce_tile.  BTY: the height
+// of the tiles whose band ranges split the two parts.
+template <int TXB, int TYB, bool TM, bool RAW, bool EXT, int PART, int BTY>
 __device__ __forceinline__ void bodyforce_tile_zr(const Grid& g, const RheoParams& R, const StencilConst& S,
                                                   const float* __restrict__ sig, const float* __restrict__ E,
                                                   float* __restrict__ W, float* __restrict__ T, StepScalars* sc,
@@ -182,7 +219,7 @@ __device__ __forceinline__ void bodyforce_tile_zr(const Grid& g, const RheoParam
   constexpr int HX = TXB + 2, HY = TYB + 2, HP = HX * HY;
   constexpr int NH = 2 * (TXB + TYB);  // halo points of one plane
   static_assert(NH <= NT, "one halo point per thread at most");
-  constexpr int NTM = RC == RHEO_EXT ? NMECH : 3;  // mechanisms whose minima are reduced
+  constexpr int NTM = EXT ? NMECH : 3;  // mechanisms whose minima are reduced
   __shared__ float pl[2][5][HP];
   __shared__ float rmin[NTM][NT / 64];
   const int tid = threadIdx.x;
@@ -190,12 +227,20 @@ __device__ __forceinline__ void bodyforce_tile_zr(const Grid& g, const RheoParam
   const int n1 = g.n1, n2 = g.n2, h3 = g.h3;
   const long H = g.H, P = (long)n1 * n2;
   const int x0 = bx * TXB, y0 = by * TYB;
-  const int z0 = (bz % gz) * zc, z1 = min(z0 + zc, h3);
+  int z0 = (bz % gz) * zc, z1 = min(z0 + zc, h3);
+  // planes [s0, s1) belong to PART_IN
+  int2 sk = make_int2(0, 0);
+  if (PART != PART_ALL) {
+    if (PART == PART_IN && z0 > R.fr.zmax) return;
+    sk = tile_band<TXB, BTY, NT>(R, g, x0, y0 & ~(BTY - 1));
+    if (PART == PART_IN) { z0 = max(z0, sk.x); z1 = min(z1, sk.y); }
+    if (z0 >= z1 || (PART == PART_OUT && z0 >= sk.x && z1 <= sk.y)) return;
+  }
   float tmin[NTM];
 #pragma unroll
   for (int k = 0; k < NTM; ++k) tmin[k] = __builtin_inff();
   int status = 0;
-  const bool trans = RC == RHEO_EXT && (R.tr[0].active || R.tr[1].active);
+  const bool trans = EXT && (R.tr[0].active || R.tr[1].active);
   // own point
   const int c1 = x0 + tx, c2 = y0 + ty;
   const int ec = (ty + 1) * HX + (tx + 1);
@@ -215,17 +260,17 @@ __device__ __forceinline__ void bodyforce_tile_zr(const Grid& g, const RheoParam
   T6 pc = zero, ph = zero, pce = zero, phe = zero;  // inputs of the next plane
   auto load_plane = [&](int z, bool halo) {
     pc = load_t6(sig, H, oc0 + P * z);
-    if (RC == RHEO_EXT && trans) pce = load_t6(E, H, oc0 + P * z);
+    if (EXT && trans) pce = load_t6(E, H, oc0 + P * z);
     if (halo && hal) {
       ph = load_t6(sig, H, oh0 + P * z);
-      if (RC == RHEO_EXT && trans) phe = load_t6(E, H, oh0 + P * z);
+      if (EXT && trans) phe = load_t6(E, H, oh0 + P * z);
     }
   };
   auto moment = [&](const T6& s, const T6& e, int p1, int p2, int z, long o) -> T6 {
     if (RAW) return s;
-    if (RC == RHEO_EXT) {
+    if (EXT) {
       T6 ed;
-      T6 m = rheology_ext<TM, !TM>(R, s, p1, p2, z, o, e, &ed, tmin, nullptr, nullptr, &status);
+      T6 m = rheology_ext<TM, !TM, PART == PART_IN>(R, s, p1, p2, z, o, e, &ed, tmin, nullptr, nullptr, &status);
       // the corrector's moment includes the inter-seismic loading
       if (!TM && R.inter) {
         const T6 a = load_t6(R.inter, H, o);
@@ -233,7 +278,7 @@ __device__ __forceinline__ void bodyforce_tile_zr(const Grid& g, const RheoParam
       }
       return m;
     }
-    return rheology<TM, RC == RHEO_CREEP>(R, s, p1, p2, z, tmin, nullptr, nullptr, &status);
+    return rheology<TM, PART == PART_IN>(R, s, p1, p2, z, tmin, nullptr, nullptr, &status);
   };
 
   const int zs = max(z0 - 1, 0), ze = min(z1, h3 - 1);
@@ -259,7 +304,7 @@ __device__ __forceinline__ void bodyforce_tile_zr(const Grid& g, const RheoParam
     }
     // plane z-1 is complete: its x3 differences take plane z below it
     const int zo = z - 1;
-    if (zo >= z0 && zo < z1) {
+    if (zo >= z0 && zo < z1 && !(PART == PART_OUT && zo >= sk.x && zo < sk.y)) {
       float v1, v2, v3;
       if (zo == 0) {
         v1 = (mc.s13 - b13) * S.idx3; v2 = (mc.s23 - b23) * S.idx3; v3 = (mc.s33 - b33) * S.idx3;
@@ -287,7 +332,7 @@ __device__ __forceinline__ void bodyforce_tile_zr(const Grid& g, const RheoParam
     b13 = mc.s13; b23 = mc.s23; b33 = mc.s33;
   }
   // the deepest plane of the grid: one-sided difference with the plane above
-  if (z1 == h3 && h3 - 1 >= z0) {
+  if (z1 == h3 && h3 - 1 >= z0 && !(PART == PART_OUT && h3 - 1 >= sk.x && h3 - 1 < sk.y)) {
     const int zo = h3 - 1;
     const long o = oc0 + P * zo;
     gst(W + o, -(f1 + (b13 - a13) * S.idx3));
@@ -317,36 +362,41 @@ __device__ __forceinline__ void bodyforce_tile_zr(const Grid& g, const RheoParam
   }
 }
 
+// The tiles of a launch: nx along x1 from x0 (periodic), ny along x2 from y0.
+struct TileBox {
+  int x0, nx, y0, ny;
+};
+
 // BATCH: the models' records are in the device array md (one model per
 // nx*ny*gz tiles); otherwise the one model's record is the argument Dv.
-template <int TXB, int TYB, bool TM, bool RAW, int RC, bool BATCH>
+template <int TXB, int TYB, bool TM, bool RAW, bool EXT, int PART, bool BATCH>
 __global__ __launch_bounds__(TXB* TYB) void k_bodyforce(Grid g, ModelDev Dv, const ModelDev* __restrict__ md,
-                                                        StencilConst S, int zc, int gz) {
+                                                        StencilConst S, int zc, int gz, TileBox tb) {
   // 1-D grid of tiles (x fastest, then y, depth chunk, model), taken in the
   // XCD-aware order so that neighbouring tiles, which share halo lines, meet
   // in one L2
-  const int nx = g.n1 / TXB, ny = g.n2 / TYB;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int bx = tile % nx, by = (tile / nx) % ny, bz = tile / (nx * ny);
+  const int bz = tile / (tb.nx * tb.ny);
+  const int bx = (tb.x0 + tile % tb.nx) % (g.n1 / TXB), by = (tb.y0 + (tile / tb.nx) % tb.ny) % (g.n2 / TYB);
   const ModelDev& D = BATCH ? md[bz / gz] : Dv;
-  bodyforce_tile<TXB, TYB, TM, RAW, RC>(g, D.R, S, RAW ? D.tau : D.sig, TM ? D.E : D.Em, D.W, D.T, D.sc, bx, by,
+  bodyforce_tile<TXB, TYB, TM, RAW, EXT, PART>(g, D.R, S, RAW ? D.tau : D.sig, TM ? D.E : D.Em, D.W, D.T, D.sc, bx, by,
                                          bz, zc, gz);
 }
 
-template <int TXB, int TYB, bool TM, bool RAW, int RC, bool BATCH>
+template <int TXB, int TYB, bool TM, bool RAW, bool EXT, int PART, int BTY, bool BATCH>
 __global__ __launch_bounds__(TXB* TYB) void k_bodyforce_zr(Grid g, ModelDev Dv, const ModelDev* __restrict__ md,
-                                                           StencilConst S, int zc, int gz) {
-  const int nx = g.n1 / TXB, ny = g.n2 / TYB;
+                                                           StencilConst S, int zc, int gz, TileBox tb) {
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int bx = tile % nx, by = (tile / nx) % ny, bz = tile / (nx * ny);
+  const int bz = tile / (tb.nx * tb.ny);
+  const int bx = (tb.x0 + tile % tb.nx) % (g.n1 / TXB), by = (tb.y0 + (tile / tb.nx) % tb.ny) % (g.n2 / TYB);
   const ModelDev& D = BATCH ? md[bz / gz] : Dv;
-  bodyforce_tile_zr<TXB, TYB, TM, RAW, RC>(g, D.R, S, RAW ? D.tau : D.sig, TM ? D.E : D.Em, D.W, D.T, D.sc, bx,
+  bodyforce_tile_zr<TXB, TYB, TM, RAW, EXT, PART, BTY>(g, D.R, S, RAW ? D.tau : D.sig, TM ? D.E : D.Em, D.W, D.T, D.sc, bx,
                                             by, bz, zc, gz);
 }
 
 // Hooke's law and the stage update of one point from its strain e (the
 // differences before the off-diagonal halving).  With transient creep
-// (RC == RHEO_EXT) the predictor also writes the mid-step strain
+// (EXT) the predictor also writes the mid-step strain
 // Em = E + Dt/2 Edot (relax.f90:690-692) and the corrector advances
 // E += Dt Edot (:792-793), Edot from the mid-step strain.  pw and ce collect
 // |moment| and |tau| of the corrector.
@@ -355,7 +405,7 @@ __global__ __launch_bounds__(TXB* TYB) void k_bodyforce_zr(Grid g, ModelDev Dv, 
 // caches to the stencil's neighbour reads of u or v (0.83 -> 0.75 ms for
 // the corrector at 512x512x256).  The divergence pass keeps cached loads of
 // the stress: its tiles re-read their halo rows.
-template <int MODE, int RC>
+template <int MODE, bool EXT, int PART>
 __device__ __forceinline__ void stress_point(const RheoParams& R, const StencilConst& S, long H, long o, int i1,
                                              int i2, int i3, T6 e, float* __restrict__ sig, float* __restrict__ tau,
                                              float* __restrict__ gam, float* __restrict__ E,
@@ -376,18 +426,18 @@ __device__ __forceinline__ void stress_point(const RheoParams& R, const StencilC
   } else if (MODE == STRESS_PRED) {
     const T6 s = load_t6_nt(sig, H, o);
     T6 m;
-    if (RC == RHEO_EXT) {
+    if (EXT) {
       const bool trans = R.tr[0].active || R.tr[1].active;
       const T6 ev = trans ? load_t6_nt(E, H, o) : T6{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       T6 ed;
-      m = rheology_ext<false, false>(R, s, i1, i2, i3, o, ev, &ed, nullptr, nullptr, nullptr, &status);
+      m = rheology_ext<false, false, PART == PART_IN>(R, s, i1, i2, i3, o, ev, &ed, nullptr, nullptr, nullptr, &status);
       if (trans) {
         const float h = (float)(sc->Dt / 2);
         store_t6_nt(Em, H, o, T6{h * ed.s11 + ev.s11, h * ed.s12 + ev.s12, h * ed.s13 + ev.s13,
                               h * ed.s22 + ev.s22, h * ed.s23 + ev.s23, h * ed.s33 + ev.s33});
       }
     } else {
-      m = rheology<false, RC == RHEO_CREEP>(R, s, i1, i2, i3, nullptr, nullptr, nullptr, &status);
+      m = rheology<false, PART == PART_IN>(R, s, i1, i2, i3, nullptr, nullptr, nullptr, &status);
     }
     const float c = -(float)(sc->Dt / 2);
     out = T6{(c * m.s11 - t.s11) + e.s11, (c * m.s12 - t.s12) + e.s12, (c * m.s13 - t.s13) + e.s13,
@@ -397,21 +447,21 @@ __device__ __forceinline__ void stress_point(const RheoParams& R, const StencilC
     float gl = 0.f, gn = 0.f;
     const float dt = (float)sc->Dt;
     T6 m;
-    if (RC == RHEO_EXT) {
+    if (EXT) {
       const bool trans = R.tr[0].active || R.tr[1].active;
       const T6 em = trans ? load_t6_nt(Em, H, o) : T6{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       T6 ed;
-      m = rheology_ext<false, true>(R, s, i1, i2, i3, o, em, &ed, nullptr, &gl, &gn, &status);
+      m = rheology_ext<false, true, PART == PART_IN>(R, s, i1, i2, i3, o, em, &ed, nullptr, &gl, &gn, &status);
       if (trans) {
         const T6 ev = load_t6_nt(E, H, o);
         store_t6_nt(E, H, o, T6{ev.s11 + dt * ed.s11, ev.s12 + dt * ed.s12, ev.s13 + dt * ed.s13,
                              ev.s22 + dt * ed.s22, ev.s23 + dt * ed.s23, ev.s33 + dt * ed.s33});
       }
     } else {
-      m = rheology<false, RC == RHEO_CREEP>(R, s, i1, i2, i3, nullptr, &gl, &gn, &status);
+      m = rheology<false, PART == PART_IN>(R, s, i1, i2, i3, nullptr, &gl, &gn, &status);
     }
     T6 t0 = t;
-    if (RC == RHEO_EXT && R.inter) {
+    if (EXT && R.inter) {
       // inter-seismic loading: its moment density joins the corrector's
       // moment and, unscaled, tau (relax.f90:795-799, :1199-1206), before
       // tau += Dt moment (:833)
@@ -436,8 +486,9 @@ __device__ __forceinline__ void stress_point(const RheoParams& R, const StencilC
   store_t6_nt(sig, H, o, out);
 }
 
-// The corrector's |moment| and |tau| sums of a workgroup, in a fixed order.
-template <int NT>
+// The corrector's |moment| and |tau| sums of a workgroup, in a fixed order;
+// ADD: to those that the launch over the other points left.
+template <int NT, bool ADD>
 __device__ __forceinline__ void block_partials(double pw, double ce, double2* __restrict__ partials, int idx) {
   __shared__ double2 red[NT / 64];
   const int tid = threadIdx.x;
@@ -450,6 +501,7 @@ __device__ __forceinline__ void block_partials(double pw, double ce, double2* __
   if (tid == 0) {
     double2 a = red[0];
     for (int w = 1; w < NT / 64; ++w) { a.x += red[w].x; a.y += red[w].y; }
+    if (ADD) { a.x += partials[idx].x; a.y += partials[idx].y; }
     partials[idx] = a;
   }
 }
@@ -460,52 +512,120 @@ __device__ __forceinline__ void block_partials(double pw, double ce, double2* __
 // serves.  64x4 tiles marched down 8 or 16 planes with the x3 neighbours in
 // registers lost the same way: 104 VGPRs against 68 in the predictor form,
 // 0.63 ms against 0.56 ms.)
-template <int MODE, int RC>
+// strain of point (i1,i2,i3) = o from the differences of X, then its stage
+// update
+template <int MODE, bool EXT, int PART>
+__device__ __forceinline__ void stress_at(const Grid& g, const RheoParams& R, const StencilConst& S,
+                                          const float* __restrict__ X, float* __restrict__ sig,
+                                          float* __restrict__ tau, float* __restrict__ gam, float* __restrict__ E,
+                                          float* __restrict__ Em, const StepScalars* sc, long o, int i1, int i2, int i3,
+                                          double& pw, double& ce, int& status) {
+  const int n1 = g.n1, n2 = g.n2, h3 = g.h3;
+  const long H = g.H;
+  const long row = o - i1;
+  const long xp = row + (i1 + 1 == n1 ? 0 : i1 + 1), xm = row + (i1 == 0 ? n1 - 1 : i1 - 1);
+  const long plane = (long)n1 * n2;
+  const long pbase = o - (long)i2 * n1;
+  const long yp = pbase + (long)(i2 + 1 == n2 ? 0 : i2 + 1) * n1, ym = pbase + (long)(i2 == 0 ? n2 - 1 : i2 - 1) * n1;
+  long zp, zm;
+  float wz;
+  if (i3 == 0) { zp = o + plane; zm = o; wz = S.idx3; }
+  else if (i3 == h3 - 1) { zp = o; zm = o - plane; wz = S.idx3; }
+  else { zp = o + plane; zm = o - plane; wz = S.k3h; }
+  const float* X0 = X;
+  const float* X1 = X + H;
+  const float* X2 = X + 2 * H;
+  T6 e;
+  e.s11 = (gld(X0 + xp) - gld(X0 + xm)) * S.k1h;
+  e.s12 = (gld(X1 + xp) - gld(X1 + xm)) * S.k1h;
+  e.s13 = (gld(X2 + xp) - gld(X2 + xm)) * S.k1h;
+  e.s12 = e.s12 + (gld(X0 + yp) - gld(X0 + ym)) * S.k2h;
+  e.s22 = (gld(X1 + yp) - gld(X1 + ym)) * S.k2h;
+  e.s23 = (gld(X2 + yp) - gld(X2 + ym)) * S.k2h;
+  e.s13 = e.s13 + (gld(X0 + zp) - gld(X0 + zm)) * wz;
+  e.s23 = e.s23 + (gld(X1 + zp) - gld(X1 + zm)) * wz;
+  e.s33 = (gld(X2 + zp) - gld(X2 + zm)) * wz;
+  stress_point<MODE, EXT, PART>(R, S, H, o, i1, i2, i3, e, sig, tau, gam, E, Em, sc, pw, ce, status);
+}
+
+template <int MODE, bool EXT, int PART>
 __device__ __forceinline__ void stress_block(const Grid& g, const RheoParams& R, const StencilConst& S,
                                              const float* __restrict__ X, float* __restrict__ sig,
                                              float* __restrict__ tau, float* __restrict__ gam,
                                              float* __restrict__ E, float* __restrict__ Em, StepScalars* sc,
                                              double2* __restrict__ partials, int blk) {
-  const int tid = threadIdx.x;
   // block blk: 256 points in address order (the corrector's partials go to
   // entry blk, so their sum keeps one order whatever the launch order of
   // the blocks; an order in which each XCD walks a contiguous eighth of the
   // grid measured 9-15 % slower at 512x512x256, see slab_tile)
-  const long o = (long)blk * 256 + tid;
-  const int n1 = g.n1, n2 = g.n2, h3 = g.h3;
-  const long H = g.H;
+  const long o = (long)blk * 256 + threadIdx.x;
   double pw = 0.0, ce = 0.0;
   int status = 0;
-  if (o < H) {
-    // n1 and n2 are powers of two (relax_model_create): shifts and masks
-    const int l1 = __builtin_ctz((unsigned)n1), l2 = __builtin_ctz((unsigned)n2);
-    const int i1 = (int)(o & (n1 - 1)), i2 = (int)((o >> l1) & (n2 - 1)), i3 = (int)(o >> (l1 + l2));
-    const long row = o - i1;
-    const long xp = row + (i1 + 1 == n1 ? 0 : i1 + 1), xm = row + (i1 == 0 ? n1 - 1 : i1 - 1);
-    const long plane = (long)n1 * n2;
-    const long pbase = o - (long)i2 * n1;
-    const long yp = pbase + (long)(i2 + 1 == n2 ? 0 : i2 + 1) * n1, ym = pbase + (long)(i2 == 0 ? n2 - 1 : i2 - 1) * n1;
-    long zp, zm;
-    float wz;
-    if (i3 == 0) { zp = o + plane; zm = o; wz = S.idx3; }
-    else if (i3 == h3 - 1) { zp = o; zm = o - plane; wz = S.idx3; }
-    else { zp = o + plane; zm = o - plane; wz = S.k3h; }
-    const float* X0 = X;
-    const float* X1 = X + H;
-    const float* X2 = X + 2 * H;
-    T6 e;
-    e.s11 = (gld(X0 + xp) - gld(X0 + xm)) * S.k1h;
-    e.s12 = (gld(X1 + xp) - gld(X1 + xm)) * S.k1h;
-    e.s13 = (gld(X2 + xp) - gld(X2 + xm)) * S.k1h;
-    e.s12 = e.s12 + (gld(X0 + yp) - gld(X0 + ym)) * S.k2h;
-    e.s22 = (gld(X1 + yp) - gld(X1 + ym)) * S.k2h;
-    e.s23 = (gld(X2 + yp) - gld(X2 + ym)) * S.k2h;
-    e.s13 = e.s13 + (gld(X0 + zp) - gld(X0 + zm)) * wz;
-    e.s23 = e.s23 + (gld(X1 + zp) - gld(X1 + zm)) * wz;
-    e.s33 = (gld(X2 + zp) - gld(X2 + zm)) * wz;
-    stress_point<MODE, RC>(R, S, H, o, i1, i2, i3, e, sig, tau, gam, E, Em, sc, pw, ce, status);
+  // n1 and n2 are powers of two (relax_model_create): shifts and masks
+  const int l1 = __builtin_ctz((unsigned)g.n1), l2 = __builtin_ctz((unsigned)g.n2);
+  const int i1 = (int)(o & (g.n1 - 1)), i2 = (int)((o >> l1) & (g.n2 - 1)), i3 = (int)(o >> (l1 + l2));
+  bool mine = o < g.H;
+  if (PART == PART_OUT) mine = mine && !(R.fr.active && in_band(R, i1, i2, i3));
+  if (mine) stress_at<MODE, EXT, PART>(g, R, S, X, sig, tau, gam, E, Em, sc, o, i1, i2, i3, pw, ce, status);
+  if (MODE == STRESS_CORR) block_partials<256, false>(pw, ce, partials, blk);
+  if (status) atomicMax(&sc->status, status);
+}
+
+// The points in the creep bands among blocks [b0, b1) (at most SEGS) of 256:
+// a point with the creep code costs ten viscous ones and the bands hold a few
+// points of every block they cross, so the workgroup first gathers the points
+// of its blocks (in address order: the sums keep one order), then takes them
+// 256 at a time: at 256x256x128 with a plane of 38x16 km 22 us (corrector)
+// beside 99 us for the other points, against 155 us for one kernel with the
+// creep code and 49 us for a band launch without the gathering.  Their sums are added to those that the launch over the other
+// points left in entry b0.
+constexpr int SEGS = 16;
+template <int MODE, bool EXT>
+__device__ __forceinline__ void stress_band(const Grid& g, const RheoParams& R, const StencilConst& S,
+                                            const float* __restrict__ X, float* __restrict__ sig,
+                                            float* __restrict__ tau, float* __restrict__ gam, float* __restrict__ E,
+                                            float* __restrict__ Em, StepScalars* sc, double2* __restrict__ partials,
+                                            int b0, int b1) {
+  __shared__ unsigned short q[SEGS * 256];
+  __shared__ unsigned long long mask[SEGS * 4];
+  __shared__ int base[SEGS * 4 + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int l1 = __builtin_ctz((unsigned)g.n1), l2 = __builtin_ctz((unsigned)g.n2);
+  if (!R.fr.active || (((long)b0 * 256) >> (l1 + l2)) >= R.fr.zmax) return;
+  const int ns = b1 - b0;
+  for (int s = 0; s < ns; ++s) {
+    const long o = (long)(b0 + s) * 256 + tid;
+    const bool in = in_band(R, (int)(o & (g.n1 - 1)), (int)((o >> l1) & (g.n2 - 1)), (int)(o >> (l1 + l2)));
+    const unsigned long long m = __ballot(in);
+    if (lane == 0) mask[4 * s + wave] = m;
   }
-  if (MODE == STRESS_CORR) block_partials<256>(pw, ce, partials, blk);
+  __syncthreads();
+  if (wave == 0) {
+    int c = lane < 4 * ns ? __popcll(mask[lane]) : 0, t = c;
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(t, off);
+      if (lane >= off) t += v;
+    }
+    base[lane] = t - c;
+    if (lane == 63) base[64] = t;
+  }
+  __syncthreads();
+  const int n = base[64];
+  if (n == 0) return;
+  for (int s = 0; s < ns; ++s) {
+    const unsigned long long m = mask[4 * s + wave];
+    if ((m >> lane) & 1)
+      q[base[4 * s + wave] + __popcll(m & ((1ull << lane) - 1))] = (unsigned short)(256 * s + tid);
+  }
+  __syncthreads();
+  double pw = 0.0, ce = 0.0;
+  int status = 0;
+  for (int i = tid; i < n; i += 256) {
+    const long o = (long)b0 * 256 + q[i];
+    stress_at<MODE, EXT, PART_IN>(g, R, S, X, sig, tau, gam, E, Em, sc, o, (int)(o & (g.n1 - 1)),
+                                  (int)((o >> l1) & (g.n2 - 1)), (int)(o >> (l1 + l2)), pw, ce, status);
+  }
+  if (MODE == STRESS_CORR) block_partials<256, true>(pw, ce, partials, b0);
   if (status) atomicMax(&sc->status, status);
 }
 
@@ -525,14 +645,25 @@ __device__ __forceinline__ int slab_tile(int b, int nb, int P) {
   return (l / q) * P + x * q + l % q;
 }
 
-template <int MODE, int RC, bool BATCH>
+template <int MODE, bool EXT, int PART, bool BATCH>
 __global__ __launch_bounds__(256) void k_stress(Grid g, ModelDev Dv, const ModelDev* __restrict__ md,
                                                StencilConst S) {
   // model blockIdx.y of the launch (BATCH) or the argument Dv
   const ModelDev& D = BATCH ? md[blockIdx.y] : Dv;
   const int blk = slab_tile(blockIdx.x, gridDim.x, (g.n1 * g.n2) / 256);
-  stress_block<MODE, RC>(g, D.R, S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em, D.sc,
+  stress_block<MODE, EXT, PART>(g, D.R, S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em, D.sc,
                          D.partials, blk);
+}
+
+// segs blocks of 256 points per workgroup
+template <int MODE, bool EXT, bool BATCH>
+__global__ __launch_bounds__(256) void k_stress_band(Grid g, ModelDev Dv, const ModelDev* __restrict__ md,
+                                                    StencilConst S, int segs) {
+  const ModelDev& D = BATCH ? md[blockIdx.y] : Dv;
+  const int b0 = blockIdx.x * segs, nb = (int)(g.H / 256);
+  if (b0 >= nb) return;
+  stress_band<MODE, EXT>(g, D.R, S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em, D.sc, D.partials,
+                         b0, min(b0 + segs, nb));
 }
 
 // ---------------------------------------------- models of uneven grids ----
@@ -554,20 +685,36 @@ __device__ __forceinline__ int work_model(const WorkItem* __restrict__ wl, int n
   return lo;
 }
 
-template <int MODE, int RC>
+template <int MODE, bool EXT, int PART>
 __global__ __launch_bounds__(256) void k_stress_list(const ModelDev* __restrict__ md,
                                                      const WorkItem* __restrict__ wl, int nm) {
   const long total = wl[nm].first;
   for (long item = blockIdx.x; item < total; item += gridDim.x) {
     const int m = work_model(wl, nm, item);
     const ModelDev& D = md[m];
-    stress_block<MODE, RC>(wl[m].g, D.R, wl[m].S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em,
+    stress_block<MODE, EXT, PART>(wl[m].g, D.R, wl[m].S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em,
                            D.sc, D.partials, (int)(item - wl[m].first));
     if (MODE == STRESS_CORR) __syncthreads();  // the partials' LDS is reused by the next item
   }
 }
 
-template <int TXB, int TYB, bool TM, bool RAW, int RC, bool ZR>
+// items in groups of SEGS, as many as belong to one model
+template <int MODE, bool EXT>
+__global__ __launch_bounds__(256) void k_stress_band_list(const ModelDev* __restrict__ md,
+                                                          const WorkItem* __restrict__ wl, int nm) {
+  const long total = wl[nm].first, last = min(total, ((long)blockIdx.x + 1) * SEGS);
+  for (long item = (long)blockIdx.x * SEGS; item < last;) {
+    const int m = work_model(wl, nm, item);
+    const ModelDev& D = md[m];
+    const long end = min(last, wl[m + 1].first);
+    stress_band<MODE, EXT>(wl[m].g, D.R, wl[m].S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em,
+                           D.sc, D.partials, (int)(item - wl[m].first), (int)(end - wl[m].first));
+    __syncthreads();  // the lists in LDS are reused
+    item = end;
+  }
+}
+
+template <int TXB, int TYB, bool TM, bool RAW, bool EXT, int PART, int BTY, bool ZR>
 __global__ __launch_bounds__(TXB* TYB) void k_bodyforce_list(const ModelDev* __restrict__ md,
                                                              const WorkItem* __restrict__ wl, int nm, int zc) {
   const long total = wl[nm].first;
@@ -580,10 +727,10 @@ __global__ __launch_bounds__(TXB* TYB) void k_bodyforce_list(const ModelDev* __r
     const int lt = (int)(item - wl[m].first);
     const int bx = lt % nx, by = (lt / nx) % ny, bz = lt / (nx * ny);
     if constexpr (ZR)
-      bodyforce_tile_zr<TXB, TYB, TM, RAW, RC>(g, D.R, wl[m].S, RAW ? D.tau : D.sig, TM ? D.E : D.Em, D.W, D.T,
+      bodyforce_tile_zr<TXB, TYB, TM, RAW, EXT, PART, BTY>(g, D.R, wl[m].S, RAW ? D.tau : D.sig, TM ? D.E : D.Em, D.W, D.T,
                                                D.sc, bx, by, bz, zc, gz);
     else
-      bodyforce_tile<TXB, TYB, TM, RAW, RC>(g, D.R, wl[m].S, RAW ? D.tau : D.sig, TM ? D.E : D.Em, D.W, D.T, D.sc,
+      bodyforce_tile<TXB, TYB, TM, RAW, EXT, PART>(g, D.R, wl[m].S, RAW ? D.tau : D.sig, TM ? D.E : D.Em, D.W, D.T, D.sc,
                                             bx, by, bz, zc, gz);
     __syncthreads();  // the tile's LDS is reused by the next item
   }
@@ -606,8 +753,10 @@ static int device_cus() {
 // Depth chunk of one divergence tile: each chunk re-reads the plane above
 // and below it.  The register-window forms (variants 4 and 5: one workgroup
 // of 64x16 tiles per CU, two of 64x8, at their register use) take the
-// deepest chunk that still gives every CU a workgroup, at least 8 planes:
-// at 512x512x256 one chunk of all 128 planes (256 workgroups) runs the
+// deepest chunk that still gives every CU a workgroup, at least 2 planes (a
+// small grid's launch lasts as long as one workgroup's chain of planes:
+// 64x64x64 takes 7.6 us in chunks of 2, 9.9 of 4, 15.1 of 8; 128^3 14.1 us in
+// chunks of 4, 17.1 of 8): at 512x512x256 one chunk of all 128 planes (256 workgroups) runs the
 // divergence in 0.250 ms against 0.275 ms for chunks of 32 planes (1024
 // workgroups, four rounds) and 0.268 ms for 64.
 int body_depth_chunk(const Grid& g, int variant, int nm) {
@@ -616,10 +765,79 @@ int body_depth_chunk(const Grid& g, int variant, int nm) {
   if (tiles <= 0) return 32;  // the tiles do not fit the grid: the launcher refuses it
   const long want = (long)device_cus() * (variant == 5 ? 1 : 2);
   long gz = (want + tiles - 1) / tiles;
-  const long gmax = (g.h3 + 7) / 8;
+  const long gmax = (g.h3 + 1) / 2;
   if (gz > gmax) gz = gmax;
   if (gz < 1) gz = 1;
   return (int)((g.h3 + gz - 1) / gz);
+}
+
+// One divergence kernel over one part of the models, chunks of zc planes, gz
+// of them
+struct BodyLaunch {
+  Grid g;
+  ModelDev Dv;
+  const ModelDev* md;
+  StencilConst S;
+  int nm, mode;
+  bool batch;
+  hipStream_t st;
+};
+template <int TX, int TY, bool ZR, bool TM, bool RAW, bool EXT, int PART, int BTY>
+static void body_launch(const BodyLaunch& b, int zc, int gz, TileBox tb) {
+  const dim3 grid((unsigned)(tb.nx * tb.ny * gz * b.nm));
+  if constexpr (ZR) {
+    if (b.batch) k_bodyforce_zr<TX, TY, TM, RAW, EXT, PART, BTY, true><<<grid, TX * TY, 0, b.st>>>(b.g, b.Dv, b.md, b.S, zc, gz, tb);
+    else k_bodyforce_zr<TX, TY, TM, RAW, EXT, PART, BTY, false><<<grid, TX * TY, 0, b.st>>>(b.g, b.Dv, b.md, b.S, zc, gz, tb);
+  } else {
+    if (b.batch) k_bodyforce<TX, TY, TM, RAW, EXT, PART, true><<<grid, TX * TY, 0, b.st>>>(b.g, b.Dv, b.md, b.S, zc, gz, tb);
+    else k_bodyforce<TX, TY, TM, RAW, EXT, PART, false><<<grid, TX * TY, 0, b.st>>>(b.g, b.Dv, b.md, b.S, zc, gz, tb);
+  }
+}
+template <int TX, int TY, bool ZR, bool EXT, int PART, int BTY>
+static void body_mode(const BodyLaunch& b, int zc, int gz, TileBox tb) {
+  if (b.mode == BODY_PRED) body_launch<TX, TY, ZR, true, false, EXT, PART, BTY>(b, zc, gz, tb);
+  else body_launch<TX, TY, ZR, false, false, EXT, PART, BTY>(b, zc, gz, tb);
+}
+// the tiles of T samples that reach samples [x0-1, x0+nx] of n (with a tile's
+// halo), from tile *t0
+static int tiles_of(int x0, int nx, int n, int T, int* t0) {
+  const int nt = n / T, a = (x0 + n - 1) / T, c = (x0 + n + nx) / T - a + 1;
+  *t0 = c >= nt ? 0 : a % nt;
+  return std::min(c, nt);
+}
+// Creeping planes: the points outside the bands on the tiles of the variant;
+// then the bands, on the same tiles in chunks of a few planes.  A tile's band
+// is some 20 planes deep and its points cost ten times a viscous one, so the
+// bands want many short chunks (2 planes, more where that made over 2048
+// workgroups), of the tiles in the bands' box only: at 256x256x128 with a
+// plane of 38x16 km the bands take 26 us beside 34 us (64x16) or 60 us (32x16)
+// for the rest, against 142 us for one kernel with the creep code over all
+// points.  The 64x16
+// tiles' bands go to 64x8 ones (at 1024 threads the creep code spills 40-137
+// registers).
+template <int TX, int TY, bool ZR, bool EXT>
+static void body_parts(const BodyLaunch& b, int rclass, int zc, int gz) {
+  const TileBox all{0, b.g.n1 / TX, 0, b.g.n2 / TY};
+  if (!(rclass & RHEO_CREEP)) {
+    body_mode<TX, TY, ZR, EXT, PART_ALL, TY>(b, zc, gz, all);
+    return;
+  }
+  body_mode<TX, TY, ZR, EXT, PART_OUT, TY>(b, zc, gz, all);
+  constexpr int IY = TX * TY > 512 ? TY / 2 : TY;
+  TileBox box{0, b.g.n1 / TX, 0, b.g.n2 / IY};
+  int depth = b.g.h3;
+  if (!b.batch) {
+    const FrictionTables& F = b.Dv.R.fr;
+    box.nx = tiles_of(F.x0, F.nx, b.g.n1, TX, &box.x0);
+    // whole tiles of the variant, as the ranges are theirs
+    box.ny = tiles_of(F.y0, F.ny, b.g.n2, TY, &box.y0) * (TY / IY);
+    box.y0 *= TY / IY;
+    depth = std::min(depth, F.zmax + 1);
+  }
+  const long tiles = (long)box.nx * box.ny * b.nm;
+  int zi = 2;
+  while (zi < b.g.h3 && tiles * ((depth + zi - 1) / zi) > 2048) zi *= 2;
+  body_mode<TX, IY, ZR, EXT, PART_IN, TY>(b, zi, (depth + zi - 1) / zi, box);
 }
 
 int launch_bodyforce(const Grid& g, const StencilConst& S, const ModelDev* md, const ModelDev* one, int nm,
@@ -627,35 +845,25 @@ int launch_bodyforce(const Grid& g, const StencilConst& S, const ModelDev* md, c
   const int zc = body_depth_chunk(g, variant, nm);
   const int gz = (g.h3 + zc - 1) / zc;
   const bool batch = !(one && nm == 1);
-  const ModelDev Dv = batch ? ModelDev{} : *one;
-  if (rclass < RHEO_VISCOUS || rclass > RHEO_EXT) return RELAX_ERR_ARG;
-#define LB(K, TX, TY, F, B)                                                                                 \
-  {                                                                                                      \
-    const dim3 grid((unsigned)((g.n1 / TX) * (g.n2 / TY) * gz * nm));                                    \
-    if (mode == BODY_PRED) K<TX, TY, true, false, F, B><<<grid, TX * TY, 0, st>>>(g, Dv, md, S, zc, gz); \
-    else if (mode == BODY_CORR) K<TX, TY, false, false, F, B><<<grid, TX * TY, 0, st>>>(g, Dv, md, S, zc, gz); \
-    else K<TX, TY, false, true, RHEO_VISCOUS, B><<<grid, TX * TY, 0, st>>>(g, Dv, md, S, zc, gz); \
-  }
-#define LF(K, TX, TY, F) { if (batch) LB(K, TX, TY, F, true) else LB(K, TX, TY, F, false) }
-#define L(K, TX, TY)                                   \
-  {                                                 \
-    if (rclass == RHEO_EXT) LF(K, TX, TY, RHEO_EXT)    \
-    else if (rclass == RHEO_CREEP) LF(K, TX, TY, RHEO_CREEP) \
-    else LF(K, TX, TY, RHEO_VISCOUS)                   \
+  if (rclass < RHEO_VISCOUS || rclass > RHEO_ALL) return RELAX_ERR_ARG;
+  const BodyLaunch b{g, batch ? ModelDev{} : *one, md, S, nm, mode, batch, st};
+#define L(TX, TY, ZR)                                                                                        \
+  {                                                                                                          \
+    if (mode == BODY_RAW) body_launch<TX, TY, ZR, false, true, false, PART_ALL, TY>(b, zc, gz, TileBox{0, g.n1 / TX, 0, g.n2 / TY}); \
+    else if (rclass & RHEO_EXT) body_parts<TX, TY, ZR, true>(b, rclass, zc, gz);                             \
+    else body_parts<TX, TY, ZR, false>(b, rclass, zc, gz);                                                   \
   }
   // variant 0: 32x16 tiles, 1: 32x8 tiles, 2: 64x8 tiles, 3: 64x8 tiles
   // 32 planes deep (16 for the others); 4 and 5: 64x8 and 64x16 tiles with
   // the x3 differences in registers (k_bodyforce_zr), body_depth_chunk deep
   if (variant < 0 || variant >= BODY_VARIANTS) return RELAX_ERR_ARG;
-  if (variant == 4 && g.n1 % 64 == 0 && g.n2 % 8 == 0) L(k_bodyforce_zr, 64, 8)
-  else if (variant == 5 && g.n1 % 64 == 0 && g.n2 % 16 == 0) L(k_bodyforce_zr, 64, 16)
+  if (variant == 4 && g.n1 % 64 == 0 && g.n2 % 8 == 0) L(64, 8, true)
+  else if (variant == 5 && g.n1 % 64 == 0 && g.n2 % 16 == 0) L(64, 16, true)
   else if (variant >= 4) return RELAX_ERR_SIZE;
-  else if (variant == 0 && g.n1 % 32 == 0 && g.n2 % 16 == 0) L(k_bodyforce, 32, 16)
-  else if (variant >= 2 && g.n1 % 64 == 0 && g.n2 % 8 == 0) L(k_bodyforce, 64, 8)
-  else if (variant != 2 && g.n1 % 32 == 0 && g.n2 % 8 == 0) L(k_bodyforce, 32, 8)
+  else if (variant == 0 && g.n1 % 32 == 0 && g.n2 % 16 == 0) L(32, 16, false)
+  else if (variant >= 2 && g.n1 % 64 == 0 && g.n2 % 8 == 0) L(64, 8, false)
+  else if (variant != 2 && g.n1 % 32 == 0 && g.n2 % 8 == 0) L(32, 8, false)
   else return RELAX_ERR_SIZE;
-#undef LB
-#undef LF
 #undef L
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
@@ -664,25 +872,39 @@ long stress_blocks(const Grid& g) { return (g.H + 255) / 256; }
 
 int launch_stress(int mode, const Grid& g, const StencilConst& S, const ModelDev* md, const ModelDev* one, int nm,
                   int rclass, hipStream_t st) {
-  const dim3 grid((unsigned)stress_blocks(g), (unsigned)nm);
   const bool batch = !(one && nm == 1);
   const ModelDev Dv = batch ? ModelDev{} : *one;
-  if (rclass < RHEO_VISCOUS || rclass > RHEO_EXT) return RELAX_ERR_ARG;
-#define K(MODE, F)                                                          \
-  {                                                                         \
-    if (batch) k_stress<MODE, F, true><<<grid, 256, 0, st>>>(g, Dv, md, S);  \
-    else k_stress<MODE, F, false><<<grid, 256, 0, st>>>(g, Dv, md, S);       \
+  if (rclass < RHEO_VISCOUS || rclass > RHEO_ALL) return RELAX_ERR_ARG;
+  const dim3 grid((unsigned)stress_blocks(g), (unsigned)nm);
+  // the creep bands' part: no deeper than they reach, as many blocks per
+  // workgroup as leave two workgroups per CU (their registers admit two)
+  const long nin = batch ? stress_blocks(g) : std::min(stress_blocks(g), ((long)g.n1 * g.n2 * Dv.R.fr.zmax + 255) / 256);
+  const int segs = (int)std::max(1L, std::min((long)SEGS, nin * nm / (2 * device_cus())));
+  const dim3 gin((unsigned)std::max(1L, (nin + segs - 1) / segs), (unsigned)nm);
+#define K(MODE, E, PART, GR)                                                     \
+  {                                                                              \
+    if (batch) k_stress<MODE, E, PART, true><<<GR, 256, 0, st>>>(g, Dv, md, S);  \
+    else k_stress<MODE, E, PART, false><<<GR, 256, 0, st>>>(g, Dv, md, S);       \
   }
-#define KM(MODE)                                          \
-  {                                                       \
-    if (rclass == RHEO_EXT) K(MODE, RHEO_EXT)             \
-    else if (rclass == RHEO_CREEP) K(MODE, RHEO_CREEP)    \
-    else K(MODE, RHEO_VISCOUS)                            \
+#define KP(MODE, E)                                                          \
+  {                                                                          \
+    if (!(rclass & RHEO_CREEP)) K(MODE, E, PART_ALL, grid)                   \
+    else {                                                                   \
+      K(MODE, E, PART_OUT, grid)                                             \
+      if (batch) k_stress_band<MODE, E, true><<<gin, 256, 0, st>>>(g, Dv, md, S, segs); \
+      else k_stress_band<MODE, E, false><<<gin, 256, 0, st>>>(g, Dv, md, S, segs);      \
+    }                                                                        \
   }
-  if (mode == STRESS_SET) K(STRESS_SET, RHEO_VISCOUS)
+#define KM(MODE)                          \
+  {                                       \
+    if (rclass & RHEO_EXT) KP(MODE, true) \
+    else KP(MODE, false)                  \
+  }
+  if (mode == STRESS_SET) K(STRESS_SET, false, PART_ALL, grid)
   else if (mode == STRESS_PRED) KM(STRESS_PRED)
   else KM(STRESS_CORR)
 #undef K
+#undef KP
 #undef KM
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
@@ -704,24 +926,34 @@ long body_items(const Grid& g, int variant) {
   return (long)(g.n1 / TX[variant]) * (g.n2 / TY[variant]) * ((g.h3 + zc - 1) / zc);
 }
 
+template <int TX, int TY, bool ZR, bool EXT, int PART, int BTY>
+static void body_list(const WorkItem* wl, const ModelDev* md, int nm, unsigned gx, int mode, int zc, hipStream_t st) {
+  if (mode == BODY_PRED)
+    k_bodyforce_list<TX, TY, true, false, EXT, PART, BTY, ZR><<<gx, TX * TY, 0, st>>>(md, wl, nm, zc);
+  else
+    k_bodyforce_list<TX, TY, false, false, EXT, PART, BTY, ZR><<<gx, TX * TY, 0, st>>>(md, wl, nm, zc);
+}
+
 int launch_bodyforce_list(const WorkItem* wl, const ModelDev* md, int nm, long total, long grid, int rclass,
                           int mode, hipStream_t st, int variant) {
-  if (rclass < RHEO_VISCOUS || rclass > RHEO_EXT || variant < 0 || variant >= BODY_VARIANTS || nm < 1)
+  if (rclass < RHEO_VISCOUS || rclass > RHEO_ALL || variant < 0 || variant >= BODY_VARIANTS || nm < 1 ||
+      mode == BODY_RAW)
     return RELAX_ERR_ARG;
   if (total < 1) return RELAX_OK;
   const int zc = variant >= 3 ? 32 : 16;
   const unsigned gx = (unsigned)(grid > 0 && grid < total ? grid : total);
-#define LB(TX, TY, ZR, F)                                                                                     \
-  {                                                                                                           \
-    if (mode == BODY_PRED) k_bodyforce_list<TX, TY, true, false, F, ZR><<<gx, TX * TY, 0, st>>>(md, wl, nm, zc); \
-    else if (mode == BODY_CORR) k_bodyforce_list<TX, TY, false, false, F, ZR><<<gx, TX * TY, 0, st>>>(md, wl, nm, zc); \
-    else k_bodyforce_list<TX, TY, false, true, RHEO_VISCOUS, ZR><<<gx, TX * TY, 0, st>>>(md, wl, nm, zc); \
+#define LP(TX, TY, ZR, E)                                                                  \
+  {                                                                                        \
+    if (!(rclass & RHEO_CREEP)) body_list<TX, TY, ZR, E, PART_ALL, TY>(wl, md, nm, gx, mode, zc, st); \
+    else {                                                                                 \
+      body_list<TX, TY, ZR, E, PART_OUT, TY>(wl, md, nm, gx, mode, zc, st);                \
+      body_list<TX, TY, ZR, E, PART_IN, TY>(wl, md, nm, gx, mode, zc, st);                 \
+    }                                                                                      \
   }
-#define L(TX, TY, ZR)                                         \
-  {                                                           \
-    if (rclass == RHEO_EXT) LB(TX, TY, ZR, RHEO_EXT)          \
-    else if (rclass == RHEO_CREEP) LB(TX, TY, ZR, RHEO_CREEP) \
-    else LB(TX, TY, ZR, RHEO_VISCOUS)                         \
+#define L(TX, TY, ZR)                          \
+  {                                            \
+    if (rclass & RHEO_EXT) LP(TX, TY, ZR, true) \
+    else LP(TX, TY, ZR, false)                 \
   }
   switch (variant) {
     case 0: L(32, 16, false) break;
@@ -730,27 +962,34 @@ int launch_bodyforce_list(const WorkItem* wl, const ModelDev* md, int nm, long t
     case 4: L(64, 8, true) break;
     default: L(64, 16, true) break;
   }
-#undef LB
+#undef LP
 #undef L
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 
 int launch_stress_list(int mode, const WorkItem* wl, const ModelDev* md, int nm, long total, long grid, int rclass,
                        hipStream_t st) {
-  if (rclass < RHEO_VISCOUS || rclass > RHEO_EXT || nm < 1) return RELAX_ERR_ARG;
+  if (rclass < RHEO_VISCOUS || rclass > RHEO_ALL || nm < 1 || mode == STRESS_SET) return RELAX_ERR_ARG;
   if (total < 1) return RELAX_OK;
   const unsigned gx = (unsigned)(grid > 0 && grid < total ? grid : total);
-#define K(MODE, F) k_stress_list<MODE, F><<<gx, 256, 0, st>>>(md, wl, nm);
-#define KM(MODE)                                          \
-  {                                                       \
-    if (rclass == RHEO_EXT) K(MODE, RHEO_EXT)             \
-    else if (rclass == RHEO_CREEP) K(MODE, RHEO_CREEP)    \
-    else K(MODE, RHEO_VISCOUS)                            \
+#define K(MODE, E, PART) k_stress_list<MODE, E, PART><<<gx, 256, 0, st>>>(md, wl, nm);
+#define KP(MODE, E)                                            \
+  {                                                            \
+    if (!(rclass & RHEO_CREEP)) { K(MODE, E, PART_ALL) }       \
+    else {                                                     \
+      K(MODE, E, PART_OUT)                                     \
+      k_stress_band_list<MODE, E><<<(unsigned)((total + SEGS - 1) / SEGS), 256, 0, st>>>(md, wl, nm); \
+    }                                                          \
   }
-  if (mode == STRESS_SET) K(STRESS_SET, RHEO_VISCOUS)
-  else if (mode == STRESS_PRED) KM(STRESS_PRED)
+#define KM(MODE)                          \
+  {                                       \
+    if (rclass & RHEO_EXT) KP(MODE, true) \
+    else KP(MODE, false)                  \
+  }
+  if (mode == STRESS_PRED) KM(STRESS_PRED)
   else KM(STRESS_CORR)
 #undef K
+#undef KP
 #undef KM
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
