@@ -77,7 +77,7 @@ struct relax_model {
   relax_batch* batch = nullptr;  // the batch the model is a member of
   // launch-shape variants of the tunable kernels (relax_model_autotune):
   // y transform columns, Green column pass, divergence tiles
-  int tune_cols = 0, tune_green = 0, tune_body = 0;
+  int tune_cols = -1, tune_green = -1, tune_body = -1;  // -1: default_shapes
   // phase timers (relax_model_profile)
   bool prof_on = false;
   int prof_n = 0;

@@ -302,6 +302,39 @@ static void tune_lookup(relax_model_t* m) {
   m->tune_body = it->second.body;
 }
 
+// The launch shapes of a model that was not tuned, from its grid and rheology
+// class (microseconds per launch, measured on every class over grids of 32^3
+// to 1024x1024x64 and 512^3):
+//  - y transform: half the columns per workgroup, for more workgroups, up to
+//    512x512x128 (256^3: 32.8 against 36.3; 512x512x256: 170.8 against 167.3);
+//    128-row planes keep the default's 64 (their 16-point columns are short:
+//    128^3 7.4 against 8.0), 1024-row planes theirs (1024x1024x64: 179 against
+//    210).
+//  - Green column pass: the register form from 64-deep columns up (64x64x128:
+//    11.0 against 16.0, 256x256x128: 51.6 against 65.1, 512x512x256: 264
+//    against 419; it has no 256-deep form); 32-deep columns radix 8 (512x512x64:
+//    87.8 against 94.9, the register form 128).  The forms round differently,
+//    and the slip of a creeping patch near the clamp of its friction law
+//    follows that rounding (5e-5 of the slip after 20 steps at 256x256x128):
+//    models with creeping planes keep the radix-16 LDS form, in a batch too
+//    (green_launches).
+//  - divergence: the register-window tiles wherever 64 divides n1, 64x8 on
+//    grids under 128^3 (64x64x64: 7.6 against 9.1 for 64x16 and 31 for the
+//    32x8 ring), else 64x16 (512x512x256: 247 against 268, ring 303).  The
+//    extended rheology keeps 168-178 registers live there, two waves per SIMD:
+//    the 64x8 window up to 4 M points (128x128x256: 57 against 66), ring tiles
+//    above (512x512x256: 741 against 828).
+static void default_shapes(const Grid& g, int rclass, int* cols, int* green, int* body) {
+  const long n = 2 * g.H;
+  if (*cols < 0) *cols = g.n2 != 128 && g.n2 != 1024 && n <= (1L << 25) ? 1 : 0;
+  if (*green < 0) *green = g.h3 == 64 || g.h3 == 128 ? 3 : g.h3 == 32 ? 2 : 0;
+  if (*body < 0) {
+    if (g.n1 % 64) *body = 1;
+    else if (rclass & RHEO_EXT) *body = n <= (1L << 22) ? 4 : n <= (1L << 23) ? 2 : 3;
+    else *body = n < (1L << 21) ? 4 : 5;
+  }
+}
+
 static TimeLine timeline(const relax_model_t* m) {
   TimeLine tl;
   tl.interval = m->desc.interval; tl.odt = m->desc.odt; tl.tscale = m->desc.tscale; tl.skip = m->desc.skip;
@@ -1058,6 +1091,10 @@ struct Ctx {
   relax_model_t* const* models;   // host handles, for the per-plane kernels
   relax_model_t* prof;            // phase timers (single model), or nullptr
   int tune_cols, tune_green, tune_body;  // launch-shape variants
+  // the first ncreep models have creeping planes; without a tuned choice their
+  // Green column pass takes variant 0
+  int ncreep;
+  bool green_tuned;
 };
 
 static Ctx single(relax_model_t* m) {
@@ -1065,6 +1102,9 @@ static Ctx single(relax_model_t* m) {
   c.lead = m; c.md = m->md_dev; c.one = &m->md_host; c.nm = 1; c.rclass = rheo_class(m);
   c.st = m->stream; c.models = &m->self; c.prof = m;
   c.tune_cols = m->tune_cols; c.tune_green = m->tune_green; c.tune_body = m->tune_body;
+  c.ncreep = c.rclass & RHEO_CREEP ? 1 : 0;
+  c.green_tuned = c.tune_green >= 0;
+  default_shapes(m->g, c.rclass, &c.tune_cols, &c.tune_green, &c.tune_body);
   return c;
 }
 
@@ -1087,6 +1127,22 @@ static YRide ypass_ride(const Ctx& c, int sign) {
     r.rp1 = g.n2; r.rn1 = 3;
   }
   return r;
+}
+
+// The Green column pass of every model of the context (W transformed in x and
+// y, in the split order of l2 points).
+static int green_launches(const Ctx& c, int l2) {
+  const relax_model_t* m = c.lead;
+  auto part = [&](int off, int n, int variant) -> int {
+    const ModelDev* md = c.md + off;
+    if (n == 0) return RELAX_OK;
+    return launch_green_columns(m->gc, m->g.h3, MFIELD(float2, md, W), MFIELD(float2, md, NQ),
+                                MFIELD(const float2, md, T), MFIELD(const float2, md, TN), n, c.st, l2, variant);
+  };
+  const int nc = c.green_tuned ? 0 : c.ncreep;
+  int rc = part(0, nc, 0);
+  if (!rc) rc = part(nc, c.nm - nc, c.tune_green);
+  return rc;
 }
 
 // Green's function of the work field W (body force, upper half) with the
@@ -1122,9 +1178,7 @@ static int model_green(const Ctx& c, int epi) {
                              c.tune_cols)))
     return rc;
   cmark(c, RELAX_PROF_FFT_Y);
-  if ((rc = launch_green_columns(m->gc, h3, MFIELD(float2, md, W), MFIELD(float2, md, NQ), MFIELD(const float2, md, T),
-                                 MFIELD(const float2, md, TN), nm, st, l2, c.tune_green)))
-    return rc;
+  if ((rc = green_launches(c, l2))) return rc;
   cmark(c, RELAX_PROF_GREEN_Z);
   if ((rc = launch_fft_ypass(ly, n2, +1, MFIELD(float2, md, W), m1, (long)ly * m1, m1, nyp, ypass_ride(c, +1), nm, st,
                              c.tune_cols)))
@@ -1908,9 +1962,10 @@ struct relax_batch {
   int tune_grid[3] = {0, 0, 0};     // the grid it was made for
   // Members of several grid classes (grid, spacing, elastic constants): the
   // records in md_dev are grouped by class, member i's at rec[i]; `ordered`
-  // lists the members in record order.  One class: rec is the identity.
+  // lists the members in record order.
   struct ClassRange {
     int off, n;
+    relax_model_t* first;  // the member added first
   };
   std::vector<int> rec;
   std::vector<relax_model_t*> ordered;
@@ -2016,8 +2071,8 @@ int relax_batch_synchronize(relax_batch_t* b) {
   return RELAX_OK;
 }
 
-// Group the members by grid class (first-seen order of the classes, the
-// members' order within each): rec, ordered and classes.
+// Group the members by grid class (first-seen order of the classes; within
+// each those with creeping planes first, then the members' order): rec, ordered and classes.
 static void batch_classes(relax_batch_t* b) {
   const int nm = (int)b->models.size();
   std::vector<int> cls(nm, -1);
@@ -2031,9 +2086,15 @@ static void batch_classes(relax_batch_t* b) {
   b->ordered.clear();
   b->classes.clear();
   for (int k = 0; k < (int)leads.size(); ++k) {
-    relax_batch_t::ClassRange r{(int)b->ordered.size(), 0};
-    for (int i = 0; i < nm; ++i)
-      if (cls[i] == k) { b->rec[i] = (int)b->ordered.size(); b->ordered.push_back(b->models[i]); ++r.n; }
+    relax_batch_t::ClassRange r{(int)b->ordered.size(), 0, b->models[leads[k]]};
+    // members with creeping planes first (class_ctx counts them)
+    for (const bool creep : {true, false})
+      for (int i = 0; i < nm; ++i)
+        if (cls[i] == k && ((rheo_class(b->models[i]) & RHEO_CREEP) != 0) == creep) {
+          b->rec[i] = (int)b->ordered.size();
+          b->ordered.push_back(b->models[i]);
+          ++r.n;
+        }
     b->classes.push_back(r);
   }
 }
@@ -2055,10 +2116,12 @@ static int mixed_body_variant(const relax_batch_t* b, int rclass) {
   const relax_model_t* lead = nullptr;
   for (const auto& k : b->classes) {
     const long pts = (long)k.n * b->ordered[k.off]->g.H;
-    if (pts > best) { best = pts; lead = b->ordered[k.off]; }
+    if (pts > best) { best = pts; lead = k.first; }
   }
   TuneChoice t;
   int v = tune_entry(b->device, lead->g, rclass, &t) ? t.body : lead->tune_body;
+  int cols = 0, green = 0;
+  default_shapes(lead->g, rclass, &cols, &green, &v);
   for (const relax_model_t* m : b->models)
     if (!body_variant_fits(m->g, v)) return 1;
   return v;
@@ -2170,13 +2233,17 @@ static Ctx class_ctx(relax_batch_t* b, const relax_batch_t::ClassRange& k, int r
   c.prof = nullptr;
   c.rclass = rclass;
   const Grid& g = c.lead->g;
-  c.tune_cols = c.lead->tune_cols; c.tune_green = c.lead->tune_green; c.tune_body = c.lead->tune_body;
+  c.tune_cols = k.first->tune_cols; c.tune_green = k.first->tune_green; c.tune_body = k.first->tune_body;
   TuneChoice t;
   if (b->tuned && b->tune_grid[0] == g.n1 && b->tune_grid[1] == g.n2 && b->tune_grid[2] == g.n3) {
     c.tune_cols = b->tune[0]; c.tune_green = b->tune[1]; c.tune_body = b->tune[2];
   } else if (tune_entry(b->device, g, rclass, &t)) {
     c.tune_cols = t.cols; c.tune_green = t.green; c.tune_body = t.body;
   }
+  c.ncreep = 0;
+  while (c.ncreep < c.nm && (rheo_class(c.models[c.ncreep]) & RHEO_CREEP)) ++c.ncreep;
+  c.green_tuned = c.tune_green >= 0;
+  default_shapes(g, rclass, &c.tune_cols, &c.tune_green, &c.tune_body);
   return c;
 }
 

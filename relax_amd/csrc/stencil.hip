@@ -750,25 +750,28 @@ static int device_cus() {
   return n;
 }
 
-// Depth chunk of one divergence tile: each chunk re-reads the plane above
-// and below it.  The register-window forms (variants 4 and 5: one workgroup
-// of 64x16 tiles per CU, two of 64x8, at their register use) take the
-// deepest chunk that still gives every CU a workgroup, at least 2 planes (a
-// small grid's launch lasts as long as one workgroup's chain of planes:
-// 64x64x64 takes 7.6 us in chunks of 2, 9.9 of 4, 15.1 of 8; 128^3 14.1 us in
-// chunks of 4, 17.1 of 8): at 512x512x256 one chunk of all 128 planes (256 workgroups) runs the
-// divergence in 0.250 ms against 0.275 ms for chunks of 32 planes (1024
-// workgroups, four rounds) and 0.268 ms for 64.
+// Depth chunk of one divergence tile.  The register-window forms (variants 4
+// and 5) hold two workgroups of 64x8 tiles or one of 64x16 per CU; a launch
+// lasts as many rounds of the device's slots as its chunks need, each the
+// chunk's planes and the two beside it (no output, no halo: 3/4 of a plane
+// each).  The chunk of the shortest launch is taken, at least 2 planes:
+// 512x512x256 walks all 128 planes in one round (0.250 ms; chunks of 32 planes
+// 0.275, of 64 0.268), 64x64x64 takes 7.6 us in chunks of 2 (9.9 of 4, 15.1 of
+// 8), 11 models of 128^3 153 us in chunks of 16 (182 us in chunks of 32,
+// whose second round is a third full).
 int body_depth_chunk(const Grid& g, int variant, int nm) {
   if (variant < 4) return variant >= 3 ? 32 : 16;
   const long tiles = (long)(g.n1 / 64) * (g.n2 / (variant == 5 ? 16 : 8)) * (nm > 0 ? nm : 1);
   if (tiles <= 0) return 32;  // the tiles do not fit the grid: the launcher refuses it
-  const long want = (long)device_cus() * (variant == 5 ? 1 : 2);
-  long gz = (want + tiles - 1) / tiles;
-  const long gmax = (g.h3 + 1) / 2;
-  if (gz > gmax) gz = gmax;
-  if (gz < 1) gz = 1;
-  return (int)((g.h3 + gz - 1) / gz);
+  const long slots = (long)device_cus() * (variant == 5 ? 1 : 2);
+  long best = -1;
+  int zbest = g.h3;
+  for (int gz = 1; gz <= (g.h3 + 1) / 2; ++gz) {
+    const int zc = (g.h3 + gz - 1) / gz;
+    const long cost = (tiles * ((g.h3 + zc - 1) / zc) + slots - 1) / slots * (2 * zc + 3);
+    if (best < 0 || cost < best) { best = cost; zbest = zc; }
+  }
+  return zbest;
 }
 
 // One divergence kernel over one part of the models, chunks of zc planes, gz
