@@ -126,11 +126,11 @@ int relax_greenfunctioncowling(float* c1, float* c2, float* c3, float* t1, float
  * in the padded layout ((sx1+2)*sx2*sx3 and (sx1+2)*sx2 floats), transformed
  * in place as relax_greenfunctioncowling does; the work is enqueued on
  * `stream` (a hipStream_t, or NULL for the null stream) and the call returns
- * without waiting.  The three traction planes it needs live in a static
- * device array of 12.0 MiB (sx1, sx2 up to 1024; larger grids return
- * RELAX_ERR_SIZE), one per device, shared by every call on that device:
- * calls that overlap on one device race.  relax_hip_init sets it up for the
- * device it selects; otherwise the first call on a device does. */
+ * without waiting.  It needs no scratch memory, so calls on different
+ * streams may overlap.  sx1, sx2 and sx3 are powers of two from 16 to 1024
+ * (others return RELAX_ERR_SIZE).  The transforms' tables are static:
+ * relax_hip_init fills them for the device it selects; otherwise the first
+ * call on a device does. */
 int relax_greenfunctioncowling_noalloc(float* c1, float* c2, float* c3, float* t1, float* t2, float* t3, int sx1,
                                        int sx2, int sx3, double dx1, double dx2, double dx3, double lambda,
                                        double mu, double gamma, void* stream);

@@ -563,8 +563,7 @@ int relax_surfacetractioncowling(double lambda, double mu, double gamma, const f
   HIP_TRY(hipMemcpy(b.p, u2, bytes, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c.p, u3, bytes, hipMemcpyHostToDevice));
   const GreenConst gc = green_const(sx1, sx2, sx3, dx1, dx2, dx3, lambda, mu, gamma);
-  if ((rc = sync_status(launch_surface_padded(gc, a.c(), b.c(), c.c(), nullptr, nullptr, nullptr, q1.c(), q2.c(),
-                                              q3.c(), 0))))
+  if ((rc = sync_status(launch_surface_padded(gc, a.c(), b.c(), c.c(), q1.c(), q2.c(), q3.c(), 0))))
     return rc;
   HIP_TRY(hipMemcpy(p1, q1.p, pb, hipMemcpyDeviceToHost));
   HIP_TRY(hipMemcpy(p2, q2.p, pb, hipMemcpyDeviceToHost));
@@ -600,27 +599,45 @@ int relax_cerrutimodified(const float* p1, const float* p2, const float* p3, dou
 
 // greenfunctioncowling on device buffers in the padded layout: v, three
 // fields of (sx1+2) sx2 sx3 floats over the full depth; t, three planes of
-// (sx1+2) sx2; p, three planes of scratch.  Enqueued on stream st; with sync
-// the call waits for it and reports the kernels' status.
-int green_full_device(float* const v[3], float* const t[3], float* const p[3], int sx1, int sx2, int sx3,
-                      double dx1, double dx2, double dx3, double lambda, double mu, double gamma, hipStream_t st,
-                      bool sync) {
+// (sx1+2) sx2.  Enqueued on stream st; with sync the call waits for it and
+// reports the kernels' status.  Each field's x1 and x2 transforms follow each
+// other (the second finds part of the field in the on-package cache); the
+// traction planes go three to a launch.
+int green_full_device(float* const v[3], float* const t[3], int sx1, int sx2, int sx3, double dx1, double dx2,
+                      double dx3, double lambda, double mu, double gamma, hipStream_t st, bool sync) {
   int rc;
   const GreenConst gc = green_const(sx1, sx2, sx3, dx1, dx2, dx3, lambda, mu, gamma);
   float2* vc[3] = {(float2*)v[0], (float2*)v[1], (float2*)v[2]};
   float2* tc[3] = {(float2*)t[0], (float2*)t[1], (float2*)t[2]};
-  float2* pc[3] = {(float2*)p[0], (float2*)p[1], (float2*)p[2]};
+  const int M = sx1 / 2;
+  const long P = M + 1;  // complex row pitch
+  // half the columns per workgroup up to 256 rows (256x256x256: 606 against 649
+  // us for the solve, 512x512x256 alike)
+  const int cv = sx2 <= 256 ? 1 : 0;
+  const auto tm = mptr3(tc[0], tc[1], tc[2]), tn = mptr3(tc[0] + M, tc[1] + M, tc[2] + M);
   for (int k = 0; k < 3; ++k) {
-    if ((rc = fftn_padded(v[k], sx1, sx2, sx3, dx1, dx2, dx3, -1, st))) return rc;
-    if ((rc = fftn_padded(t[k], sx1, sx2, 1, dx1, dx2, dx3, -1, st))) return rc;
+    if ((rc = launch_fft_x_r2c(sx1, v[k], sx1 + 2, vc[k], P, vc[k] + M, P, (long)sx2 * sx3, (float)(dx1 * dx2 * dx3), st)) ||
+        (rc = launch_fft_cols(sx2, -1, mptr(vc[k]), P, (long)sx2 * P, M + 1, sx3, 1, st, cv)))
+      return rc;
   }
-  if ((rc = launch_elastic_padded(gc, vc[0], vc[1], vc[2], st))) return rc;
-  if ((rc = launch_surface_padded(gc, vc[0], vc[1], vc[2], tc[0], tc[1], tc[2], pc[0], pc[1], pc[2], st))) return rc;
-  if ((rc = launch_cerruti_padded(gc, pc[0], pc[1], pc[2], vc[0], vc[1], vc[2], st))) return rc;
+  if ((rc = launch_fft_x_r2c(sx1, mptr3<const float>(t[0], t[1], t[2]), sx1 + 2, tm, P, tn, P, sx2,
+                             (float)(dx1 * dx2), 3, st)) ||
+      (rc = launch_fft_cols(sx2, -1, tm, P, (long)sx2 * P, M + 1, 1, 3, st)))
+    return rc;
+  if ((rc = launch_green_full(gc, vc, tc, st))) return rc;
+  const double sc = 1.0 / (sx1 * dx1 * sx2 * dx2 * sx3 * dx3), sc2 = 1.0 / (sx1 * dx1 * sx2 * dx2);
   for (int k = 0; k < 3; ++k) {
-    if ((rc = fftn_padded(v[k], sx1, sx2, sx3, dx1, dx2, dx3, +1, st))) return rc;
-    if ((rc = fftn_padded(t[k], sx1, sx2, 1, dx1, dx2, dx3, +1, st))) return rc;
+    if ((rc = launch_fft_cols(sx2, +1, mptr(vc[k]), P, (long)sx2 * P, M + 1, sx3, 1, st, cv)) ||
+        (rc = launch_fft_x_c2r(sx1, EPI_PLAIN, vc[k], P, vc[k] + M, P, v[k], sx1 + 2, (long)sx2 * sx3, (float)sc, nullptr,
+                               0, nullptr, st)))
+      return rc;
   }
+  if ((rc = launch_fft_cols(sx2, +1, tm, P, (long)sx2 * P, M + 1, 1, 3, st)) ||
+      (rc = launch_fft_x_c2r(sx1, EPI_PLAIN, mptr3<const float2>(tc[0], tc[1], tc[2]), P,
+                             mptr3<const float2>(tc[0] + M, tc[1] + M, tc[2] + M), P, mptr3(t[0], t[1], t[2]), sx1 + 2,
+                             sx2, (float)sc2, mptr3<const float>(nullptr, nullptr, nullptr), 0,
+                             mptr<const StepScalars>(nullptr), 3, st)))
+    return rc;
   if (!sync) return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
   HIP_TRY(hipStreamSynchronize(st));
   return sync_status(RELAX_OK);
@@ -635,9 +652,9 @@ int relax_greenfunctioncowling(float* c1, float* c2, float* c3, float* t1, float
   if ((rc = has_device())) return rc;
   const long rows = (long)sx2 * sx3;
   const size_t vb = (size_t)(sx1 + 2) * rows * 4, pb = (size_t)(sx1 + 2) * sx2 * 4;
-  Buf v[3], t[3], p[3];
+  Buf v[3], t[3];
   for (int k = 0; k < 3; ++k)
-    if ((rc = v[k].alloc(vb)) || (rc = t[k].alloc(pb)) || (rc = p[k].alloc(pb))) return rc;
+    if ((rc = v[k].alloc(vb)) || (rc = t[k].alloc(pb))) return rc;
   float* hc[3] = {c1, c2, c3};
   float* ht[3] = {t1, t2, t3};
   for (int k = 0; k < 3; ++k) {
@@ -646,8 +663,7 @@ int relax_greenfunctioncowling(float* c1, float* c2, float* c3, float* t1, float
   }
   float* vd[3] = {v[0].f(), v[1].f(), v[2].f()};
   float* td[3] = {t[0].f(), t[1].f(), t[2].f()};
-  float* pd[3] = {p[0].f(), p[1].f(), p[2].f()};
-  if ((rc = green_full_device(vd, td, pd, sx1, sx2, sx3, dx1, dx2, dx3, lambda, mu, gamma, 0, true))) return rc;
+  if ((rc = green_full_device(vd, td, sx1, sx2, sx3, dx1, dx2, dx3, lambda, mu, gamma, 0, true))) return rc;
   for (int k = 0; k < 3; ++k) {
     if ((rc = get_real(hc[k], v[k].f(), sx1, rows, align_data))) return rc;
     if ((rc = get_real(ht[k], t[k].f(), sx1, sx2, align_data))) return rc;
@@ -656,57 +672,21 @@ int relax_greenfunctioncowling(float* c1, float* c2, float* c3, float* t1, float
 }
 
 // ------------------------------------------ greenfunctioncowling, no allocation --
-// The three traction planes of the surface correction, for grids of up to
-// 1024 x 1024 horizontally, in a static device array: every device the
-// library runs on holds one (12.0 MiB) until the process ends, and every
-// call on a device shares it.  Host code uses the address that
-// hipGetSymbolAddress returns for the current device, never the array's
-// name.
-static const long NOALLOC_MAX_N = 1024;
-static const long NOALLOC_PLANE = (NOALLOC_MAX_N + 2) * NOALLOC_MAX_N;  // floats per plane
-static __device__ __align__(256) float scratch[3 * NOALLOC_PLANE];
-static std::mutex g_scratch_mu;
-static std::map<int, float*> g_scratch;  // device -> address of its scratch
-
-// The current device's scratch address, looked up once per device.
-static int scratch_address(float** out) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return RELAX_ERR_HIP;
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  auto it = g_scratch.find(dev);
-  if (it == g_scratch.end()) {
-    float* p = nullptr;
-    if (hipGetSymbolAddress((void**)&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) return RELAX_ERR_HIP;
-    it = g_scratch.emplace(dev, p).first;
-  }
-  *out = it->second;
-  return RELAX_OK;
-}
-
-// Per-device set-up of the allocation-free entry: the scratch address and
-// the twiddle tables of every transform length (relax_hip_init calls it).
-int noalloc_setup() {
-  float* p = nullptr;
-  if (int rc = scratch_address(&p)) return rc;
-  return twiddle_table(2) ? RELAX_OK : RELAX_ERR_HIP;
-}
+// Per-device set-up of the allocation-free entry: the twiddle tables of every
+// transform length (relax_hip_init calls it).
+int noalloc_setup() { return twiddle_table(2) ? RELAX_OK : RELAX_ERR_HIP; }
 
 int relax_greenfunctioncowling_noalloc(float* c1, float* c2, float* c3, float* t1, float* t2, float* t3, int sx1,
                                        int sx2, int sx3, double dx1, double dx2, double dx3, double lambda,
                                        double mu, double gamma, void* stream) {
   if (!c1 || !c2 || !c3 || !t1 || !t2 || !t3) return RELAX_ERR_ARG;
-  if (!pow2_in(sx1, 16, NOALLOC_MAX_N) || !pow2_in(sx2, 16, NOALLOC_MAX_N) || !pow2_in(sx3, 16, 1024))
-    return RELAX_ERR_SIZE;
-  if ((long)(sx1 + 2) * sx2 > NOALLOC_PLANE) return RELAX_ERR_SIZE;
+  if (!pow2_in(sx1, 16, 1024) || !pow2_in(sx2, 16, 1024) || !pow2_in(sx3, 16, 1024)) return RELAX_ERR_SIZE;
   int rc;
   if ((rc = has_device())) return rc;
-  float* base = nullptr;
-  if ((rc = noalloc_setup()) || (rc = scratch_address(&base))) return rc;
-  const long plane = (long)(sx1 + 2) * sx2;
+  if ((rc = noalloc_setup())) return rc;
   float* v[3] = {c1, c2, c3};
   float* t[3] = {t1, t2, t3};
-  float* pp[3] = {base, base + plane, base + 2 * plane};
-  return green_full_device(v, t, pp, sx1, sx2, sx3, dx1, dx2, dx3, lambda, mu, gamma, (hipStream_t)stream, false);
+  return green_full_device(v, t, sx1, sx2, sx3, dx1, dx2, dx3, lambda, mu, gamma, (hipStream_t)stream, false);
 }
 
 // ========================================================= elastic3d.f90 ==

@@ -325,22 +325,28 @@ __global__ __launch_bounds__(NT) void k_green_columns(ColumnConsts C, double mu,
 //    linear in u, so each thread sums k3 u1, k3 u2, k3 u3, u3 and
 //    k1 u1 + k2 u2 over its frequencies (12 operations per frequency) and
 //    the column's traction is formed from the five sums once.
-template <int H3>
+//
+// FULL: the full depth of 2 H3 points on padded spectra (the FullGreen
+// argument) instead of the pruned half: the halves' inputs are x[z] + x[z+H3]
+// and (x[z] - x[z+H3]) w_n3^z, the outputs E' + w^-z O' and E' - w^-z O'.  The
+// last tile of a k2 row has one column (n1/2 + 1 of them): the others read
+// that column again and store nothing.
+struct FullGreen {
+  float2* v[3];
+  const float2* t[3];
+};
+template <int H3, bool FULL>
 __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu, double alpha, double gamma, int n1,
                                                    int n2, int n3, MPtr<float2> W_m, MPtr<float2> NQ_m,
                                                    MPtr<const float2> TM_m, MPtr<const float2> TN_m,
-                                                   const float2* __restrict__ tw3, int l2) {
+                                                   const float2* __restrict__ tw3, int l2, FullGreen F) {
   constexpr int TX = 16, NT = 512, Q = H3 / 16;
-  static_assert(Q == 2 || Q == 4 || Q == 8, "H3 = 32, 64 or 128");
+  static_assert(Q == 4 || Q == 8 || (Q == 2 && !FULL), "H3 = 32 (pruned only), 64 or 128");
   constexpr int NA = 3 * Q * TX;  // step-A threads
   constexpr int NB = 16 * TX;     // step-B threads per half
   constexpr int RS = 16 * TX + 16;  // float2 per (c, j) group (padded: j groups on alternate banks)
   constexpr int NW = NT / 64;
   constexpr unsigned RSRC3 = 0x00020000u;  // raw buffer, 32-bit data format
-  float2* W = W_m.at(blockIdx.y);
-  float2* NQ = NQ_m.at(blockIdx.y);
-  const float2* __restrict__ TM = TM_m.at(blockIdx.y);
-  const float2* __restrict__ TN = TN_m.at(blockIdx.y);
   __shared__ float2 buf[3 * Q * RS];
   __shared__ float2 stw[2 * H3];
   __shared__ float2 tws[16 * 16];  // w_H3^(a b), row a
@@ -356,9 +362,32 @@ __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu,
   const int acol = tid % TX, aj = (tid / TX) % Q, ac = tid / (TX * Q);  // step A
   const int bcol = tid % TX, bk1 = (tid / TX) % 16, half = tid / NB;    // step B
   const bool isA = tid < NA;
-  const GreenTileAddr A = green_tile<TX>(xcd_tile(blockIdx.x, gridDim.x), bcol, n1, n2, H3, l2, W, NQ, TM, TN);
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(A.base, (short)0, 0x7fffffff, RSRC3);
-  const unsigned voff = (unsigned)((ac * A.cs + aj * A.zs + acol) * (long)sizeof(float2));
+  GreenTileAddr A;
+  float2* vbase;
+  unsigned voff;
+  bool vstore = true;
+  int tcol = TX;  // columns of the tile
+  long frow = 0;
+  if constexpr (FULL) {
+    const int h1 = n1 / 2 + 1, nch = (h1 + TX - 1) / TX, tile = xcd_tile(blockIdx.x, gridDim.x);
+    A.k2i = tile / nch;
+    const int k10 = (tile % nch) * TX;
+    A.k1i = k10 + bcol;
+    A.zs = (long)h1 * n2;
+    frow = (long)A.k2i * h1 + k10;
+    tcol = min(TX, h1 - k10);
+    vstore = acol < tcol;
+    // a component's TX Q threads are whole waves (Q >= 4)
+    const int cu = __builtin_amdgcn_readfirstlane(ac);
+    vbase = (cu == 0 ? F.v[0] : cu == 1 ? F.v[1] : F.v[2]) + frow;
+    voff = (unsigned)((aj * A.zs + min(acol, tcol - 1)) * (long)sizeof(float2));
+  } else {
+    A = green_tile<TX>(xcd_tile(blockIdx.x, gridDim.x), bcol, n1, n2, H3, l2, W_m.at(blockIdx.y), NQ_m.at(blockIdx.y),
+                       TM_m.at(blockIdx.y), TN_m.at(blockIdx.y));
+    vbase = A.base;
+    voff = (unsigned)((ac * A.cs + aj * A.zs + acol) * (long)sizeof(float2));
+  }
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(vbase, (short)0, 0x7fffffff, RSRC3);
   const unsigned zstep = (unsigned)(Q * A.zs * (long)sizeof(float2));  // uniform: the scalar offset
 
   // step A of one half: DFT16, twiddle, into the buffer.  The odd half
@@ -371,6 +400,16 @@ __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu,
     for (int m = 0; m < 16; ++m)
       x[m] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, m * zstep, 0));
   };
+  // FULL: the other half of the depth joins at step A
+  const unsigned zhalf = (unsigned)(H3 * A.zs * (long)sizeof(float2));
+  auto join = [&](bool odd) {
+    float2 b[16];
+#pragma unroll
+    for (int m = 0; m < 16; ++m)
+      b[m] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, zhalf + m * zstep, 0));
+#pragma unroll
+    for (int m = 0; m < 16; ++m) x[m] = odd ? csub(x[m], b[m]) : cadd(x[m], b[m]);
+  };
   if (isA) load();
   for (int e = tid; e < 2 * H3; e += NT) stw[e] = tw3[e];
   if (tid < 256) tws[tid] = tw3[2 * (((tid >> 4) * (tid & 15)) % H3)];
@@ -379,6 +418,7 @@ __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu,
   auto stepA = [&](bool odd) {
     if (!isA) return;
     float2* y = x;
+    if (FULL) join(odd);
     if (odd) {
 #pragma unroll
       for (int m = 0; m < 16; ++m) y[m] = cmul(x[m], stw[Q * m + aj]);
@@ -481,7 +521,10 @@ __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu,
       const float2 d = make_float2(C.mod2pi * S[2].x + C.lam2pi * S[4].x, C.mod2pi * S[2].y + C.lam2pi * S[4].y);
       acc = make_float2(-d.y - C.grav * S[3].x, d.x - C.grav * S[3].y);
     }
-    const float2 tt = gload(A.tbase + c * A.tcs + t);
+    float2 tt;
+    if constexpr (FULL)
+      tt = t < tcol ? gload((c == 0 ? F.t[0] : c == 1 ? F.t[1] : F.t[2]) + frow + t) : make_float2(0.f, 0.f);
+    else tt = gload(A.tbase + c * A.tcs + t);
     // p = t - p / (sx3 dx3)   (green.f90:373-375, :1082-1084)
     pv[c][t] = make_float2(tt.x - acc.x / C.inv_n3dx3, tt.y - acc.y / C.inv_n3dx3);
   }
@@ -528,8 +571,11 @@ __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu,
     typedef unsigned u2v __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int m = 0; m < 16; ++m) {
-      const float2 v = cadd(x[m], cmul(o[m], cconj(stw[Q * m + aj])));
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, v), rs, voff, m * zstep, 0);
+      const float2 ow = cmul(o[m], cconj(stw[Q * m + aj]));
+      const float2 v = cadd(x[m], ow);
+      if (vstore) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, v), rs, voff, m * zstep, 0);
+      if (FULL && vstore)
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, csub(x[m], ow)), rs, voff, zhalf + m * zstep, 0);
     }
   }
 }
@@ -542,8 +588,8 @@ static int green_reg_launch(const GreenConst& gc, const ColumnConsts& C, double 
   const int m1 = gc.n1 / 2;
   if (HH < 32 || HH > 128 || m1 % TX || gc.n2 % TX) return RELAX_ERR_SIZE;
   const int nb = (m1 / TX) * gc.n2 + gc.n2 / TX;
-  k_green_reg<(HH < 32 ? 32 : HH > 128 ? 128 : HH)><<<dim3(nb, nm), 512, 0, st>>>(
-      C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, gc.n3, W, NQ, TM, TN, tw3, l2);
+  k_green_reg<(HH < 32 ? 32 : HH > 128 ? 128 : HH), false><<<dim3(nb, nm), 512, 0, st>>>(
+      C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, gc.n3, W, NQ, TM, TN, tw3, l2, FullGreen{});
   return RELAX_OK;
 }
 
@@ -597,6 +643,131 @@ int launch_green_columns(const GreenConst& gc, int h3, MPtr<float2> W, MPtr<floa
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 
+// ------------------------------------------- full-depth column pass --------
+// greenfunctioncowling between the x2 transforms, over the full depth, on
+// padded spectra: TX of the n1/2+1 columns of a k2 row of all three components
+// in LDS (48 KB at 512 and 1024 depths), transformed along x3, multiplied by
+// the Green's function, corrected and transformed back.  In place of five
+// passes over the fields (x3 transform, elastic response, traction sum, Cerruti
+// correction, x3 transform back) one that reads and writes them once: the
+// solve takes 369 us instead of 691 at 128x128x512, 777 instead of 1366 at
+// 128x128x1024.  Bound by its vector instructions and the LDS passes of the
+// transforms.  128 and 256 depths take the register form (k_green_reg, FULL):
+// 590 us at 512x512x256 against 888 us for this one in 8-column tiles (the
+// five passes took 1790).
+template <int N3>
+struct FullTile {
+  static constexpr int TX = N3 <= 64 ? 16 : 2048 / N3;
+  static constexpr int NT = N3 >= 512 ? 384 : 192;
+};
+template <int N3>
+__global__ __launch_bounds__(FullTile<N3>::NT) void k_green_full(ColumnConsts C, double mu, double alpha, double gamma,
+                                                                 int n1, int n2, float2* v1, float2* v2, float2* v3,
+                                                                 const float2* t1, const float2* t2, const float2* t3,
+                                                                 const float2* __restrict__ tw3) {
+  constexpr int TX = FullTile<N3>::TX, NT = FullTile<N3>::NT, NW = NT / 64;
+  static_assert(64 % TX == 0, "a thread keeps one column");
+  constexpr int SB = N3 * TX + 12;  // padded as in k_green_columns
+  __shared__ float2 s[3 * SB];
+  __shared__ float2 red[3][NW][TX];
+  __shared__ float2 pv[3][TX];
+  __shared__ float2 stw[N3];
+  const int tid = threadIdx.x, tx = tid % TX;
+  const int h1 = n1 / 2 + 1, nch = (h1 + TX - 1) / TX;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int k2i = tile / nch, k10 = (tile % nch) * TX;
+  const long row = (long)k2i * h1 + k10, zs = (long)h1 * n2;
+  float2* const v[3] = {v1, v2, v3};
+  const float2* const t[3] = {t1, t2, t3};
+  const bool own = k10 + tx < h1;
+  for (int e = tid; e < N3; e += NT) stw[e] = tw3[e];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    for (int z = tid / TX; z < N3; z += NT / TX)
+      s[c * SB + z * TX + tx] = own ? gload(v[c] + row + z * zs + tx) : make_float2(0.f, 0.f);
+  __syncthreads();
+  lds_fft<N3, 3 * TX, NT, TX, 1, SB, TX, -1, 1, true, 16>(s, stw, tid);
+
+  const float k1 = (float)(k10 + tx) * C.ik1, k2 = wavenumber23f(k2i, n2, C.ik2);
+  float2 ps1 = make_float2(0.f, 0.f), ps2 = ps1, ps3 = ps1;
+  for (int m = tid / TX; m < N3; m += NT / TX) {
+    const float k3 = wavenumber23f(m, N3, C.ik3);
+    float2& c1 = s[m * TX + tx];
+    float2& c2 = s[SB + m * TX + tx];
+    float2& c3 = s[2 * SB + m * TX + tx];
+    float2 a1 = c1, a2 = c2, a3 = c3;
+    if (k10 + tx == 0 && k2i == 0 && m == 0) a1 = a2 = a3 = make_float2(0.f, 0.f);
+    else elastic_point(C, k1, k2, k3, a1, a2, a3);
+    c1 = a1; c2 = a2; c3 = a3;
+    float2 s1, s2, s3;
+    traction_point(C, k1, k2, k3, a1, a2, a3, s1, s2, s3);
+    ps1 = cadd(ps1, s1); ps2 = cadd(ps2, s2); ps3 = cadd(ps3, s3);
+  }
+  // the sums over k3 in a fixed order: lanes of a column, then the waves
+#pragma unroll
+  for (int off = 32; off >= TX; off >>= 1) {
+    ps1.x += __shfl_xor(ps1.x, off); ps1.y += __shfl_xor(ps1.y, off);
+    ps2.x += __shfl_xor(ps2.x, off); ps2.y += __shfl_xor(ps2.y, off);
+    ps3.x += __shfl_xor(ps3.x, off); ps3.y += __shfl_xor(ps3.y, off);
+  }
+  if ((tid & 63) < TX) {
+    red[0][tid >> 6][tx] = ps1; red[1][tid >> 6][tx] = ps2; red[2][tid >> 6][tx] = ps3;
+  }
+  __syncthreads();
+  if (tid < 3 * TX) {
+    const int c = tid / TX, x = tid % TX;
+    float2 acc = red[c][0][x];
+    for (int w = 1; w < NW; ++w) acc = cadd(acc, red[c][w][x]);
+    const float2* tc = c == 0 ? t[0] : c == 1 ? t[1] : t[2];
+    const float2 tt = k10 + x < h1 ? gload(tc + row + x) : make_float2(0.f, 0.f);
+    // p = t - p / (sx3 dx3)   (green.f90:373-375, :1082-1084)
+    pv[c][x] = make_float2(tt.x - acc.x / C.inv_n3dx3, tt.y - acc.y / C.inv_n3dx3);
+  }
+  __syncthreads();
+  {
+    const float2 p1 = pv[0][tx], p2 = pv[1][tx], p3 = pv[2][tx];
+    const CerrutiCol cc = cerruti_column(C, mu, alpha, gamma, k1, k2, p1, p2, p3);
+    for (int m = tid / TX; m < N3; m += NT / TX)
+      cerruti_point(C, cc, p1, p2, wavenumber23f(m, N3, C.ik3), s[m * TX + tx], s[SB + m * TX + tx],
+                    s[2 * SB + m * TX + tx]);
+  }
+  __syncthreads();
+  lds_fft<N3, 3 * TX, NT, TX, 1, SB, TX, +1, 1, true, 16>(s, stw, tid);
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    for (int z = tid / TX; z < N3; z += NT / TX)
+      if (own) gstore(v[c] + row + z * zs + tx, s[c * SB + z * TX + tx]);
+}
+
+int launch_green_full(const GreenConst& gc, float2* const v[3], const float2* const t[3], hipStream_t st) {
+  const float2* tw3 = twiddle_table(gc.n3);
+  if (!tw3) return RELAX_ERR_NOMEM;
+  const ColumnConsts C = make_consts(gc);
+  const double alpha = (gc.lambda + gc.mu) / (gc.lambda + 2.0 * gc.mu);
+  const int h1 = gc.n1 / 2 + 1;
+#define X(N)                                                                                                  \
+  case N: {                                                                                                   \
+    const unsigned nb = (unsigned)((h1 + FullTile<N>::TX - 1) / FullTile<N>::TX) * (unsigned)gc.n2;           \
+    k_green_full<N><<<nb, FullTile<N>::NT, 0, st>>>(C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, v[0], v[1], v[2], \
+                                                   t[0], t[1], t[2], tw3);                                    \
+    break;                                                                                                    \
+  }
+#define R(N)                                                                                                  \
+  case N: {                                                                                                   \
+    const unsigned nb = (unsigned)((h1 + 15) / 16) * (unsigned)gc.n2;                                         \
+    k_green_reg<N / 2, true><<<nb, 512, 0, st>>>(C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, gc.n3, {}, {}, {}, {}, \
+                                                tw3, 0, FullGreen{{v[0], v[1], v[2]}, {t[0], t[1], t[2]}});   \
+    break;                                                                                                    \
+  }
+  switch (gc.n3) {
+    X(16) X(32) X(64) R(128) R(256) X(512) X(1024)
+    default: return RELAX_ERR_SIZE;
+  }
+#undef R
+#undef X
+  return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
+}
+
 // --------------------------------------- per-routine padded-spectrum kernels --
 // Spectra are (sx1/2+1) complex per row, rows (k2) then planes (k3).
 __global__ void k_elastic_padded(ColumnConsts C, int n1, int n2, int n3, float2* f1, float2* f2, float2* f3) {
@@ -616,8 +787,7 @@ __global__ void k_elastic_padded(ColumnConsts C, int n1, int n2, int n3, float2*
 
 // one thread per (k1,k2) column, k3 summed in the reference's order
 __global__ void k_surface_padded(ColumnConsts C, int n1, int n2, int n3, const float2* u1, const float2* u2,
-                                 const float2* u3, const float2* t1, const float2* t2, const float2* t3,
-                                 float2* p1, float2* p2, float2* p3) {
+                                 const float2* u3, float2* p1, float2* p2, float2* p3) {
   const int h1 = n1 / 2 + 1;
   const long o = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (o >= (long)h1 * n2) return;
@@ -633,9 +803,6 @@ __global__ void k_surface_padded(ColumnConsts C, int n1, int n2, int n3, const f
   a1 = make_float2(a1.x / C.inv_n3dx3, a1.y / C.inv_n3dx3);
   a2 = make_float2(a2.x / C.inv_n3dx3, a2.y / C.inv_n3dx3);
   a3 = make_float2(a3.x / C.inv_n3dx3, a3.y / C.inv_n3dx3);
-  if (t1) {  // greenfunctioncowling: p = t - p
-    a1 = csub(t1[o], a1); a2 = csub(t2[o], a2); a3 = csub(t3[o], a3);
-  }
   p1[o] = a1; p2[o] = a2; p3[o] = a3;
 }
 
@@ -667,13 +834,11 @@ int launch_elastic_padded(const GreenConst& gc, float2* f1, float2* f2, float2* 
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 
-int launch_surface_padded(const GreenConst& gc, const float2* u1, const float2* u2, const float2* u3,
-                          const float2* t1, const float2* t2, const float2* t3, float2* p1, float2* p2,
-                          float2* p3, hipStream_t st) {
+int launch_surface_padded(const GreenConst& gc, const float2* u1, const float2* u2, const float2* u3, float2* p1,
+                          float2* p2, float2* p3, hipStream_t st) {
   const ColumnConsts C = make_consts(gc);
   const long n = (long)(gc.n1 / 2 + 1) * gc.n2;
-  k_surface_padded<<<(unsigned)((n + 127) / 128), 128, 0, st>>>(C, gc.n1, gc.n2, gc.n3, u1, u2, u3, t1, t2, t3, p1,
-                                                                 p2, p3);
+  k_surface_padded<<<(unsigned)((n + 127) / 128), 128, 0, st>>>(C, gc.n1, gc.n2, gc.n3, u1, u2, u3, p1, p2, p3);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 

@@ -87,11 +87,13 @@ struct GreenConst {
 // holds y frequency 8*k1 + k2); the traction planes TM are in natural order
 int launch_green_columns(const GreenConst& gc, int h3, MPtr<float2> W, MPtr<float2> NQ, MPtr<const float2> TM,
                          MPtr<const float2> TN, int nm, hipStream_t st, int l2 = 0, int variant = 0);
+// the same over the full depth, on padded spectra (rows of n1/2+1 complex): v
+// transformed along x1 and x2, t the spectra of the traction planes
+int launch_green_full(const GreenConst& gc, float2* const v[3], const float2* const t[3], hipStream_t st);
 // per-routine kernels on padded full spectra (row pitch n1/2+1 complex)
 int launch_elastic_padded(const GreenConst& gc, float2* f1, float2* f2, float2* f3, hipStream_t st);
-int launch_surface_padded(const GreenConst& gc, const float2* u1, const float2* u2, const float2* u3,
-                          const float2* t1, const float2* t2, const float2* t3, float2* p1, float2* p2,
-                          float2* p3, hipStream_t st);
+int launch_surface_padded(const GreenConst& gc, const float2* u1, const float2* u2, const float2* u3, float2* p1,
+                          float2* p2, float2* p3, hipStream_t st);
 int launch_cerruti_padded(const GreenConst& gc, const float2* p1, const float2* p2, const float2* p3,
                           float2* u1, float2* u2, float2* u3, hipStream_t st);
 
@@ -109,11 +111,10 @@ int launch_traction(const relax_source_t* l, int nl, int n1, int n2, double dx1,
                     int rate, float* t3, long ld, hipStream_t st);
 
 // compat.hip: greenfunctioncowling over the full depth on device buffers in
-// the padded layout (v: fields of (sx1+2) sx2 sx3, t and p: planes of
+// the padded layout (v: fields of (sx1+2) sx2 sx3, t: planes of
 // (sx1+2) sx2), enqueued on stream st (and waited for with sync)
-int green_full_device(float* const v[3], float* const t[3], float* const p[3], int sx1, int sx2, int sx3,
-                      double dx1, double dx2, double dx3, double lambda, double mu, double gamma, hipStream_t st,
-                      bool sync);
+int green_full_device(float* const v[3], float* const t[3], int sx1, int sx2, int sx3, double dx1, double dx2,
+                      double dx3, double lambda, double mu, double gamma, hipStream_t st, bool sync);
 
 // model.hip: tensilesource (elastic3d.f90:2315-2411) and mogisource
 // (:2458-2509) of np cracks / point sources into f (3 fields of n1 n2 n3

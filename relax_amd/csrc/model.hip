@@ -1820,11 +1820,10 @@ int relax_model_event(relax_model_t* m, const relax_event_t* ev, double nyquist)
     // in the padded layout
     const long ld = g.n1 + 2, vs = ld * g.n2 * g.n3, ts = ld * g.n2;
     float* scratch = nullptr;
-    const size_t bytes = (size_t)(3 * vs + 6 * ts) * 4;
+    const size_t bytes = (size_t)(3 * vs + 3 * ts) * 4;
     HIP_TRY(rx_malloc(&scratch, bytes));
     float* v[3] = {scratch, scratch + vs, scratch + 2 * vs};
     float* tr[3] = {scratch + 3 * vs, scratch + 3 * vs + ts, scratch + 3 * vs + 2 * ts};
-    float* pp[3] = {scratch + 3 * vs + 3 * ts, scratch + 3 * vs + 4 * ts, scratch + 3 * vs + 5 * ts};
     rc = hipMemsetAsync(scratch, 0, bytes, m->stream) == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
     if (!rc && nbig)
       rc = launch_source(m->shear_dev, m->shear_slip, nbig, mu, g.n1, g.n2, g.h3, dx1, dx2, dx3, v[0], ld, vs, tr[0],
@@ -1839,7 +1838,7 @@ int relax_model_event(relax_model_t* m, const relax_event_t* ev, double nyquist)
     if (!rc && nl)
       rc = launch_traction(m->loads_dev, nl, g.n1, g.n2, dx1, dx2, t, 0.0, 0, tr[2], ld, m->stream);
     if (!rc && hipStreamSynchronize(m->stream) != hipSuccess) rc = RELAX_ERR_HIP;
-    if (!rc) rc = green_full_device(v, tr, pp, g.n1, g.n2, g.n3, dx1, dx2, dx3, lam, mu, m->desc.gamma, m->stream, true);
+    if (!rc) rc = green_full_device(v, tr, g.n1, g.n2, g.n3, dx1, dx2, dx3, lam, mu, m->desc.gamma, m->stream, true);
     if (!rc) {
       k_add_padded_top<<<blocks_of(H), 256, 0, m->stream>>>(m->u, scratch, g.n1, g.n2, g.h3, H, vs);
       if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess) rc = RELAX_ERR_HIP;

@@ -40,15 +40,17 @@ struct ModelDev {
   RheoParams R;
 };
 
-// One pointer argument of a launch: the pointer itself (one buffer), or the
-// field of every record of a ModelDev array (entry m for model m).
+// One pointer argument of a launch: the pointer itself (one buffer, or one of
+// three), or the field of every record of a ModelDev array (entry m for model m).
 template <class T>
 struct MPtr {
   T* p = nullptr;
+  T* p1 = nullptr;
+  T* p2 = nullptr;
   const char* rec = nullptr;  // address of the field in record 0
   int stride = 0;             // sizeof(ModelDev)
   __device__ __forceinline__ T* at(int m) const {
-    return rec ? *reinterpret_cast<T* const*>(rec + (long)m * stride) : p;
+    return rec ? *reinterpret_cast<T* const*>(rec + (long)m * stride) : m == 0 ? p : m == 1 ? p1 : p2;
   }
 };
 
@@ -71,6 +73,15 @@ template <class T>
 inline MPtr<T> mptr(T* p) {
   MPtr<T> r;
   r.p = p;
+  return r;
+}
+
+template <class T>
+inline MPtr<T> mptr3(T* p, T* p1, T* p2) {
+  MPtr<T> r;
+  r.p = p;
+  r.p1 = p1;
+  r.p2 = p2;
   return r;
 }
 
