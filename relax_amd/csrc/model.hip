@@ -1348,18 +1348,121 @@ int relax_model_run(relax_model_t* m, int nsteps, const double* dt_override, rel
 }
 
 // --------------------------------------------------- coseismic set-up ----
+// The source kernels add a list of sources, each of which reaches a small part
+// of the grid, point by point in the list's order.  A workgroup takes
+// SRC_POINTS points in address order (whole rows), gathers, still in order,
+// the sources whose gates along x2 and x3 the rows can pass, and visits the
+// samples along x1 that these reach, packed onto its threads; most workgroups
+// gather none and leave.  The FP64 tapers and Gaussians of the points visited
+// bound it, and the launches: 40 patches at 512x512x256 took 673 us (k_source)
+// and 669 us (k_add_shear) with every point testing every source, 51 and 39 us
+// so, with 1024 points to a workgroup 87 and 67, with 8192 62 and 45.  A crack
+// and two point sources over 256x256x256: 139 and 133 us before, 29 and 23 now.
+constexpr int SRC_POINTS = 2048, SRC_LIST = 1024;
+
+struct SrcShared {
+  unsigned short list[SRC_LIST];
+  int cnt[4], lo, hi;
+};
+// where a source's gates lie: |x - cx| <= r, and whether the rows reach it
+struct SrcHit {
+  bool hit;
+  double cx, r;
+};
+// ranges of the shifted coordinates of points [o0, o0 + SRC_POINTS) of an
+// n1 x n2 x n3 grid along x2 and x3; full: x3 shifted as well (n3 planes)
+struct SrcBox {
+  double ya, yb, za, zb;
+  bool top;  // has points of plane 0
+};
+__device__ __forceinline__ SrcBox src_box(long r0, long r1, int n2, int n3, double dx2, double dx3, bool full) {
+  const int p0 = (int)(r0 / n2), p1 = (int)(r1 / n2);
+  int i0 = (int)(r0 % n2), i1 = (int)(r1 % n2);
+  if (p0 != p1) { i0 = 0; i1 = n2 - 1; }
+  SrcBox b;
+  b.top = p0 == 0;
+  // samples from n/2 on are the negative coordinates: a range across is all.
+  // A quarter sample more on either side: the points' gates may round apart.
+  const bool wy = i0 < n2 / 2 && i1 >= n2 / 2, wz = full && p0 < n3 / 2 && p1 >= n3 / 2;
+  b.ya = wy ? -1e300 : d_shifted(i0, n2, dx2) - 0.25 * dx2;
+  b.yb = wy ? 1e300 : d_shifted(i1, n2, dx2) + 0.25 * dx2;
+  b.za = wz ? -1e300 : (full ? d_shifted(p0, n3, dx3) : (double)p0 * dx3) - 0.25 * dx3;
+  b.zb = wz ? 1e300 : (full ? d_shifted(p1, n3, dx3) : (double)p1 * dx3) + 0.25 * dx3;
+  return b;
+}
+// whether some c in [a, b] has |c - c0| <= r
+__device__ __forceinline__ bool src_reach(double a, double b, double c0, double r) {
+  return !(a - c0 > r) && !(b - c0 < -r);
+}
+// The points of this workgroup that the sources k < np may reach:
+// hit(box, k) gives a source's SrcHit, point(o, i1, i2, i3, k0, nl) adds the
+// sources k0 + list[0..nl) to the point at address o.  All 256 threads call.
+template <class H, class F>
+__device__ __forceinline__ void src_points(SrcShared& sh, int np, int n1, int n2, int n3, double dx1, double dx2,
+                                           double dx3, bool full, H hit, F point) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const long o0 = (long)blockIdx.x * SRC_POINTS, o1 = min(o0 + SRC_POINTS, (long)n1 * n2 * n3);
+  const long r0 = o0 / n1, r1 = (o1 - 1) / n1;
+  const SrcBox B = src_box(r0, r1, n2, n3, dx2, dx3, full);
+  for (int k0 = 0; k0 < np; k0 += SRC_LIST) {
+    const int k1 = min(np, k0 + SRC_LIST);
+    __syncthreads();  // the list of the previous round is read
+    if (tid == 0) { sh.lo = n1; sh.hi = -n1; }
+    int nl = 0;
+    for (int base = k0; base < k1; base += 256) {
+      const int k = base + tid;
+      const SrcHit h = k < k1 ? hit(B, k) : SrcHit{false, 0, 0};
+      const unsigned long long m = __ballot(h.hit);
+      __syncthreads();  // cnt of the previous round is read, lo and hi are set
+      if (lane == 0) sh.cnt[wave] = __popcll(m);
+      __syncthreads();
+      int at = nl;
+      for (int w = 0; w < 4; ++w) {
+        if (w < wave) at += sh.cnt[w];
+        nl += sh.cnt[w];
+      }
+      if (h.hit) {
+        sh.list[at + __popcll(m & ((1ull << lane) - 1))] = (unsigned short)(k - k0);
+        // samples -n1/2 <= j < n1/2 along x1 within reach, one more each side
+        const double a = (h.cx - h.r) / dx1 - 1.0, b = (h.cx + h.r) / dx1 + 1.0;
+        atomicMin(&sh.lo, a > -0.5 * n1 ? (int)floor(fmin(a, (double)n1)) : -((n1 + 1) / 2));
+        atomicMax(&sh.hi, b < 0.5 * n1 ? (int)ceil(fmax(b, -(double)n1)) : n1 / 2);
+      }
+    }
+    if (nl == 0) continue;
+    __syncthreads();
+    // i1 < n1/2 is j = i1 and the others j = i1 - n1
+    const int lo = max(sh.lo, n1 / 2 - n1), m = min(sh.hi, n1 / 2 - 1) - lo + 1;
+    if (m <= 0) continue;
+    const int total = (int)(r1 - r0 + 1) * m;
+    for (int q = tid; q < total; q += 256) {
+      const int row = q / m, j = lo + (q - row * m), i1 = j < 0 ? j + n1 : j;
+      const long o = (r0 + row) * n1 + i1;
+      if (o < o0 || o >= o1) continue;
+      point(o, i1, (int)((r0 + row) % n2), (int)((r0 + row) / n2), k0, nl);
+    }
+  }
+}
+static unsigned src_blocks(long n) { return (unsigned)((n + SRC_POINTS - 1) / SRC_POINTS); }
+
 // momentdensityshear (elastic3d.f90:2661-2750) of a list of patches added to
 // tau, as dislocations does at each event (relax.f90:1199-1206)
-__global__ void k_add_shear(const PlaneDev* __restrict__ P, const double* __restrict__ slip, int np, float rmu,
-                            Grid g, double dx1, double dx2, double dx3, float* tau) {
+__global__ __launch_bounds__(256) void k_add_shear(const PlaneDev* __restrict__ P, const double* __restrict__ slip,
+                                                   int np, float rmu, Grid g, double dx1, double dx2, double dx3,
+                                                   float* tau) {
+  __shared__ SrcShared sh;
   const long H = g.H;
-  for (long o = blockIdx.x * (long)blockDim.x + threadIdx.x; o < H; o += (long)gridDim.x * blockDim.x) {
-    const int i1 = o % g.n1, i2 = (o / g.n1) % g.n2, i3 = o / ((long)g.n1 * g.n2);
+  const auto hit = [&](const SrcBox& B, int k) {
+    const PlaneDev& p = P[k];
+    return SrcHit{src_reach(B.za, B.zb, p.z, p.Lp) && src_reach(B.ya, B.yb, p.y, p.Wp), p.x, p.Wp};
+  };
+  src_points(sh, np, g.n1, g.n2, g.h3, dx1, dx2, dx3, false, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
     const double x3 = (double)i3 * dx3;
     const double x1 = d_shifted(i1, g.n1, dx1), x2 = d_shifted(i2, g.n2, dx2);
     float acc[6] = {0, 0, 0, 0, 0, 0};
     bool any = false;
-    for (int k = 0; k < np; ++k) {
+    for (int l = 0; l < nl; ++l) {
+      const int k = k0 + sh.list[l];
       const PlaneDev& p = P[k];
       if (fabs(x3 - p.z) > p.Lp) continue;
       if ((fabs(x1 - p.x) > p.Wp) || (fabs(x2 - p.y) > p.Wp)) continue;
@@ -1382,7 +1485,7 @@ __global__ void k_add_shear(const PlaneDev* __restrict__ P, const double* __rest
     }
     if (any)
       for (int c = 0; c < 6; ++c) tau[c * H + o] = acc[c];
-  }
+  });
 }
 
 // The patch list m->shear_host and its slips in device form (grow-only)
@@ -1407,7 +1510,7 @@ static int stage_planes(relax_model_t* m, const double* slip) {
 // momentdensityshear of the staged patches [k0, k0+n) added to tau
 static int add_shear(relax_model_t* m, int k0, int n) {
   if (n == 0) return RELAX_OK;
-  k_add_shear<<<grid_1d(m->g.H), 256, 0, m->stream>>>(m->shear_dev + k0, m->shear_slip + k0, n,
+  k_add_shear<<<src_blocks(m->g.H), 256, 0, m->stream>>>(m->shear_dev + k0, m->shear_slip + k0, n,
                                                       2.0f * (float)m->desc.mu, m->g, m->desc.dx1, m->desc.dx2,
                                                       m->desc.dx3, m->tau);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
@@ -1429,73 +1532,84 @@ int relax_model_add_shear(relax_model_t* m, const relax_plane_t* patches, const 
 // the planes' contributions added in their order with the reference's
 // rounding (two FP32 roundings per plane and component); threads of the top
 // plane also add the surface traction (n sdyad mu s b) e3.
-__global__ void k_source(const PlaneDev* __restrict__ P, const double* __restrict__ slip, int np, double mu,
+__global__ __launch_bounds__(256) void k_source(const PlaneDev* __restrict__ P, const double* __restrict__ slip, int np, double mu,
                          int n1, int n2, int h3, double dx1, double dx2, double dx3, float* f, long ld, long fs,
                          float* t, long ts) {
-  const long N = (long)n1 * n2 * h3;
-  const long o = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (o >= N) return;
-  const int i1 = o % n1, i2 = (o / n1) % n2, i3 = o / ((long)n1 * n2);
-  const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
-  const long of = i1 + ld * (i2 + (long)n2 * i3), ot = i1 + ld * i2;
-  float f1 = f[of], f2 = f[fs + of], f3 = f[2 * fs + of];
-  float t1 = 0.f, t2 = 0.f, t3 = 0.f;
-  if (i3 == 0) { t1 = t[ot]; t2 = t[ts + ot]; t3 = t[2 * ts + ot]; }
-  for (int k = 0; k < np; ++k) {
+  __shared__ SrcShared sh;
+  const auto hit = [&](const SrcBox& B, int k) {
+    // the surface traction has no gate in depth
     const PlaneDev& p = P[k];
-    const double wl = fmax(p.Lp, p.Wp);
-    if ((fabs(x1 - p.x) > wl) || (fabs(x2 - p.y) > wl)) continue;
-    const double cs = p.cstrike, ss = p.sstrike, cd = p.cdip, sd = p.sdip;
-    const double xx = cs * x1 - ss * x2;
-    const double x1s = cd * xx - sd * x3, x1i = cd * xx + sd * x3;
-    if ((fabs(x1s - p.xr) > 7.01 * dx1) && (fabs(x1i - p.xr) > 7.01 * dx1)) continue;
-    const double x2s = ss * x1 + cs * x2, x3s = sd * xx + cd * x3, x3i = -sd * xx + cd * x3;
-    const double cr = cos(p.rake), sr = sin(p.rake), s = slip[k];
-    const double om2 = d_omega((x2s - p.yr) / p.W, p.beta);
-    if (i3 == 0) {
-      // the moment density at the surface (source and image apertures)
-      const double ap = d_gauss(x1s - p.xr, dx1) * om2 * d_omega((x3s - p.zr) / p.L, p.beta) +
-                        d_gauss(x1i - p.xr, dx1) * om2 * d_omega((x3i + p.zr) / p.L, p.beta);
-      const double n[3] = {p.n[0] * ap, p.n[1] * ap, p.n[2] * ap};
-      const double b[3] = {mu * s * p.r[0], mu * s * p.r[1], mu * s * p.r[2]};
-      t1 = t1 + (float)((n[0] * b[2] + n[2] * b[0]) / 2.0);
-      t2 = t2 + (float)((n[1] * b[2] + n[2] * b[1]) / 2.0);
-      t3 = t3 + (float)(n[2] * b[2]);
+    return SrcHit{src_reach(B.ya, B.yb, p.y, fmax(p.Lp, p.Wp)) &&
+           (B.top || src_reach(B.za, B.zb, p.z, p.Lp) || src_reach(B.za, B.zb, -p.z, p.Lp)), p.x, fmax(p.Lp, p.Wp)};
+  };
+  src_points(sh, np, n1, n2, h3, dx1, dx2, dx3, false, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+    const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
+    const long of = i1 + ld * (i2 + (long)n2 * i3), ot = i1 + ld * i2;
+    float f1, f2, f3, t1, t2, t3;
+    bool any = false;
+    for (int l = 0; l < nl; ++l) {
+      const int k = k0 + sh.list[l];
+      const PlaneDev& p = P[k];
+      const double wl = fmax(p.Lp, p.Wp);
+      if ((fabs(x1 - p.x) > wl) || (fabs(x2 - p.y) > wl)) continue;
+      const double cs = p.cstrike, ss = p.sstrike, cd = p.cdip, sd = p.sdip;
+      const double xx = cs * x1 - ss * x2;
+      const double x1s = cd * xx - sd * x3, x1i = cd * xx + sd * x3;
+      if ((fabs(x1s - p.xr) > 7.01 * dx1) && (fabs(x1i - p.xr) > 7.01 * dx1)) continue;
+      if (!any) {
+        f1 = f[of]; f2 = f[fs + of]; f3 = f[2 * fs + of];
+        if (i3 == 0) { t1 = t[ot]; t2 = t[ts + ot]; t3 = t[2 * ts + ot]; }
+        any = true;
+      }
+      const double x2s = ss * x1 + cs * x2, x3s = sd * xx + cd * x3, x3i = -sd * xx + cd * x3;
+      const double cr = cos(p.rake), sr = sin(p.rake), s = slip[k];
+      const double om2 = d_omega((x2s - p.yr) / p.W, p.beta);
+      if (i3 == 0) {
+        // the moment density at the surface (source and image apertures)
+        const double ap = d_gauss(x1s - p.xr, dx1) * om2 * d_omega((x3s - p.zr) / p.L, p.beta) +
+                          d_gauss(x1i - p.xr, dx1) * om2 * d_omega((x3i + p.zr) / p.L, p.beta);
+        const double n[3] = {p.n[0] * ap, p.n[1] * ap, p.n[2] * ap};
+        const double b[3] = {mu * s * p.r[0], mu * s * p.r[1], mu * s * p.r[2]};
+        t1 = t1 + (float)((n[0] * b[2] + n[2] * b[0]) / 2.0);
+        t2 = t2 + (float)((n[1] * b[2] + n[2] * b[1]) / 2.0);
+        t3 = t3 + (float)(n[2] * b[2]);
+      }
+      if ((fabs(x3 - p.z) > p.Lp) && (fabs(x3 + p.z) > p.Lp)) continue;
+      const double scale = -mu * s;
+      const double om2p = d_omegap((x2s - p.yr) / p.W, p.beta);
+      double g = d_gauss(x1s - p.xr, dx1);
+      double om3 = d_omega((x3s - p.zr) / p.L, p.beta);
+      const double sourc = scale * d_gaussp(x1s - p.xr, dx1) * om2 * om3;
+      const double dblcp = scale / p.W * g * om2p * om3;
+      const double dipcs = scale / p.L * g * om2 * d_omegap((x3s - p.zr) / p.L, p.beta);
+      g = d_gauss(x1i - p.xr, dx1);
+      om3 = d_omega((x3i + p.zr) / p.L, p.beta);
+      const double image = scale * d_gaussp(x1i - p.xr, dx1) * om2 * om3;
+      const double cplei = scale / p.W * g * om2p * om3;
+      if (2.01 * RELAX_DEG2RAD > p.dip) {
+        // near-vertical planes (dip measured from the vertical) use the image
+        f1 = (float)((double)f1 + (cr * ss * (sourc + image) + cr * cd * cs * (dblcp + cplei)));
+        f2 = (float)((double)f2 + (cr * cs * (sourc + image) - cr * cd * ss * (dblcp + cplei)));
+        f3 = (float)((double)f3 + (-cr * sd * (dblcp - cplei)));
+      } else {
+        f1 = (float)((double)f1 + (cr * ss * sourc + cr * cd * cs * dblcp));
+        f2 = (float)((double)f2 + (cr * cs * sourc - cr * cd * ss * dblcp));
+        f3 = (float)((double)f3 + (-cr * sd * dblcp));
+      }
+      f1 = (float)((double)f1 + (cd * sr * cs * dipcs + sd * sr * cs * sourc));
+      f2 = (float)((double)f2 + (-cd * sr * ss * dipcs - sd * sr * ss * sourc));
+      f3 = (float)((double)f3 + (cd * sr * sourc - sd * sr * dipcs));
     }
-    if ((fabs(x3 - p.z) > p.Lp) && (fabs(x3 + p.z) > p.Lp)) continue;
-    const double scale = -mu * s;
-    const double om2p = d_omegap((x2s - p.yr) / p.W, p.beta);
-    double g = d_gauss(x1s - p.xr, dx1);
-    double om3 = d_omega((x3s - p.zr) / p.L, p.beta);
-    const double sourc = scale * d_gaussp(x1s - p.xr, dx1) * om2 * om3;
-    const double dblcp = scale / p.W * g * om2p * om3;
-    const double dipcs = scale / p.L * g * om2 * d_omegap((x3s - p.zr) / p.L, p.beta);
-    g = d_gauss(x1i - p.xr, dx1);
-    om3 = d_omega((x3i + p.zr) / p.L, p.beta);
-    const double image = scale * d_gaussp(x1i - p.xr, dx1) * om2 * om3;
-    const double cplei = scale / p.W * g * om2p * om3;
-    if (2.01 * RELAX_DEG2RAD > p.dip) {
-      // near-vertical planes (dip measured from the vertical) use the image
-      f1 = (float)((double)f1 + (cr * ss * (sourc + image) + cr * cd * cs * (dblcp + cplei)));
-      f2 = (float)((double)f2 + (cr * cs * (sourc + image) - cr * cd * ss * (dblcp + cplei)));
-      f3 = (float)((double)f3 + (-cr * sd * (dblcp - cplei)));
-    } else {
-      f1 = (float)((double)f1 + (cr * ss * sourc + cr * cd * cs * dblcp));
-      f2 = (float)((double)f2 + (cr * cs * sourc - cr * cd * ss * dblcp));
-      f3 = (float)((double)f3 + (-cr * sd * dblcp));
-    }
-    f1 = (float)((double)f1 + (cd * sr * cs * dipcs + sd * sr * cs * sourc));
-    f2 = (float)((double)f2 + (-cd * sr * ss * dipcs - sd * sr * ss * sourc));
-    f3 = (float)((double)f3 + (cd * sr * sourc - sd * sr * dipcs));
-  }
-  f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3;
-  if (i3 == 0) { t[ot] = t1; t[ts + ot] = t2; t[2 * ts + ot] = t3; }
+    if (!any) return;
+    f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3;
+    if (i3 == 0) { t[ot] = t1; t[ts + ot] = t2; t[2 * ts + ot] = t3; }
+  });
 }
 
 int launch_source(const PlaneDev* P, const double* slip, int np, double mu, int n1, int n2, int h3, double dx1,
                   double dx2, double dx3, float* f, long ld, long fs, float* t, long ts, hipStream_t st) {
   const long N = (long)n1 * n2 * h3;
-  k_source<<<(unsigned)((N + 255) / 256), 256, 0, st>>>(P, slip, np, mu, n1, n2, h3, dx1, dx2, dx3, f, ld, fs, t,
+  k_source<<<src_blocks(N), 256, 0, st>>>(P, slip, np, mu, n1, n2, h3, dx1, dx2, dx3, f, ld, fs, t,
                                                         ts);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
@@ -1504,169 +1618,196 @@ int launch_source(const PlaneDev* P, const double* slip, int np, double mu, int 
 // depth (x3 from the shifted coordinates, so that the images above the
 // surface land in the lower half of the grid), the cracks added in their
 // order with one rounding each
-__global__ void k_tensile_source(const PlaneDev* __restrict__ P, const double* __restrict__ opening, int np,
+__global__ __launch_bounds__(256) void k_tensile_source(const PlaneDev* __restrict__ P, const double* __restrict__ opening, int np,
                                  double lambda, double mu, int n1, int n2, int n3, double dx1, double dx2, double dx3,
                                  float* f, long ld, long fs) {
-  const long o = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (o >= (long)n1 * n2 * n3) return;
-  const int i1 = o % n1, i2 = (o / n1) % n2, i3 = o / ((long)n1 * n2);
-  const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = d_shifted(i3, n3, dx3);
-  const long of = i1 + ld * (i2 + (long)n2 * i3);
-  float f1 = f[of], f2 = f[fs + of], f3 = f[2 * fs + of];
-  bool any = false;
-  for (int k = 0; k < np; ++k) {
+  __shared__ SrcShared sh;
+  const auto hit = [&](const SrcBox& B, int k) {
     const PlaneDev& p = P[k];
-    if ((fabs(x3 - p.z) > p.Lp) && (fabs(x3 + p.z) > p.Lp)) continue;
-    if ((fabs(x1 - p.x) > p.Wp) || (fabs(x2 - p.y) > p.Wp)) continue;
-    const double cs = p.cstrike, ss = p.sstrike, cd = p.cdip, sd = p.sdip;
-    const double xx = cs * x1 - ss * x2;
-    const double x1s = cd * xx - sd * x3, x1i = cd * xx + sd * x3;
-    if ((fabs(x1s - p.xr) > 7.01 * dx1) && (fabs(x1i - p.xr) > 7.01 * dx1)) continue;
-    const double x2s = ss * x1 + cs * x2, x3s = sd * xx + cd * x3, x3i = -sd * xx + cd * x3;
-    const double scale1 = -opening[k] * (lambda + 2.0 * mu), scale2 = -opening[k] * lambda;
-    double t1 = d_gauss(x1s - p.xr, dx1);
-    const double t2 = d_omega((x2s - p.yr) / p.W, p.beta);
-    double t3 = d_omega((x3s - p.zr) / p.L, p.beta);
-    const double sourc = scale1 * d_gaussp(x1s - p.xr, dx1) * t2 * t3;
-    const double dblcp = scale2 / p.W * t1 * d_omegap((x2s - p.yr) / p.W, p.beta) * t3;
-    const double dipcs = scale2 / p.L * t1 * t2 * d_omegap((x3s - p.zr) / p.L, p.beta);
-    t1 = d_gauss(x1i - p.xr, dx1);
-    t3 = d_omega((x3i + p.zr) / p.L, p.beta);
-    const double image = scale1 * d_gaussp(x1i - p.xr, dx1) * t2 * t3;
-    const double cplei = scale2 / p.W * t1 * d_omegap((x2s - p.yr) / p.W, p.beta) * t3;
-    const double dipci = scale2 / p.L * t1 * t2 * d_omegap((x3i + p.zr) / p.L, p.beta);
-    f1 = (float)((double)f1 + cs * cd * (sourc + image) + ss * (dblcp + cplei) + cs * sd * (dipcs + dipci));
-    f2 = (float)((double)f2 - ss * cd * (sourc + image) + cs * (dblcp + cplei) - ss * sd * (dipcs + dipci));
-    f3 = (float)((double)f3 - sd * (sourc - image) + cd * (dipcs - dipci));
-    any = true;
-  }
-  if (any) { f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3; }
+    return SrcHit{src_reach(B.ya, B.yb, p.y, p.Wp) &&
+           (src_reach(B.za, B.zb, p.z, p.Lp) || src_reach(B.za, B.zb, -p.z, p.Lp)), p.x, p.Wp};
+  };
+  src_points(sh, np, n1, n2, n3, dx1, dx2, dx3, true, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+    const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = d_shifted(i3, n3, dx3);
+    const long of = i1 + ld * (i2 + (long)n2 * i3);
+    float f1, f2, f3;
+    bool any = false;
+    for (int l = 0; l < nl; ++l) {
+      const int k = k0 + sh.list[l];
+      const PlaneDev& p = P[k];
+      if ((fabs(x3 - p.z) > p.Lp) && (fabs(x3 + p.z) > p.Lp)) continue;
+      if ((fabs(x1 - p.x) > p.Wp) || (fabs(x2 - p.y) > p.Wp)) continue;
+      const double cs = p.cstrike, ss = p.sstrike, cd = p.cdip, sd = p.sdip;
+      const double xx = cs * x1 - ss * x2;
+      const double x1s = cd * xx - sd * x3, x1i = cd * xx + sd * x3;
+      if ((fabs(x1s - p.xr) > 7.01 * dx1) && (fabs(x1i - p.xr) > 7.01 * dx1)) continue;
+      const double x2s = ss * x1 + cs * x2, x3s = sd * xx + cd * x3, x3i = -sd * xx + cd * x3;
+      const double scale1 = -opening[k] * (lambda + 2.0 * mu), scale2 = -opening[k] * lambda;
+      double t1 = d_gauss(x1s - p.xr, dx1);
+      const double t2 = d_omega((x2s - p.yr) / p.W, p.beta);
+      double t3 = d_omega((x3s - p.zr) / p.L, p.beta);
+      const double sourc = scale1 * d_gaussp(x1s - p.xr, dx1) * t2 * t3;
+      const double dblcp = scale2 / p.W * t1 * d_omegap((x2s - p.yr) / p.W, p.beta) * t3;
+      const double dipcs = scale2 / p.L * t1 * t2 * d_omegap((x3s - p.zr) / p.L, p.beta);
+      t1 = d_gauss(x1i - p.xr, dx1);
+      t3 = d_omega((x3i + p.zr) / p.L, p.beta);
+      const double image = scale1 * d_gaussp(x1i - p.xr, dx1) * t2 * t3;
+      const double cplei = scale2 / p.W * t1 * d_omegap((x2s - p.yr) / p.W, p.beta) * t3;
+      const double dipci = scale2 / p.L * t1 * t2 * d_omegap((x3i + p.zr) / p.L, p.beta);
+      if (!any) { f1 = f[of]; f2 = f[fs + of]; f3 = f[2 * fs + of]; }
+      f1 = (float)((double)f1 + cs * cd * (sourc + image) + ss * (dblcp + cplei) + cs * sd * (dipcs + dipci));
+      f2 = (float)((double)f2 - ss * cd * (sourc + image) + cs * (dblcp + cplei) - ss * sd * (dipcs + dipci));
+      f3 = (float)((double)f3 - sd * (sourc - image) + cd * (dipcs - dipci));
+      any = true;
+    }
+    if (any) { f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3; }
+  });
 }
 
 // mogisource, elastic3d.f90:2458-2509: point dilatation sources (volume
 // change in slip) and their images over the full depth
-__global__ void k_mogi_source(const relax_source_t* __restrict__ M, int nm, double lambda, double mu, int n1, int n2,
+__global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __restrict__ M, int nm, double lambda, double mu, int n1, int n2,
                               int n3, double dx1, double dx2, double dx3, float* f, long ld, long fs) {
-  const long o = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (o >= (long)n1 * n2 * n3) return;
-  const int i1 = o % n1, i2 = (o / n1) % n2, i3 = o / ((long)n1 * n2);
-  const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = d_shifted(i3, n3, dx3);
-  const double Wp = 6.0 * fmax(dx1, fmax(dx2, dx3)), Lp = Wp;
-  const long of = i1 + ld * (i2 + (long)n2 * i3);
-  float f1 = f[of], f2 = f[fs + of], f3 = f[2 * fs + of];
-  bool any = false;
-  for (int k = 0; k < nm; ++k) {
+  __shared__ SrcShared sh;
+  const auto hit = [&](const SrcBox& B, int k) {
     const relax_source_t& s = M[k];
-    if ((fabs(x3 - s.z) > Lp) && (fabs(x3 + s.z) > Lp)) continue;
-    if ((fabs(x1 - s.x) > Wp) || (fabs(x2 - s.y) > Wp)) continue;
-    const double scale = -(lambda + 2.0 * mu / 3.0) * s.slip;
-    const double t1 = d_gauss(x1 - s.x, dx1), t2 = d_gauss(x2 - s.y, dx2);
-    double t3 = d_gauss(x3 - s.z, dx3);
-    const double s1 = scale * d_gaussp(x1 - s.x, dx1) * t2 * t3, s2 = scale * t1 * d_gaussp(x2 - s.y, dx2) * t3;
-    const double s3 = scale * t1 * t2 * d_gaussp(x3 - s.z, dx3);
-    t3 = d_gauss(x3 + s.z, dx3);
-    const double m1 = scale * d_gaussp(x1 - s.x, dx1) * t2 * t3, m2 = scale * t1 * d_gaussp(x2 - s.y, dx2) * t3;
-    const double m3 = scale * t1 * t2 * d_gaussp(x3 + s.z, dx3);
-    f1 = (float)((double)f1 + (s1 + m1));
-    f2 = (float)((double)f2 + (s2 + m2));
-    f3 = (float)((double)f3 + (s3 - m3));
-    any = true;
-  }
-  if (any) { f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3; }
+    const double r = 6.0 * fmax(dx1, fmax(dx2, dx3));
+    return SrcHit{src_reach(B.ya, B.yb, s.y, r) && (src_reach(B.za, B.zb, s.z, r) || src_reach(B.za, B.zb, -s.z, r)), s.x, r};
+  };
+  src_points(sh, nm, n1, n2, n3, dx1, dx2, dx3, true, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+    // a source at the surface and its image cancel exactly in f3
+#pragma clang fp contract(off)
+    const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = d_shifted(i3, n3, dx3);
+    const double Wp = 6.0 * fmax(dx1, fmax(dx2, dx3)), Lp = Wp;
+    const long of = i1 + ld * (i2 + (long)n2 * i3);
+    float f1, f2, f3;
+    bool any = false;
+    for (int l = 0; l < nl; ++l) {
+      const int k = k0 + sh.list[l];
+      const relax_source_t& s = M[k];
+      if ((fabs(x3 - s.z) > Lp) && (fabs(x3 + s.z) > Lp)) continue;
+      if ((fabs(x1 - s.x) > Wp) || (fabs(x2 - s.y) > Wp)) continue;
+      const double scale = -(lambda + 2.0 * mu / 3.0) * s.slip;
+      const double t1 = d_gauss(x1 - s.x, dx1), t2 = d_gauss(x2 - s.y, dx2);
+      double t3 = d_gauss(x3 - s.z, dx3);
+      const double s1 = scale * d_gaussp(x1 - s.x, dx1) * t2 * t3, s2 = scale * t1 * d_gaussp(x2 - s.y, dx2) * t3;
+      const double s3 = scale * t1 * t2 * d_gaussp(x3 - s.z, dx3);
+      t3 = d_gauss(x3 + s.z, dx3);
+      const double m1 = scale * d_gaussp(x1 - s.x, dx1) * t2 * t3, m2 = scale * t1 * d_gaussp(x2 - s.y, dx2) * t3;
+      const double m3 = scale * t1 * t2 * d_gaussp(x3 + s.z, dx3);
+      if (!any) { f1 = f[of]; f2 = f[fs + of]; f3 = f[2 * fs + of]; }
+      f1 = (float)((double)f1 + (s1 + m1));
+      f2 = (float)((double)f2 + (s2 + m2));
+      f3 = (float)((double)f3 + (s3 - m3));
+      any = true;
+    }
+    if (any) { f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3; }
+  });
 }
 
 // momentdensitytensile, elastic3d.f90:3137-3215: Hooke's law of
 // n sdyad (opening n), n carrying the aperture; each crack adds in turn
-__global__ void k_add_tensile(const PlaneDev* __restrict__ P, const double* __restrict__ opening, int np,
+__global__ __launch_bounds__(256) void k_add_tensile(const PlaneDev* __restrict__ P, const double* __restrict__ opening, int np,
                               double lambda, double mu, int n1, int n2, int h3, double dx1, double dx2, double dx3,
                               float* sig, long H) {
-  const long o = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (o >= (long)n1 * n2 * h3) return;
-  const int i1 = o % n1, i2 = (o / n1) % n2, i3 = o / ((long)n1 * n2);
-  const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
-  const float m2 = (float)(2.0 * mu);
-  float acc[6];
-  bool any = false;
-  for (int k = 0; k < np; ++k) {
+  __shared__ SrcShared sh;
+  const auto hit = [&](const SrcBox& B, int k) {
     const PlaneDev& p = P[k];
-    if (fabs(x3 - p.z) > p.Lp) continue;
-    if ((fabs(x1 - p.x) > p.Wp) || (fabs(x2 - p.y) > p.Wp)) continue;
-    const double xx = p.cstrike * x1 - p.sstrike * x2;
-    const double x1s = p.cdip * xx - p.sdip * x3, x1i = p.cdip * xx + p.sdip * x3;
-    if ((fabs(x1s - p.xr) > 7.01 * dx1) && (fabs(x1i - p.xr) > 7.01 * dx1)) continue;
-    const double x2s = p.sstrike * x1 + p.cstrike * x2;
-    const double x3s = p.sdip * xx + p.cdip * x3, x3i = -p.sdip * xx + p.cdip * x3;
-    const double t2 = d_omega((x2s - p.yr) / p.W, p.beta);
-    double ap = d_gauss(x1s - p.xr, dx1) * t2 * d_omega((x3s - p.zr) / p.L, p.beta);
-    ap = ap + d_gauss(x1i - p.xr, dx1) * t2 * d_omega((x3i + p.zr) / p.L, p.beta);
-    const double n[3] = {p.n[0] * ap, p.n[1] * ap, p.n[2] * ap};
-    const double b[3] = {opening[k] * n[0], opening[k] * n[1], opening[k] * n[2]};
-    float e[6] = {(float)(n[0] * b[0]), (float)((n[0] * b[1] + n[1] * b[0]) / 2.0),
-                  (float)((n[0] * b[2] + n[2] * b[0]) / 2.0), (float)(n[1] * b[1]),
-                  (float)((n[1] * b[2] + n[2] * b[1]) / 2.0), (float)(n[2] * b[2])};
-    // isotropicstressstrain, elastic3d.f90:129-142
-    const double tr = (double)(e[0] + e[3] + e[5]);
-    for (float& v : e) v = m2 * v;
-    e[0] = (float)((double)e[0] + lambda * tr);
-    e[3] = (float)((double)e[3] + lambda * tr);
-    e[5] = (float)((double)e[5] + lambda * tr);
-    if (!any)
-      for (int c = 0; c < 6; ++c) acc[c] = sig[c * H + o];
-    for (int c = 0; c < 6; ++c) acc[c] = acc[c] + e[c];
-    any = true;
-  }
-  if (any)
-    for (int c = 0; c < 6; ++c) sig[c * H + o] = acc[c];
+    return SrcHit{src_reach(B.ya, B.yb, p.y, p.Wp) && src_reach(B.za, B.zb, p.z, p.Lp), p.x, p.Wp};
+  };
+  src_points(sh, np, n1, n2, h3, dx1, dx2, dx3, false, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+    const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
+    const float m2 = (float)(2.0 * mu);
+    float acc[6];
+    bool any = false;
+    for (int l = 0; l < nl; ++l) {
+      const int k = k0 + sh.list[l];
+      const PlaneDev& p = P[k];
+      if (fabs(x3 - p.z) > p.Lp) continue;
+      if ((fabs(x1 - p.x) > p.Wp) || (fabs(x2 - p.y) > p.Wp)) continue;
+      const double xx = p.cstrike * x1 - p.sstrike * x2;
+      const double x1s = p.cdip * xx - p.sdip * x3, x1i = p.cdip * xx + p.sdip * x3;
+      if ((fabs(x1s - p.xr) > 7.01 * dx1) && (fabs(x1i - p.xr) > 7.01 * dx1)) continue;
+      const double x2s = p.sstrike * x1 + p.cstrike * x2;
+      const double x3s = p.sdip * xx + p.cdip * x3, x3i = -p.sdip * xx + p.cdip * x3;
+      const double t2 = d_omega((x2s - p.yr) / p.W, p.beta);
+      double ap = d_gauss(x1s - p.xr, dx1) * t2 * d_omega((x3s - p.zr) / p.L, p.beta);
+      ap = ap + d_gauss(x1i - p.xr, dx1) * t2 * d_omega((x3i + p.zr) / p.L, p.beta);
+      const double n[3] = {p.n[0] * ap, p.n[1] * ap, p.n[2] * ap};
+      const double b[3] = {opening[k] * n[0], opening[k] * n[1], opening[k] * n[2]};
+      float e[6] = {(float)(n[0] * b[0]), (float)((n[0] * b[1] + n[1] * b[0]) / 2.0),
+                    (float)((n[0] * b[2] + n[2] * b[0]) / 2.0), (float)(n[1] * b[1]),
+                    (float)((n[1] * b[2] + n[2] * b[1]) / 2.0), (float)(n[2] * b[2])};
+      // isotropicstressstrain, elastic3d.f90:129-142
+      const double tr = (double)(e[0] + e[3] + e[5]);
+      for (float& v : e) v = m2 * v;
+      e[0] = (float)((double)e[0] + lambda * tr);
+      e[3] = (float)((double)e[3] + lambda * tr);
+      e[5] = (float)((double)e[5] + lambda * tr);
+      if (!any)
+        for (int c = 0; c < 6; ++c) acc[c] = sig[c * H + o];
+      for (int c = 0; c < 6; ++c) acc[c] = acc[c] + e[c];
+      any = true;
+    }
+    if (any)
+      for (int c = 0; c < 6; ++c) sig[c * H + o] = acc[c];
+  });
 }
 
 // momentdensitymogi, elastic3d.f90:3240-3286: kappa o G on the diagonal
-__global__ void k_add_mogi(const relax_source_t* __restrict__ M, int nm, double lambda, double mu, int n1, int n2,
+__global__ __launch_bounds__(256) void k_add_mogi(const relax_source_t* __restrict__ M, int nm, double lambda, double mu, int n1, int n2,
                            int h3, double dx1, double dx2, double dx3, float* sig, long H) {
-  const long o = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (o >= (long)n1 * n2 * h3) return;
-  const int i1 = o % n1, i2 = (o / n1) % n2, i3 = o / ((long)n1 * n2);
-  const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
-  const double kappa = lambda + 2.0 / 3.0 * mu;
-  const double Wp = 6.0 * fmax(dx1, fmax(dx2, dx3)), Lp = Wp;
-  float a11 = 0.f, a22 = 0.f, a33 = 0.f;
-  bool any = false;
-  for (int k = 0; k < nm; ++k) {
+  __shared__ SrcShared sh;
+  const auto hit = [&](const SrcBox& B, int k) {
     const relax_source_t& s = M[k];
-    if (fabs(x3 - s.z) > Lp) continue;
-    if ((fabs(x1 - s.x) > Wp) || (fabs(x2 - s.y) > Wp)) continue;
-    double g = s.slip * d_gauss(x1 - s.x, dx1) * d_gauss(x2 - s.y, dx2) * d_gauss(x3 - s.z, dx3);
-    g = kappa * g;
-    const float m = (float)g;
-    if (!any) { a11 = sig[o]; a22 = sig[3 * H + o]; a33 = sig[5 * H + o]; }
-    a11 = a11 + m; a22 = a22 + m; a33 = a33 + m;
-    any = true;
-  }
-  if (any) { sig[o] = a11; sig[3 * H + o] = a22; sig[5 * H + o] = a33; }
+    const double r = 6.0 * fmax(dx1, fmax(dx2, dx3));
+    return SrcHit{src_reach(B.ya, B.yb, s.y, r) && src_reach(B.za, B.zb, s.z, r), s.x, r};
+  };
+  src_points(sh, nm, n1, n2, h3, dx1, dx2, dx3, false, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+    const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
+    const double kappa = lambda + 2.0 / 3.0 * mu;
+    const double Wp = 6.0 * fmax(dx1, fmax(dx2, dx3)), Lp = Wp;
+    float a11 = 0.f, a22 = 0.f, a33 = 0.f;
+    bool any = false;
+    for (int l = 0; l < nl; ++l) {
+      const int k = k0 + sh.list[l];
+      const relax_source_t& s = M[k];
+      if (fabs(x3 - s.z) > Lp) continue;
+      if ((fabs(x1 - s.x) > Wp) || (fabs(x2 - s.y) > Wp)) continue;
+      double g = s.slip * d_gauss(x1 - s.x, dx1) * d_gauss(x2 - s.y, dx2) * d_gauss(x3 - s.z, dx3);
+      g = kappa * g;
+      const float m = (float)g;
+      if (!any) { a11 = sig[o]; a22 = sig[3 * H + o]; a33 = sig[5 * H + o]; }
+      a11 = a11 + m; a22 = a22 + m; a33 = a33 + m;
+      any = true;
+    }
+    if (any) { sig[o] = a11; sig[3 * H + o] = a22; sig[5 * H + o] = a33; }
+  });
 }
 
 static unsigned blocks_of(long n) { return (unsigned)((n + 255) / 256); }
 
 int launch_tensile_source(const PlaneDev* P, const double* opening, int np, double lambda, double mu, int n1, int n2,
                           int n3, double dx1, double dx2, double dx3, float* f, long ld, long fs, hipStream_t st) {
-  k_tensile_source<<<blocks_of((long)n1 * n2 * n3), 256, 0, st>>>(P, opening, np, lambda, mu, n1, n2, n3, dx1, dx2,
+  k_tensile_source<<<src_blocks((long)n1 * n2 * n3), 256, 0, st>>>(P, opening, np, lambda, mu, n1, n2, n3, dx1, dx2,
                                                                   dx3, f, ld, fs);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 int launch_mogi_source(const relax_source_t* M, int nm, double lambda, double mu, int n1, int n2, int n3,
                        double dx1, double dx2, double dx3, float* f, long ld, long fs, hipStream_t st) {
-  k_mogi_source<<<blocks_of((long)n1 * n2 * n3), 256, 0, st>>>(M, nm, lambda, mu, n1, n2, n3, dx1, dx2, dx3, f, ld,
+  k_mogi_source<<<src_blocks((long)n1 * n2 * n3), 256, 0, st>>>(M, nm, lambda, mu, n1, n2, n3, dx1, dx2, dx3, f, ld,
                                                                fs);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 int launch_add_tensile(const PlaneDev* P, const double* opening, int np, double lambda, double mu, int n1, int n2,
                        int h3, double dx1, double dx2, double dx3, float* sig, long H, hipStream_t st) {
-  k_add_tensile<<<blocks_of((long)n1 * n2 * h3), 256, 0, st>>>(P, opening, np, lambda, mu, n1, n2, h3, dx1, dx2, dx3,
+  k_add_tensile<<<src_blocks((long)n1 * n2 * h3), 256, 0, st>>>(P, opening, np, lambda, mu, n1, n2, h3, dx1, dx2, dx3,
                                                                sig, H);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 int launch_add_mogi(const relax_source_t* M, int nm, double lambda, double mu, int n1, int n2, int h3, double dx1,
                     double dx2, double dx3, float* sig, long H, hipStream_t st) {
-  k_add_mogi<<<blocks_of((long)n1 * n2 * h3), 256, 0, st>>>(M, nm, lambda, mu, n1, n2, h3, dx1, dx2, dx3, sig, H);
+  k_add_mogi<<<src_blocks((long)n1 * n2 * h3), 256, 0, st>>>(M, nm, lambda, mu, n1, n2, h3, dx1, dx2, dx3, sig, H);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 
@@ -1903,7 +2044,7 @@ int relax_model_set_interseismic(relax_model_t* m, const relax_event_t* ev) {
   if ((rc = stage_planes(m, amp.data()))) return rc;
   const double dx1 = m->desc.dx1, dx2 = m->desc.dx2, dx3 = m->desc.dx3;
   if (ns) {
-    k_add_shear<<<grid_1d(H), 256, 0, m->stream>>>(m->shear_dev, m->shear_slip, ns, 2.0f * (float)m->desc.mu, g,
+    k_add_shear<<<src_blocks(H), 256, 0, m->stream>>>(m->shear_dev, m->shear_slip, ns, 2.0f * (float)m->desc.mu, g,
                                                    dx1, dx2, dx3, m->mi);
     if (hipGetLastError() != hipSuccess) return RELAX_ERR_HIP;
   }
