@@ -580,16 +580,197 @@ __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu,
   }
 }
 
+// The register form for H3 = 256 (16 x 16).  At this depth the three components
+// of a thread's frequencies (96 registers) do not fit beside step A, so a
+// thread has one component, c = tid / 64 (a wave each), and 16 frequencies of
+// either half; every thread takes part in every step, for the even half and
+// then the odd.  For the sum k.c of elasticresponse the spectrum goes through
+// the transpose buffer once more.
+//
+// 4 columns per workgroup, 30 KB of LDS, three waves: workgroups this small
+// wait for few others at each of the 15 barriers and four of them share a
+// compute unit.  512x512x512: 800 us (LDS form k_green_columns 1112; 8 columns
+// 1257, though its rows are 64 contiguous bytes; the vector instructions take
+// 605, the memory 320).  Four waves per SIMD instead of three: the same.
+constexpr int DEEP_TX = 4;  // columns per workgroup
+__global__ __launch_bounds__(48 * DEEP_TX, 3) void k_green_deep(ColumnConsts C, double mu, double alpha, double gamma,
+                                                               int n1, int n2, MPtr<float2> W_m, MPtr<float2> NQ_m,
+                                                               MPtr<const float2> TM_m, MPtr<const float2> TN_m,
+                                                               const float2* __restrict__ tw3, int l2) {
+  constexpr int H3 = 256, TX = DEEP_TX, NT = 48 * TX, Q = 16;
+  constexpr int RS = 16 * TX + TX;         // float2 per (c, j) group (j groups on alternate banks)
+  constexpr unsigned RSRC3 = 0x00020000u;  // raw buffer, 32-bit data format
+  __shared__ float2 buf[3 * Q * RS];
+  __shared__ float2 stw[H3];   // w_n3^z
+  __shared__ float2 tws[256];  // w_H3^(j k1), row j
+  __shared__ float2 red[2][3][TX];
+  __shared__ float2 pv[3][TX];
+  __shared__ CerrutiCol ccs[TX];
+  const int tid = threadIdx.x;
+  const int col = tid % TX, r = (tid / TX) % 16;  // r: j of step A, k1 of step B
+  static_assert(16 * TX == 64, "a component is a wave");
+  const int c = __builtin_amdgcn_readfirstlane(tid / 64);
+
+  const GreenTileAddr A = green_tile<TX>(xcd_tile(blockIdx.x, gridDim.x), col, n1, n2, H3, l2, W_m.at(blockIdx.y),
+                                         NQ_m.at(blockIdx.y), TM_m.at(blockIdx.y), TN_m.at(blockIdx.y));
+  const unsigned voff = (unsigned)((r * A.zs + col) * (long)sizeof(float2));
+  // a component is under 2 GiB (n1, n2 <= 1024)
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(A.base + c * A.cs, (short)0, 0x7fffffff, RSRC3);
+  const unsigned zstep = (unsigned)(Q * A.zs * (long)sizeof(float2));  // uniform: the scalar offset
+
+  float2 x[16];
+  auto load = [&]() {
+#pragma unroll
+    for (int m = 0; m < 16; ++m)
+      x[m] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, m * zstep, 0));
+  };
+  float2* const arow = buf + (c * Q + r) * RS + col;        // step A: group (c, j = r), [k1 * TX]
+  float2* const brow = buf + c * Q * RS + r * TX + col;     // step B: column k1 = r of component c, [j * RS]
+  const float2* const prow = buf + r * TX + col;            // the three components of a frequency
+  load();
+  for (int e = tid; e < 256; e += NT) {
+    stw[e] = tw3[e];
+    tws[e] = tw3[2 * (e >> 4) * (e & 15)];
+  }
+  __syncthreads();
+
+  const float k1w = (float)A.k1i * C.ik1;
+  const float k2w = wavenumber23f(A.k2i, n2, C.ik2);
+  const float kh2 = k1w * k1w + k2w * k2w;
+  // wavenumber23f(2 (r + 16 k2) + odd, 512): negative from k2 = 8 on
+  auto wave3 = [&](int k2, bool odd) {
+    return ((float)(2 * r + (odd ? 1 : 0)) + (float)(k2 < Q / 2 ? 32 * k2 : 32 * k2 - 2 * H3)) * C.ik3;
+  };
+  // this component's wavenumber is kx + kz k3
+  const float kx = c == 0 ? k1w : c == 1 ? k2w : 0.f, kz = c == 2 ? 1.f : 0.f;
+  // this component's sums of k3 u and u over the frequencies
+  float2 Sk = make_float2(0.f, 0.f), Su = Sk;
+  auto forward = [&](bool odd, float2* X) {
+    if (odd) {
+#pragma unroll
+      for (int m = 0; m < 16; ++m) x[m] = cmul(x[m], stw[Q * m + r]);
+    }
+    dft16<-1>(x);
+    arow[0] = x[0];
+#pragma unroll
+    for (int k1 = 1; k1 < 16; ++k1) arow[k1 * TX] = cmul(x[k1], tws[16 * r + k1]);
+    if (!odd) load();  // in flight during the even half's step B
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < Q; ++j) X[j] = brow[j * RS];
+    dft16<-1>(X);
+    __syncthreads();
+    // elasticresponse (green.f90:63-86) as s c - k (k.c)
+#pragma unroll
+    for (int k2 = 0; k2 < Q; ++k2) brow[k2 * RS] = X[k2];
+    __syncthreads();
+#pragma unroll
+    for (int k2 = 0; k2 < Q; ++k2) {
+      const float k3 = wave3(k2, odd);
+      const float kc = fmaf(kz, k3, kx);
+      const float r2 = fmaf(k3, k3, kh2);
+      const float denom = C.ratio1 * __builtin_amdgcn_rcpf(r2 * r2);
+      const float s = r2 * C.ratio2p1;
+      const float2 a1 = prow[k2 * RS], a2 = prow[(Q + k2) * RS], a3 = prow[(2 * Q + k2) * RS];
+      const float2 d = make_float2(k1w * a1.x + k2w * a2.x + k3 * a3.x, k1w * a1.y + k2w * a2.y + k3 * a3.y);
+      float2 a = make_float2((s * X[k2].x - kc * d.x) * denom, (s * X[k2].y - kc * d.y) * denom);
+      // the k = 0 frequency is zeroed (green.f90:96-99)
+      if (!odd && k2 == 0 && A.k1i == 0 && A.k2i == 0 && r == 0) a = make_float2(0.f, 0.f);
+      X[k2] = a;
+      Sk = make_float2(fmaf(k3, a.x, Sk.x), fmaf(k3, a.y, Sk.y));
+      Su = cadd(Su, a);
+      if (k2 % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // the other components' reads stay few in registers
+    }
+    __syncthreads();
+  };
+  float2 X0[Q], X1[Q];
+  forward(false, X0);
+  forward(true, X1);
+
+  // a column's sums: lanes TX apart in the component's wave
+#pragma unroll
+  for (int off = 32; off >= TX; off >>= 1) {
+    Sk.x += __shfl_xor(Sk.x, off); Sk.y += __shfl_xor(Sk.y, off);
+    Su.x += __shfl_xor(Su.x, off); Su.y += __shfl_xor(Su.y, off);
+  }
+  if ((tid & 63) < TX) { red[0][c][col] = Sk; red[1][c][col] = Su; }
+  __syncthreads();
+  if (tid < 3 * TX) {
+    const int d = tid / TX, t = tid % TX;
+    const float q1 = __shfl(k1w, t), q2 = __shfl(k2w, t);
+    // sum_k3 of the traction summands (green.f90:357-359):
+    //   i 2 pi mu (k3 u1 + k1 u3), i 2 pi mu (k3 u2 + k2 u3),
+    //   i 2 pi ((l+2m) k3 u3 + l (k1 u1 + k2 u2)) - 2 mu alpha gamma u3
+    const float2 u3 = red[1][2][t];
+    float2 acc;
+    if (d < 2) {
+      const float qc = d == 0 ? q1 : q2;
+      const float2 sk = red[0][d][t];
+      const float2 a = make_float2(sk.x + qc * u3.x, sk.y + qc * u3.y);
+      acc = make_float2(-C.mu2pi * a.y, C.mu2pi * a.x);
+    } else {
+      const float2 sk = red[0][2][t], u1 = red[1][0][t], u2 = red[1][1][t];
+      const float2 h = make_float2(q1 * u1.x + q2 * u2.x, q1 * u1.y + q2 * u2.y);
+      const float2 e = make_float2(C.mod2pi * sk.x + C.lam2pi * h.x, C.mod2pi * sk.y + C.lam2pi * h.y);
+      acc = make_float2(-e.y - C.grav * u3.x, e.x - C.grav * u3.y);
+    }
+    const float2 tt = gload(A.tbase + d * A.tcs + t);
+    // p = t - p / (sx3 dx3)   (green.f90:373-375, :1082-1084)
+    pv[d][t] = make_float2(tt.x - acc.x / C.inv_n3dx3, tt.y - acc.y / C.inv_n3dx3);
+  }
+  __syncthreads();
+  // one thread per column forms its constants, the others read them
+  if (tid < TX) ccs[tid] = cerruti_column(C, mu, alpha, gamma, k1w, k2w, pv[0][tid], pv[1][tid], pv[2][tid]);
+  __syncthreads();
+  const CerrutiCol& cc = ccs[col];
+  const float2 ca = cc.A[c], cb = cc.B[c];
+  const float beta = cc.beta, beta2 = cc.beta2;
+  const bool corr = !cc.zero;
+  // the Cerruti correction of this component, then B^-1 into the buffer
+  auto inverse = [&](bool odd, float2* X) {
+    if (corr) {
+#pragma unroll
+      for (int k2 = 0; k2 < Q; ++k2) {
+        const float tk3 = (float)RELAX_PI2 * wave3(k2, odd);
+        const float fi = 2.f * beta * __builtin_amdgcn_rcpf(tk3 * tk3 + beta2);
+        const float fk = fi * (tk3 * fi);
+        X[k2] = make_float2(X[k2].x + (fi * ca.x + fk * cb.x), X[k2].y + (fi * ca.y + fk * cb.y));
+      }
+    }
+    dft16<+1>(X);
+    brow[0] = X[0];
+#pragma unroll
+    for (int j = 1; j < Q; ++j) brow[j * RS] = cmul(X[j], cconj(tws[16 * j + r]));
+    __syncthreads();
+    float2* y = odd ? X : x;
+#pragma unroll
+    for (int k1 = 0; k1 < 16; ++k1) y[k1] = arow[k1 * TX];
+    dft16<+1>(y);
+  };
+  inverse(false, X0);  // x = E'
+  __syncthreads();
+  inverse(true, X1);   // X1 = O'
+  typedef unsigned u2v __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int m = 0; m < 16; ++m) {
+    const float2 ow = cmul(X1[m], cconj(stw[Q * m + r]));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, cadd(x[m], ow)), rs, voff, m * zstep, 0);
+  }
+}
+
 template <int HH>
 static int green_reg_launch(const GreenConst& gc, const ColumnConsts& C, double alpha, MPtr<float2> W,
                             MPtr<float2> NQ, MPtr<const float2> TM, MPtr<const float2> TN, int nm,
                             const float2* tw3, int l2, hipStream_t st) {
-  constexpr int TX = 16;
+  constexpr int TX = HH == 256 ? DEEP_TX : 16;
   const int m1 = gc.n1 / 2;
-  if (HH < 32 || HH > 128 || m1 % TX || gc.n2 % TX) return RELAX_ERR_SIZE;
+  if (HH < 32 || m1 % TX || gc.n2 % TX) return RELAX_ERR_SIZE;
   const int nb = (m1 / TX) * gc.n2 + gc.n2 / TX;
-  k_green_reg<(HH < 32 ? 32 : HH > 128 ? 128 : HH), false><<<dim3(nb, nm), 512, 0, st>>>(
-      C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, gc.n3, W, NQ, TM, TN, tw3, l2, FullGreen{});
+  if constexpr (HH == 256)
+    k_green_deep<<<dim3(nb, nm), 48 * DEEP_TX, 0, st>>>(C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, W, NQ, TM, TN, tw3, l2);
+  else
+    k_green_reg<(HH < 32 ? 32 : HH), false><<<dim3(nb, nm), 512, 0, st>>>(
+        C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, gc.n3, W, NQ, TM, TN, tw3, l2, FullGreen{});
   return RELAX_OK;
 }
 

@@ -312,12 +312,12 @@ static void tune_lookup(relax_model_t* m) {
 //    210).
 //  - Green column pass: the register form from 64-deep columns up (64x64x128:
 //    11.0 against 16.0, 256x256x128: 51.6 against 65.1, 512x512x256: 264
-//    against 419; it has no 256-deep form); 32-deep columns radix 8 (512x512x64:
-//    87.8 against 94.9, the register form 128).  The forms round differently,
-//    and the slip of a creeping patch near the clamp of its friction law
-//    follows that rounding (5e-5 of the slip after 20 steps at 256x256x128):
-//    models with creeping planes keep the radix-16 LDS form, in a batch too
-//    (green_launches).
+//    against 419, 512x512x512: 800 against 1112); 32-deep columns radix 8
+//    (512x512x64: 87.8 against 94.9, the register form 128).  The forms round
+//    differently, and the slip of a creeping patch near the clamp of its
+//    friction law follows that rounding (5e-5 of the slip after 20 steps at
+//    256x256x128): models with creeping planes keep the radix-16 LDS form, in a
+//    batch too (green_launches).
 //  - divergence: the register-window tiles wherever 64 divides n1, 64x8 on
 //    grids under 128^3 (64x64x64: 7.6 against 9.1 for 64x16 and 31 for the
 //    32x8 ring), else 64x16 (512x512x256: 247 against 268, ring 303).  The
@@ -327,7 +327,7 @@ static void tune_lookup(relax_model_t* m) {
 static void default_shapes(const Grid& g, int rclass, int* cols, int* green, int* body) {
   const long n = 2 * g.H;
   if (*cols < 0) *cols = g.n2 != 128 && g.n2 != 1024 && n <= (1L << 25) ? 1 : 0;
-  if (*green < 0) *green = g.h3 == 64 || g.h3 == 128 ? 3 : g.h3 == 32 ? 2 : 0;
+  if (*green < 0) *green = g.h3 >= 64 ? 3 : g.h3 == 32 ? 2 : 0;
   if (*body < 0) {
     if (g.n1 % 64) *body = 1;
     else if (rclass & RHEO_EXT) *body = n <= (1L << 22) ? 4 : n <= (1L << 23) ? 2 : 3;

@@ -6,8 +6,8 @@ import numpy as np
 import pytest
 
 import oracle as O
-from _cases import rel_l2
-from relax_amd import green
+from _cases import rel_l2, small_spec
+from relax_amd import green, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -28,3 +28,24 @@ def test_full_depth_solve(n):
     green.greenfunctioncowling(*c, *t, 0.9, 1.1, 0.7, LAM, MU, GAM)
     for a, b in zip(c, ref):
         assert rel_l2(a[..., :n1], b[..., :n1]) < 4e-6
+
+
+@pytest.mark.parametrize("n", [(32, 32, 512), (64, 128, 512), (128, 32, 512)])
+def test_deep_half_columns_match_the_lds_form(n):
+    """The register form of 256-deep half columns (with the Nyquist columns,
+    the split and the unsplit y order) against the form that keeps them in
+    LDS: FP32 rounding of the same transforms, 1e-5 after three steps as for
+    the other depths."""
+    s = small_spec("powerlaw")
+    s.update(sx1=n[0], sx2=n[1], sx3=n[2])
+    out = {}
+    for v in (0, 3):
+        with workloads.build(s) as m:
+            m.set_tuning(green=v)
+            for _ in range(3):
+                m.step(info=False)
+            out[v] = m.download()
+    for k in ("u1", "u2", "u3"):
+        assert rel_l2(out[3][k][..., :n[0]], out[0][k][..., :n[0]]) < 1e-5, k
+    for k in ("sig", "tau"):
+        assert rel_l2(out[3][k], out[0][k]) < 1e-5, k
