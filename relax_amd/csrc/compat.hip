@@ -604,7 +604,8 @@ int relax_cerrutimodified(const float* p1, const float* p2, const float* p3, dou
 // other (the second finds part of the field in the on-package cache); the
 // traction planes go three to a launch.
 int green_full_device(float* const v[3], float* const t[3], int sx1, int sx2, int sx3, double dx1, double dx2,
-                      double dx3, double lambda, double mu, double gamma, hipStream_t st, bool sync) {
+                      double dx3, double lambda, double mu, double gamma, hipStream_t st, bool sync, float* top,
+                      long H) {
   int rc;
   const GreenConst gc = green_const(sx1, sx2, sx3, dx1, dx2, dx3, lambda, mu, gamma);
   float2* vc[3] = {(float2*)v[0], (float2*)v[1], (float2*)v[2]};
@@ -624,8 +625,18 @@ int green_full_device(float* const v[3], float* const t[3], int sx1, int sx2, in
                              (float)(dx1 * dx2), 3, st)) ||
       (rc = launch_fft_cols(sx2, -1, tm, P, (long)sx2 * P, M + 1, 1, 3, st)))
     return rc;
-  if ((rc = launch_green_full(gc, vc, tc, st))) return rc;
+  if ((rc = launch_green_full(gc, vc, tc, st, top != nullptr))) return rc;
   const double sc = 1.0 / (sx1 * dx1 * sx2 * dx2 * sx3 * dx3), sc2 = 1.0 / (sx1 * dx1 * sx2 * dx2);
+  // a model's event: the upper half alone, added to u by the x transform, and
+  // no tractions (256x256x128: the y and x transforms back 103 -> 79 us, and 50
+  // us less for the sum and the tractions)
+  for (int k = 0; top && k < 3; ++k) {
+    if ((rc = launch_fft_cols(sx2, +1, mptr(vc[k]), P, (long)sx2 * P, M + 1, sx3 / 2, 1, st, cv)) ||
+        (rc = launch_fft_x_c2r(sx1, EPI_ADD, vc[k], P, vc[k] + M, P, top + k * H, sx1, (long)sx2 * (sx3 / 2), (float)sc,
+                               top + k * H, sx1, nullptr, st)))
+      return rc;
+  }
+  if (top) return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
   for (int k = 0; k < 3; ++k) {
     if ((rc = launch_fft_cols(sx2, +1, mptr(vc[k]), P, (long)sx2 * P, M + 1, sx3, 1, st, cv)) ||
         (rc = launch_fft_x_c2r(sx1, EPI_PLAIN, vc[k], P, vc[k] + M, P, v[k], sx1 + 2, (long)sx2 * sx3, (float)sc, nullptr,
@@ -840,7 +851,7 @@ int relax_source(double mu, double slip, double x, double y, double z, double L,
   HIP_TRY(hipMemcpy(pl.p, &P, sizeof(PlaneDev), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(sl.p, &slip, sizeof(double), hipMemcpyHostToDevice));
   if ((rc = launch_source((const PlaneDev*)pl.p, (const double*)sl.p, 1, mu, sx1, sx2, sx3 / 2, dx1, dx2, dx3,
-                          f.f(), ld, fs, t.f(), ts, 0)))
+                          field3(f.f(), fs), ld, t.f(), ts, 0)))
     return rc;
   if ((rc = sync_status(RELAX_OK))) return rc;
   for (int c = 0; c < 3; ++c) {
@@ -866,7 +877,7 @@ int relax_tensilesource(double lambda, double mu, double s, double x, double y, 
   HIP_TRY(hipMemcpy(pl.p, &P, sizeof(PlaneDev), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(op.p, &s, sizeof(double), hipMemcpyHostToDevice));
   if ((rc = launch_tensile_source((const PlaneDev*)pl.p, (const double*)op.p, 1, lambda, mu, sx1, sx2, sx3, dx1, dx2,
-                                  dx3, f.f(), ld, fs, 0)))
+                                  dx3, field3(f.f(), fs), ld, 0)))
     return rc;
   if ((rc = sync_status(RELAX_OK))) return rc;
   for (int c = 0; c < 3; ++c) HIP_TRY(hipMemcpy(fh[c], f.f() + c * fs, fs * 4, hipMemcpyDeviceToHost));
@@ -886,8 +897,8 @@ int relax_mogisource(double lambda, double mu, double o, double xs, double ys, d
   relax_source_t M{};
   M.slip = o; M.x = xs; M.y = ys; M.z = zs;
   HIP_TRY(hipMemcpy(ms.p, &M, sizeof(M), hipMemcpyHostToDevice));
-  if ((rc = launch_mogi_source((const relax_source_t*)ms.p, 1, lambda, mu, sx1, sx2, sx3, dx1, dx2, dx3, f.f(), ld,
-                               fs, 0)))
+  if ((rc = launch_mogi_source((const relax_source_t*)ms.p, 1, lambda, mu, sx1, sx2, sx3, dx1, dx2, dx3,
+                               field3(f.f(), fs), ld, 0)))
     return rc;
   if ((rc = sync_status(RELAX_OK))) return rc;
   for (int c = 0; c < 3; ++c) HIP_TRY(hipMemcpy(fh[c], f.f() + c * fs, fs * 4, hipMemcpyDeviceToHost));

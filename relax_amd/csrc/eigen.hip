@@ -132,8 +132,7 @@ __device__ __forceinline__ void tetra_dist(const TetraDev& T, double x1, double 
 
 __global__ __launch_bounds__(256) void k_eigen_source(const CuboidDev* __restrict__ C, int nc,
                                                       const TetraDev* __restrict__ T, int nt, int n1, int n2, int h3,
-                                                      double dx1, double dx2, double dx3, float* f, long ld,
-                                                      long fs) {
+                                                      double dx1, double dx2, double dx3, Field3 f, long ld) {
   const long o = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (o >= (long)n1 * n2 * h3) return;
   const int i1 = o % n1, i2 = (o / n1) % n2, i3 = o / ((long)n1 * n2);
@@ -144,7 +143,7 @@ __global__ __launch_bounds__(256) void k_eigen_source(const CuboidDev* __restric
   for (int k = 0; k < nc; ++k) {
     const CuboidDev& c = C[k];
     if ((fabs(x1 - c.x) > c.lim) || (fabs(x2 - c.y) > c.lim) || (fabs(x3 - c.z) > c.lim)) continue;
-    if (!any) { f1 = f[of]; f2 = f[fs + of]; f3 = f[2 * fs + of]; any = true; }
+    if (!any) { f1 = f.c[0][of]; f2 = f.c[1][of]; f3 = f.c[2][of]; any = true; }
     const double cs = c.cs, ss = c.ss, cd = c.cd, sd = c.sd, b = c.beta;
     const double x2r = cs * x1 - ss * x2;
     const double x1s = cd * x2r - sd * x3, x1i = cd * x2r + sd * x3;
@@ -187,7 +186,7 @@ __global__ __launch_bounds__(256) void k_eigen_source(const CuboidDev* __restric
     if (fabs(dist[0]) > 7.0 * dx1 && fabs(dist[1]) > 7.0 * dx1 && fabs(dist[2]) > 7.0 * dx1 &&
         fabs(dist[3]) > 7.0 * dx1)
       continue;
-    if (!any) { f1 = f[of]; f2 = f[fs + of]; f3 = f[2 * fs + of]; any = true; }
+    if (!any) { f1 = f.c[0][of]; f2 = f.c[1][of]; f3 = f.c[2][of]; any = true; }
     double H[4], dl[4];
     for (int j = 0; j < 4; ++j) {
       H[j] = d_gaussi(dist[j], dx1);
@@ -199,7 +198,7 @@ __global__ __launch_bounds__(256) void k_eigen_source(const CuboidDev* __restric
     f2 = (float)((double)f2 + t.tr[0][1] * w0 + t.tr[1][1] * w1 + t.tr[2][1] * w2 + t.tr[3][1] * w3);
     f3 = (float)((double)f3 + t.tr[0][2] * w0 + t.tr[1][2] * w1 + t.tr[2][2] * w2 + t.tr[3][2] * w3);
   }
-  if (any) { f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3; }
+  if (any) { f.c[0][of] = f1; f.c[1][of] = f2; f.c[2][of] = f3; }
 }
 
 // (q + ekk lambda I) + 2 mu E, rounded after each operation
@@ -305,7 +304,7 @@ int eigen_stage(relax_model_t* m, const relax_event_t* ev) {
   return RELAX_OK;
 }
 
-int eigen_body_force(relax_model_t* m, float* f, long ld, long fs) {
+int eigen_body_force(relax_model_t* m, const Field3& f, long ld) {
   if (m->cur_ncub + m->cur_ntet == 0) return RELAX_OK;
   const Grid& g = m->g;
   const CuboidDev* C = static_cast<const CuboidDev*>(m->eig_dev);
@@ -313,7 +312,7 @@ int eigen_body_force(relax_model_t* m, float* f, long ld, long fs) {
                                                          m->cur_ncub * sizeof(CuboidDev));
   const long N = (long)g.n1 * g.n2 * g.h3;
   k_eigen_source<<<(unsigned)((N + 255) / 256), 256, 0, m->stream>>>(
-      C, m->cur_ncub, T, m->cur_ntet, g.n1, g.n2, g.h3, m->desc.dx1, m->desc.dx2, m->desc.dx3, f, ld, fs);
+      C, m->cur_ncub, T, m->cur_ntet, g.n1, g.n2, g.h3, m->desc.dx1, m->desc.dx2, m->desc.dx3, f, ld);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 

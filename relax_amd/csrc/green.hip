@@ -334,6 +334,7 @@ __global__ __launch_bounds__(NT) void k_green_columns(ColumnConsts C, double mu,
 struct FullGreen {
   float2* v[3];
   const float2* t[3];
+  bool upper;  // only the upper half of the result is written
 };
 template <int H3, bool FULL>
 __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu, double alpha, double gamma, int n1,
@@ -574,7 +575,7 @@ __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu,
       const float2 ow = cmul(o[m], cconj(stw[Q * m + aj]));
       const float2 v = cadd(x[m], ow);
       if (vstore) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, v), rs, voff, m * zstep, 0);
-      if (FULL && vstore)
+      if (FULL && vstore && !F.upper)
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, csub(x[m], ow)), rs, voff, zhalf + m * zstep, 0);
     }
   }
@@ -845,7 +846,7 @@ template <int N3>
 __global__ __launch_bounds__(FullTile<N3>::NT) void k_green_full(ColumnConsts C, double mu, double alpha, double gamma,
                                                                  int n1, int n2, float2* v1, float2* v2, float2* v3,
                                                                  const float2* t1, const float2* t2, const float2* t3,
-                                                                 const float2* __restrict__ tw3) {
+                                                                 const float2* __restrict__ tw3, int nz) {
   constexpr int TX = FullTile<N3>::TX, NT = FullTile<N3>::NT, NW = NT / 64;
   static_assert(64 % TX == 0, "a thread keeps one column");
   constexpr int SB = N3 * TX + 12;  // padded as in k_green_columns
@@ -916,11 +917,11 @@ __global__ __launch_bounds__(FullTile<N3>::NT) void k_green_full(ColumnConsts C,
   lds_fft<N3, 3 * TX, NT, TX, 1, SB, TX, +1, 1, true, 16>(s, stw, tid);
 #pragma unroll
   for (int c = 0; c < 3; ++c)
-    for (int z = tid / TX; z < N3; z += NT / TX)
+    for (int z = tid / TX; z < nz; z += NT / TX)
       if (own) gstore(v[c] + row + z * zs + tx, s[c * SB + z * TX + tx]);
 }
 
-int launch_green_full(const GreenConst& gc, float2* const v[3], const float2* const t[3], hipStream_t st) {
+int launch_green_full(const GreenConst& gc, float2* const v[3], const float2* const t[3], hipStream_t st, bool upper) {
   const float2* tw3 = twiddle_table(gc.n3);
   if (!tw3) return RELAX_ERR_NOMEM;
   const ColumnConsts C = make_consts(gc);
@@ -930,14 +931,14 @@ int launch_green_full(const GreenConst& gc, float2* const v[3], const float2* co
   case N: {                                                                                                   \
     const unsigned nb = (unsigned)((h1 + FullTile<N>::TX - 1) / FullTile<N>::TX) * (unsigned)gc.n2;           \
     k_green_full<N><<<nb, FullTile<N>::NT, 0, st>>>(C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, v[0], v[1], v[2], \
-                                                   t[0], t[1], t[2], tw3);                                    \
+                                                   t[0], t[1], t[2], tw3, upper ? N / 2 : N);                                 \
     break;                                                                                                    \
   }
 #define R(N)                                                                                                  \
   case N: {                                                                                                   \
     const unsigned nb = (unsigned)((h1 + 15) / 16) * (unsigned)gc.n2;                                         \
     k_green_reg<N / 2, true><<<nb, 512, 0, st>>>(C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, gc.n3, {}, {}, {}, {}, \
-                                                tw3, 0, FullGreen{{v[0], v[1], v[2]}, {t[0], t[1], t[2]}});   \
+                                                tw3, 0, FullGreen{{v[0], v[1], v[2]}, {t[0], t[1], t[2]}, upper});   \
     break;                                                                                                    \
   }
   switch (gc.n3) {

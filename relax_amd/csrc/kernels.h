@@ -88,8 +88,9 @@ struct GreenConst {
 int launch_green_columns(const GreenConst& gc, int h3, MPtr<float2> W, MPtr<float2> NQ, MPtr<const float2> TM,
                          MPtr<const float2> TN, int nm, hipStream_t st, int l2 = 0, int variant = 0);
 // the same over the full depth, on padded spectra (rows of n1/2+1 complex): v
-// transformed along x1 and x2, t the spectra of the traction planes
-int launch_green_full(const GreenConst& gc, float2* const v[3], const float2* const t[3], hipStream_t st);
+// transformed along x1 and x2, t the spectra of the traction planes; upper:
+// only the upper half of the result is written
+int launch_green_full(const GreenConst& gc, float2* const v[3], const float2* const t[3], hipStream_t st, bool upper);
 // per-routine kernels on padded full spectra (row pitch n1/2+1 complex)
 int launch_elastic_padded(const GreenConst& gc, float2* f1, float2* f2, float2* f3, hipStream_t st);
 int launch_surface_padded(const GreenConst& gc, const float2* u1, const float2* u2, const float2* u3, float2* p1,
@@ -97,13 +98,19 @@ int launch_surface_padded(const GreenConst& gc, const float2* u1, const float2* 
 int launch_cerruti_padded(const GreenConst& gc, const float2* p1, const float2* p2, const float2* p3,
                           float2* u1, float2* u2, float2* u3, hipStream_t st);
 
+// The three components of a vector field (rows of one pitch)
+struct Field3 {
+  float* c[3];
+};
+inline Field3 field3(float* f, long fs) { return Field3{{f, f + fs, f + 2 * fs}}; }
+
 // model.hip: the body force of source() (elastic3d.f90:2064-2252) of the
 // np planes P (slips slip) added to the top half of f (3 planes of
 // n1*n2*h3, packed rows of ld floats, plane stride fs) and their surface
 // traction to t (3 planes of n1*n2, row stride ld, plane stride ts).
 struct PlaneDev;
 int launch_source(const PlaneDev* P, const double* slip, int np, double mu, int n1, int n2, int h3, double dx1,
-                  double dx2, double dx3, float* f, long ld, long fs, float* t, long ts, hipStream_t st);
+                  double dx2, double dx3, Field3 f, long ld, float* t, long ts, hipStream_t st);
 
 // model.hip: traction() of the surface loads l subtracted from t3 (n1*n2,
 // row stride ld) at time t, or their rate over [t, t+Dt] when rate != 0
@@ -112,9 +119,12 @@ int launch_traction(const relax_source_t* l, int nl, int n1, int n2, double dx1,
 
 // compat.hip: greenfunctioncowling over the full depth on device buffers in
 // the padded layout (v: fields of (sx1+2) sx2 sx3, t: planes of
-// (sx1+2) sx2), enqueued on stream st (and waited for with sync)
+// (sx1+2) sx2), enqueued on stream st (and waited for with sync).  With top,
+// a model's u (three planes of H, packed rows): the upper half of the solution
+// is added to it and v and t are left as scratch.
 int green_full_device(float* const v[3], float* const t[3], int sx1, int sx2, int sx3, double dx1, double dx2,
-                      double dx3, double lambda, double mu, double gamma, hipStream_t st, bool sync);
+                      double dx3, double lambda, double mu, double gamma, hipStream_t st, bool sync, float* top = nullptr,
+                      long H = 0);
 
 // model.hip: tensilesource (elastic3d.f90:2315-2411) and mogisource
 // (:2458-2509) of np cracks / point sources into f (3 fields of n1 n2 n3
@@ -122,9 +132,9 @@ int green_full_device(float* const v[3], float* const t[3], int sx1, int sx2, in
 // moment densities (:3137-3215, :3240-3286) into a tensor field of the
 // top half (6 planes of H)
 int launch_tensile_source(const PlaneDev* P, const double* opening, int np, double lambda, double mu, int n1, int n2,
-                          int n3, double dx1, double dx2, double dx3, float* f, long ld, long fs, hipStream_t st);
+                          int n3, double dx1, double dx2, double dx3, Field3 f, long ld, hipStream_t st);
 int launch_mogi_source(const relax_source_t* M, int nm, double lambda, double mu, int n1, int n2, int n3,
-                       double dx1, double dx2, double dx3, float* f, long ld, long fs, hipStream_t st);
+                       double dx1, double dx2, double dx3, Field3 f, long ld, hipStream_t st);
 int launch_add_tensile(const PlaneDev* P, const double* opening, int np, double lambda, double mu, int n1, int n2,
                        int h3, double dx1, double dx2, double dx3, float* sig, long H, hipStream_t st);
 int launch_add_mogi(const relax_source_t* M, int nm, double lambda, double mu, int n1, int n2, int h3, double dx1,

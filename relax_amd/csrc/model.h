@@ -98,5 +98,5 @@ int model_stress_set(relax_model_t* m);
 // staged on the device, their body forces added to the top half of f (row
 // stride ld, component stride fs), their moment densities added to tau
 int eigen_stage(relax_model_t* m, const relax_event_t* ev);
-int eigen_body_force(relax_model_t* m, float* f, long ld, long fs);
+int eigen_body_force(relax_model_t* m, const Field3& f, long ld);
 int eigen_moment(relax_model_t* m);

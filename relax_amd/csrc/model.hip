@@ -1533,8 +1533,8 @@ int relax_model_add_shear(relax_model_t* m, const relax_plane_t* patches, const 
 // rounding (two FP32 roundings per plane and component); threads of the top
 // plane also add the surface traction (n sdyad mu s b) e3.
 __global__ __launch_bounds__(256) void k_source(const PlaneDev* __restrict__ P, const double* __restrict__ slip, int np, double mu,
-                         int n1, int n2, int h3, double dx1, double dx2, double dx3, float* f, long ld, long fs,
-                         float* t, long ts) {
+                         int n1, int n2, int h3, double dx1, double dx2, double dx3, Field3 f, long ld, float* t,
+                         long ts) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
     // the surface traction has no gate in depth
@@ -1557,7 +1557,7 @@ __global__ __launch_bounds__(256) void k_source(const PlaneDev* __restrict__ P, 
       const double x1s = cd * xx - sd * x3, x1i = cd * xx + sd * x3;
       if ((fabs(x1s - p.xr) > 7.01 * dx1) && (fabs(x1i - p.xr) > 7.01 * dx1)) continue;
       if (!any) {
-        f1 = f[of]; f2 = f[fs + of]; f3 = f[2 * fs + of];
+        f1 = f.c[0][of]; f2 = f.c[1][of]; f3 = f.c[2][of];
         if (i3 == 0) { t1 = t[ot]; t2 = t[ts + ot]; t3 = t[2 * ts + ot]; }
         any = true;
       }
@@ -1601,16 +1601,15 @@ __global__ __launch_bounds__(256) void k_source(const PlaneDev* __restrict__ P, 
       f3 = (float)((double)f3 + (cd * sr * sourc - sd * sr * dipcs));
     }
     if (!any) return;
-    f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3;
+    f.c[0][of] = f1; f.c[1][of] = f2; f.c[2][of] = f3;
     if (i3 == 0) { t[ot] = t1; t[ts + ot] = t2; t[2 * ts + ot] = t3; }
   });
 }
 
 int launch_source(const PlaneDev* P, const double* slip, int np, double mu, int n1, int n2, int h3, double dx1,
-                  double dx2, double dx3, float* f, long ld, long fs, float* t, long ts, hipStream_t st) {
+                  double dx2, double dx3, Field3 f, long ld, float* t, long ts, hipStream_t st) {
   const long N = (long)n1 * n2 * h3;
-  k_source<<<src_blocks(N), 256, 0, st>>>(P, slip, np, mu, n1, n2, h3, dx1, dx2, dx3, f, ld, fs, t,
-                                                        ts);
+  k_source<<<src_blocks(N), 256, 0, st>>>(P, slip, np, mu, n1, n2, h3, dx1, dx2, dx3, f, ld, t, ts);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 
@@ -1620,7 +1619,7 @@ int launch_source(const PlaneDev* P, const double* slip, int np, double mu, int 
 // order with one rounding each
 __global__ __launch_bounds__(256) void k_tensile_source(const PlaneDev* __restrict__ P, const double* __restrict__ opening, int np,
                                  double lambda, double mu, int n1, int n2, int n3, double dx1, double dx2, double dx3,
-                                 float* f, long ld, long fs) {
+                                 Field3 f, long ld) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
     const PlaneDev& p = P[k];
@@ -1654,20 +1653,20 @@ __global__ __launch_bounds__(256) void k_tensile_source(const PlaneDev* __restri
       const double image = scale1 * d_gaussp(x1i - p.xr, dx1) * t2 * t3;
       const double cplei = scale2 / p.W * t1 * d_omegap((x2s - p.yr) / p.W, p.beta) * t3;
       const double dipci = scale2 / p.L * t1 * t2 * d_omegap((x3i + p.zr) / p.L, p.beta);
-      if (!any) { f1 = f[of]; f2 = f[fs + of]; f3 = f[2 * fs + of]; }
+      if (!any) { f1 = f.c[0][of]; f2 = f.c[1][of]; f3 = f.c[2][of]; }
       f1 = (float)((double)f1 + cs * cd * (sourc + image) + ss * (dblcp + cplei) + cs * sd * (dipcs + dipci));
       f2 = (float)((double)f2 - ss * cd * (sourc + image) + cs * (dblcp + cplei) - ss * sd * (dipcs + dipci));
       f3 = (float)((double)f3 - sd * (sourc - image) + cd * (dipcs - dipci));
       any = true;
     }
-    if (any) { f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3; }
+    if (any) { f.c[0][of] = f1; f.c[1][of] = f2; f.c[2][of] = f3; }
   });
 }
 
 // mogisource, elastic3d.f90:2458-2509: point dilatation sources (volume
 // change in slip) and their images over the full depth
 __global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __restrict__ M, int nm, double lambda, double mu, int n1, int n2,
-                              int n3, double dx1, double dx2, double dx3, float* f, long ld, long fs) {
+                              int n3, double dx1, double dx2, double dx3, Field3 f, long ld) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
     const relax_source_t& s = M[k];
@@ -1695,13 +1694,13 @@ __global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __res
       t3 = d_gauss(x3 + s.z, dx3);
       const double m1 = scale * d_gaussp(x1 - s.x, dx1) * t2 * t3, m2 = scale * t1 * d_gaussp(x2 - s.y, dx2) * t3;
       const double m3 = scale * t1 * t2 * d_gaussp(x3 + s.z, dx3);
-      if (!any) { f1 = f[of]; f2 = f[fs + of]; f3 = f[2 * fs + of]; }
+      if (!any) { f1 = f.c[0][of]; f2 = f.c[1][of]; f3 = f.c[2][of]; }
       f1 = (float)((double)f1 + (s1 + m1));
       f2 = (float)((double)f2 + (s2 + m2));
       f3 = (float)((double)f3 + (s3 - m3));
       any = true;
     }
-    if (any) { f[of] = f1; f[fs + of] = f2; f[2 * fs + of] = f3; }
+    if (any) { f.c[0][of] = f1; f.c[1][of] = f2; f.c[2][of] = f3; }
   });
 }
 
@@ -1785,18 +1784,15 @@ __global__ __launch_bounds__(256) void k_add_mogi(const relax_source_t* __restri
   });
 }
 
-static unsigned blocks_of(long n) { return (unsigned)((n + 255) / 256); }
-
 int launch_tensile_source(const PlaneDev* P, const double* opening, int np, double lambda, double mu, int n1, int n2,
-                          int n3, double dx1, double dx2, double dx3, float* f, long ld, long fs, hipStream_t st) {
+                          int n3, double dx1, double dx2, double dx3, Field3 f, long ld, hipStream_t st) {
   k_tensile_source<<<src_blocks((long)n1 * n2 * n3), 256, 0, st>>>(P, opening, np, lambda, mu, n1, n2, n3, dx1, dx2,
-                                                                  dx3, f, ld, fs);
+                                                                  dx3, f, ld);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 int launch_mogi_source(const relax_source_t* M, int nm, double lambda, double mu, int n1, int n2, int n3,
-                       double dx1, double dx2, double dx3, float* f, long ld, long fs, hipStream_t st) {
-  k_mogi_source<<<src_blocks((long)n1 * n2 * n3), 256, 0, st>>>(M, nm, lambda, mu, n1, n2, n3, dx1, dx2, dx3, f, ld,
-                                                               fs);
+                       double dx1, double dx2, double dx3, Field3 f, long ld, hipStream_t st) {
+  k_mogi_source<<<src_blocks((long)n1 * n2 * n3), 256, 0, st>>>(M, nm, lambda, mu, n1, n2, n3, dx1, dx2, dx3, f, ld);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 int launch_add_tensile(const PlaneDev* P, const double* opening, int np, double lambda, double mu, int n1, int n2,
@@ -1870,17 +1866,6 @@ static PlaneDev source_plane(const relax_source_t& s, double dx1, double dx3) {
   return make_plane(p, s.beta, dx1, dx3);
 }
 
-// u += the top half of a full-depth field in the padded layout
-__global__ void k_add_padded_top(float* __restrict__ u, const float* __restrict__ v, int n1, int n2, int h3, long H,
-                                 long vs) {
-  const long o = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (o >= H) return;
-  const int i1 = o % n1;
-  const long r = o / n1;  // row (i2, i3)
-  const long q = i1 + (long)(n1 + 2) * r;
-  for (int c = 0; c < 3; ++c) u[c * H + o] = u[c * H + o] + v[c * vs + q];
-}
-
 int relax_model_event(relax_model_t* m, const relax_event_t* ev, double nyquist) {
   if (!m || m->batch || !ev || ev->ns < 0 || ev->nt < 0 || ev->nm < 0 || ev->nl < 0 || (ev->ns > 0 && !ev->s) ||
       (ev->nt > 0 && !ev->ts) || (ev->nm > 0 && !ev->m) || (ev->nl > 0 && !ev->l) || ev->nc < 0 || ev->nth < 0 ||
@@ -1945,10 +1930,10 @@ int relax_model_event(relax_model_t* m, const relax_event_t* ev, double nyquist)
     // adding to u (relax.f90:362-371, :877-884)
     HIP_TRY(hipMemsetAsync(m->W, 0, 3 * H * 4, m->stream));
     HIP_TRY(hipMemsetAsync(m->T, 0, 3L * g.n1 * g.n2 * 4, m->stream));
-    if (nbig && (rc = launch_source(m->shear_dev, m->shear_slip, nbig, mu, g.n1, g.n2, g.h3, dx1, dx2, dx3, m->W,
-                                    g.n1, H, m->T, (long)g.n1 * g.n2, m->stream)))
+    if (nbig && (rc = launch_source(m->shear_dev, m->shear_slip, nbig, mu, g.n1, g.n2, g.h3, dx1, dx2, dx3,
+                                    field3(m->W, H), g.n1, m->T, (long)g.n1 * g.n2, m->stream)))
       return rc;
-    if ((rc = eigen_body_force(m, m->W, g.n1, H))) return rc;
+    if ((rc = eigen_body_force(m, field3(m->W, H), g.n1))) return rc;
     if (nl && (rc = launch_traction(m->loads_dev, nl, g.n1, g.n2, dx1, dx2, t, 0.0, 0, m->T + 2L * g.n1 * g.n2, g.n1,
                                     m->stream)))
       return rc;
@@ -1957,36 +1942,32 @@ int relax_model_event(relax_model_t* m, const relax_event_t* ev, double nyquist)
     if ((rc = model_green(c, EPI_ADD))) return rc;
   } else {
     // tensile cracks and point sources put images above the surface, in the
-    // lower half of the grid: the full-depth Green solve on scratch fields
-    // in the padded layout
+    // lower half of the grid: the full-depth Green solve in the padded layout.
+    // It works in sig, which the stress pass below writes anew, and W: two
+    // components take 4H (1 + 2/n1) of sig's 6H floats, the third and the
+    // tractions less than W's 3H from n1, n3 = 32 up.  (Scratch of its own was
+    // allocated and freed by each event: 386 us of 1180 at 256x256x128.)
     const long ld = g.n1 + 2, vs = ld * g.n2 * g.n3, ts = ld * g.n2;
-    float* scratch = nullptr;
-    const size_t bytes = (size_t)(3 * vs + 3 * ts) * 4;
-    HIP_TRY(rx_malloc(&scratch, bytes));
-    float* v[3] = {scratch, scratch + vs, scratch + 2 * vs};
-    float* tr[3] = {scratch + 3 * vs, scratch + 3 * vs + ts, scratch + 3 * vs + 2 * ts};
-    rc = hipMemsetAsync(scratch, 0, bytes, m->stream) == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
-    if (!rc && nbig)
-      rc = launch_source(m->shear_dev, m->shear_slip, nbig, mu, g.n1, g.n2, g.h3, dx1, dx2, dx3, v[0], ld, vs, tr[0],
-                         ts, m->stream);
-    if (!rc) rc = eigen_body_force(m, v[0], ld, vs);
-    if (!rc && ntbig)
-      rc = launch_tensile_source(m->shear_dev + t0, m->shear_slip + t0, ntbig, lam, mu, g.n1, g.n2, g.n3, dx1, dx2,
-                                 dx3, v[0], ld, vs, m->stream);
-    if (!rc && nm)
-      rc = launch_mogi_source(m->loads_dev + nl, nm, lam, mu, g.n1, g.n2, g.n3, dx1, dx2, dx3, v[0], ld, vs,
-                              m->stream);
-    if (!rc && nl)
-      rc = launch_traction(m->loads_dev, nl, g.n1, g.n2, dx1, dx2, t, 0.0, 0, tr[2], ld, m->stream);
-    if (!rc && hipStreamSynchronize(m->stream) != hipSuccess) rc = RELAX_ERR_HIP;
-    if (!rc) rc = green_full_device(v, tr, g.n1, g.n2, g.n3, dx1, dx2, dx3, lam, mu, m->desc.gamma, m->stream, true);
-    if (!rc) {
-      k_add_padded_top<<<blocks_of(H), 256, 0, m->stream>>>(m->u, scratch, g.n1, g.n2, g.h3, H, vs);
-      if (hipGetLastError() != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess) rc = RELAX_ERR_HIP;
-    }
-    (void)hipStreamSynchronize(m->stream);
-    (void)rx_free(scratch);
-    if (rc) return rc;
+    if (2 * vs > 6 * H || vs + 3 * ts > 3 * H) return RELAX_ERR_SIZE;
+    float* v[3] = {m->sig, m->sig + vs, m->W};
+    float* tr[3] = {m->W + vs, m->W + vs + ts, m->W + vs + 2 * ts};
+    const Field3 f{{v[0], v[1], v[2]}};
+    HIP_TRY(hipMemsetAsync(m->sig, 0, 2 * vs * 4, m->stream));
+    HIP_TRY(hipMemsetAsync(m->W, 0, (vs + 3 * ts) * 4, m->stream));
+    if (nbig && (rc = launch_source(m->shear_dev, m->shear_slip, nbig, mu, g.n1, g.n2, g.h3, dx1, dx2, dx3, f, ld, tr[0],
+                                    ts, m->stream)))
+      return rc;
+    if ((rc = eigen_body_force(m, f, ld))) return rc;
+    if (ntbig && (rc = launch_tensile_source(m->shear_dev + t0, m->shear_slip + t0, ntbig, lam, mu, g.n1, g.n2, g.n3,
+                                             dx1, dx2, dx3, f, ld, m->stream)))
+      return rc;
+    if (nm && (rc = launch_mogi_source(m->loads_dev + nl, nm, lam, mu, g.n1, g.n2, g.n3, dx1, dx2, dx3, f, ld, m->stream)))
+      return rc;
+    if (nl && (rc = launch_traction(m->loads_dev, nl, g.n1, g.n2, dx1, dx2, t, 0.0, 0, tr[2], ld, m->stream)))
+      return rc;
+    if ((rc = green_full_device(v, tr, g.n1, g.n2, g.n3, dx1, dx2, dx3, lam, mu, m->desc.gamma, m->stream, false, m->u,
+                                H)))
+      return rc;
   }
   // the moment densities of every source into tau, then
   // sig = -tau + C:eps(u) (relax.f90:887-889)

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from _cases import rel_l2, small_spec
+from _cases import oracle_initial_state, rel_l2, small_spec
 from relax_amd import green, workloads
 
 pytestmark = pytest.mark.gpu
@@ -49,3 +49,23 @@ def test_deep_half_columns_match_the_lds_form(n):
         assert rel_l2(out[3][k][..., :n[0]], out[0][k][..., :n[0]]) < 1e-5, k
     for k in ("sig", "tau"):
         assert rel_l2(out[3][k], out[0][k]) < 1e-5, k
+
+
+@pytest.mark.parametrize("n", [(32, 32, 32), (64, 32, 64), (32, 32, 128), (32, 64, 256), (32, 32, 512)])
+def test_cracks_and_point_sources_add_their_upper_half(n):
+    """An event with images above the surface solves over the full depth and
+    adds the upper half to u, at every depth of the column kernels; the second
+    event of the same sources doubles u.  u as for the full-depth solve (4e-6)
+    with two roundings of the sum; tau and sig as the set-up's."""
+    s = small_spec("powerlaw")
+    s.update(sx1=n[0], sx2=n[1], sx3=n[2], tensile=[(1.5e-3, -6.0, 4.0, 1.0, 6.0, 4.0, 30.0, 70.0)],
+             mogi=[(4e-3, 8.0, -6.0, 4.0), (-2e-3, -9.0, -9.0, 1.5)])
+    st = oracle_initial_state(s)
+    with workloads.build(s) as m:
+        one = m.download()
+        m.event(nyquist=workloads.NYQUIST, **workloads.event_sources(s, 1))
+        two = m.download()
+    for k in ("u1", "u2", "u3"):
+        assert rel_l2(one[k][..., :n[0]], st[k][..., :n[0]]) < 5e-6, k
+        assert rel_l2(two[k][..., :n[0]], 2 * st[k][..., :n[0]]) < 5e-6, k
+    assert rel_l2(one["tau"], st["tau"]) < 1e-6 and rel_l2(one["sig"], st["sig"]) < 1e-5
