@@ -459,7 +459,8 @@ int relax_batch_scalars(relax_batch_t* b, relax_step_info_t* infos);
  * launch over all current members (their scratch buffers), so the choice
  * fits the batch's size; the batch keeps it, and later batches of the same
  * device, grid and rheology class in the process start from it.  A batch
- * without a choice launches with its first member's shapes.  Members equal
+ * without a choice launches with its first member's shapes (its grid's and
+ * rheology class's defaults when untuned).  Members equal
  * their single runs bitwise when those use the same shapes.  RELAX_ERR_ARG
  * for a batch of several grid classes: tune each class as a batch of its
  * own, and a mixed batch takes those choices per class.  No counterpart in

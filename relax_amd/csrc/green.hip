@@ -768,17 +768,18 @@ static int green_reg_launch(const GreenConst& gc, const ColumnConsts& C, double 
   if (HH < 32 || m1 % TX || gc.n2 % TX) return RELAX_ERR_SIZE;
   const int nb = (m1 / TX) * gc.n2 + gc.n2 / TX;
   if constexpr (HH == 256)
-    k_green_deep<<<dim3(nb, nm), 48 * DEEP_TX, 0, st>>>(C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, W, NQ, TM, TN, tw3, l2);
+    k_green_deep<<<dim3(nb, nm), 48 * DEEP_TX, 0, st>>>(C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, W, NQ, TM, TN, tw3,
+                                                        l2);
   else
     k_green_reg<(HH < 32 ? 32 : HH), false><<<dim3(nb, nm), 512, 0, st>>>(
         C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, gc.n3, W, NQ, TM, TN, tw3, l2, FullGreen{});
   return RELAX_OK;
 }
 
-// Launch shapes of the column pass: columns per workgroup, threads, largest
-// radix.  Variant 0 is the default (measured at 512x512x256: 4 columns of
-// 128 with 256 threads and radix 16 is 4 % faster than 8 columns with 512
-// threads, 25 % faster than radix 8); the autotuner may pick another.
+// Launch shapes of the LDS column pass: columns per workgroup, threads, largest
+// radix.  Variant 0 is the fastest of them at 512x512x256 (4 columns of 128
+// with 256 threads and radix 16 is 4 % faster than 8 columns with 512 threads,
+// 25 % faster than radix 8); variant 3 is the register form.
 template <int H3, int V>
 struct GreenVariant {
   static constexpr int TX0 = H3 >= 128 ? 4 : 16;
@@ -931,7 +932,7 @@ int launch_green_full(const GreenConst& gc, float2* const v[3], const float2* co
   case N: {                                                                                                   \
     const unsigned nb = (unsigned)((h1 + FullTile<N>::TX - 1) / FullTile<N>::TX) * (unsigned)gc.n2;           \
     k_green_full<N><<<nb, FullTile<N>::NT, 0, st>>>(C, gc.mu, alpha, gc.gamma, gc.n1, gc.n2, v[0], v[1], v[2], \
-                                                   t[0], t[1], t[2], tw3, upper ? N / 2 : N);                                 \
+                                                   t[0], t[1], t[2], tw3, upper ? N / 2 : N);            \
     break;                                                                                                    \
   }
 #define R(N)                                                                                                  \

@@ -1528,19 +1528,20 @@ int relax_model_add_shear(relax_model_t* m, const relax_plane_t* patches, const 
   return rc;
 }
 
-// source, elastic3d.f90:2064-2252: one thread per point of the top half,
-// the planes' contributions added in their order with the reference's
+// source, elastic3d.f90:2064-2252: the points of the top half, the
+// planes' contributions added in their order with the reference's
 // rounding (two FP32 roundings per plane and component); threads of the top
 // plane also add the surface traction (n sdyad mu s b) e3.
-__global__ __launch_bounds__(256) void k_source(const PlaneDev* __restrict__ P, const double* __restrict__ slip, int np, double mu,
-                         int n1, int n2, int h3, double dx1, double dx2, double dx3, Field3 f, long ld, float* t,
-                         long ts) {
+__global__ __launch_bounds__(256) void k_source(const PlaneDev* __restrict__ P, const double* __restrict__ slip, int np,
+                                                double mu, int n1, int n2, int h3, double dx1, double dx2, double dx3,
+                                                Field3 f, long ld, float* t, long ts) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
     // the surface traction has no gate in depth
     const PlaneDev& p = P[k];
     return SrcHit{src_reach(B.ya, B.yb, p.y, fmax(p.Lp, p.Wp)) &&
-           (B.top || src_reach(B.za, B.zb, p.z, p.Lp) || src_reach(B.za, B.zb, -p.z, p.Lp)), p.x, fmax(p.Lp, p.Wp)};
+                      (B.top || src_reach(B.za, B.zb, p.z, p.Lp) || src_reach(B.za, B.zb, -p.z, p.Lp)),
+                  p.x, fmax(p.Lp, p.Wp)};
   };
   src_points(sh, np, n1, n2, h3, dx1, dx2, dx3, false, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
     const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
@@ -1617,14 +1618,16 @@ int launch_source(const PlaneDev* P, const double* slip, int np, double mu, int 
 // depth (x3 from the shifted coordinates, so that the images above the
 // surface land in the lower half of the grid), the cracks added in their
 // order with one rounding each
-__global__ __launch_bounds__(256) void k_tensile_source(const PlaneDev* __restrict__ P, const double* __restrict__ opening, int np,
-                                 double lambda, double mu, int n1, int n2, int n3, double dx1, double dx2, double dx3,
-                                 Field3 f, long ld) {
+__global__ __launch_bounds__(256) void k_tensile_source(const PlaneDev* __restrict__ P,
+                                                        const double* __restrict__ opening, int np, double lambda,
+                                                        double mu, int n1, int n2, int n3, double dx1, double dx2,
+                                                        double dx3, Field3 f, long ld) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
     const PlaneDev& p = P[k];
     return SrcHit{src_reach(B.ya, B.yb, p.y, p.Wp) &&
-           (src_reach(B.za, B.zb, p.z, p.Lp) || src_reach(B.za, B.zb, -p.z, p.Lp)), p.x, p.Wp};
+                      (src_reach(B.za, B.zb, p.z, p.Lp) || src_reach(B.za, B.zb, -p.z, p.Lp)),
+                  p.x, p.Wp};
   };
   src_points(sh, np, n1, n2, n3, dx1, dx2, dx3, true, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
     const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = d_shifted(i3, n3, dx3);
@@ -1665,13 +1668,16 @@ __global__ __launch_bounds__(256) void k_tensile_source(const PlaneDev* __restri
 
 // mogisource, elastic3d.f90:2458-2509: point dilatation sources (volume
 // change in slip) and their images over the full depth
-__global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __restrict__ M, int nm, double lambda, double mu, int n1, int n2,
-                              int n3, double dx1, double dx2, double dx3, Field3 f, long ld) {
+__global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __restrict__ M, int nm, double lambda,
+                                                     double mu, int n1, int n2, int n3, double dx1, double dx2,
+                                                     double dx3, Field3 f, long ld) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
     const relax_source_t& s = M[k];
     const double r = 6.0 * fmax(dx1, fmax(dx2, dx3));
-    return SrcHit{src_reach(B.ya, B.yb, s.y, r) && (src_reach(B.za, B.zb, s.z, r) || src_reach(B.za, B.zb, -s.z, r)), s.x, r};
+    return SrcHit{src_reach(B.ya, B.yb, s.y, r) &&
+                      (src_reach(B.za, B.zb, s.z, r) || src_reach(B.za, B.zb, -s.z, r)),
+                  s.x, r};
   };
   src_points(sh, nm, n1, n2, n3, dx1, dx2, dx3, true, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
     // a source at the surface and its image cancel exactly in f3
@@ -1706,9 +1712,10 @@ __global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __res
 
 // momentdensitytensile, elastic3d.f90:3137-3215: Hooke's law of
 // n sdyad (opening n), n carrying the aperture; each crack adds in turn
-__global__ __launch_bounds__(256) void k_add_tensile(const PlaneDev* __restrict__ P, const double* __restrict__ opening, int np,
-                              double lambda, double mu, int n1, int n2, int h3, double dx1, double dx2, double dx3,
-                              float* sig, long H) {
+__global__ __launch_bounds__(256) void k_add_tensile(const PlaneDev* __restrict__ P,
+                                                     const double* __restrict__ opening, int np, double lambda,
+                                                     double mu, int n1, int n2, int h3, double dx1, double dx2,
+                                                     double dx3, float* sig, long H) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
     const PlaneDev& p = P[k];
@@ -1754,8 +1761,9 @@ __global__ __launch_bounds__(256) void k_add_tensile(const PlaneDev* __restrict_
 }
 
 // momentdensitymogi, elastic3d.f90:3240-3286: kappa o G on the diagonal
-__global__ __launch_bounds__(256) void k_add_mogi(const relax_source_t* __restrict__ M, int nm, double lambda, double mu, int n1, int n2,
-                           int h3, double dx1, double dx2, double dx3, float* sig, long H) {
+__global__ __launch_bounds__(256) void k_add_mogi(const relax_source_t* __restrict__ M, int nm, double lambda, double mu,
+                                                  int n1, int n2, int h3, double dx1, double dx2, double dx3,
+                                                  float* sig, long H) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
     const relax_source_t& s = M[k];
@@ -1954,14 +1962,15 @@ int relax_model_event(relax_model_t* m, const relax_event_t* ev, double nyquist)
     const Field3 f{{v[0], v[1], v[2]}};
     HIP_TRY(hipMemsetAsync(m->sig, 0, 2 * vs * 4, m->stream));
     HIP_TRY(hipMemsetAsync(m->W, 0, (vs + 3 * ts) * 4, m->stream));
-    if (nbig && (rc = launch_source(m->shear_dev, m->shear_slip, nbig, mu, g.n1, g.n2, g.h3, dx1, dx2, dx3, f, ld, tr[0],
-                                    ts, m->stream)))
+    if (nbig && (rc = launch_source(m->shear_dev, m->shear_slip, nbig, mu, g.n1, g.n2, g.h3, dx1, dx2, dx3, f, ld,
+                                    tr[0], ts, m->stream)))
       return rc;
     if ((rc = eigen_body_force(m, f, ld))) return rc;
     if (ntbig && (rc = launch_tensile_source(m->shear_dev + t0, m->shear_slip + t0, ntbig, lam, mu, g.n1, g.n2, g.n3,
                                              dx1, dx2, dx3, f, ld, m->stream)))
       return rc;
-    if (nm && (rc = launch_mogi_source(m->loads_dev + nl, nm, lam, mu, g.n1, g.n2, g.n3, dx1, dx2, dx3, f, ld, m->stream)))
+    if (nm && (rc = launch_mogi_source(m->loads_dev + nl, nm, lam, mu, g.n1, g.n2, g.n3, dx1, dx2, dx3, f, ld,
+                                       m->stream)))
       return rc;
     if (nl && (rc = launch_traction(m->loads_dev, nl, g.n1, g.n2, dx1, dx2, t, 0.0, 0, tr[2], ld, m->stream)))
       return rc;
