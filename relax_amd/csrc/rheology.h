@@ -160,9 +160,13 @@ __device__ __forceinline__ float friction_point(const RheoParams& R, const Plane
   if (ratio > 20) { *status = RELAX_ERR_FRICTION; return __builtin_inff(); }
   const double it = 1.0 / taus;
   ts0 *= it; ts1 *= it; ts2 *= it;
-  // sinh(x) = (e + e/(e+1))/2 with e = exp(x) - 1, clamped as my_sinh
-  const double e = expm1(fmin(ratio, 11.0));
-  const double gd = R.fr.v0[i3] * (e + e / (e + 1.0));
+  // d_my_sinh of either sign: sinh(x) = (e + e/(e+1))/2 with e = exp(x) - 1 on
+  // |x| <= 11 (for x < 0 the quotient would cancel), the sign of the ratio (a
+  // negative (a-b) sigma); a NaN ratio (0/0) passes the clamp as it does there
+  double x = fabs(ratio);
+  if (x > 11.0) x = 11.0;
+  const double e = expm1(x);
+  const double gd = R.fr.v0[i3] * copysign(e + e / (e + 1.0), ratio);
   float cand = (float)(tau * P.minlw / ((double)R.mu * gd));
   if (cand != cand) cand = __builtin_inff();
   if (vel) *vel = (float)((double)*vel + gd * impulse * sqrt(RELAX_PI2) * dx1);
