@@ -817,28 +817,7 @@ int relax_model_set_planes(relax_model_t* m, const relax_plane_t* planes, int np
   m->R.fr.planes = m->planes_dev;
   m->R.fr.np = np;
   m->R.fr.active = (np > 0) && m->mech[2];
-  // the box of the planes' bands: their points have x3 <= |z| + Lp and x1, x2
-  // within max(Wp, Lp) of the centre (friction3d.f90:136-148)
-  FrictionTables& F = m->R.fr;
-  double lo[2] = {1e9, 1e9}, hi[3] = {-1e9, -1e9, -1.0};
-  const double d[2] = {m->desc.dx1, m->desc.dx2};
-  for (const PlaneDev& p : m->plane_dev_host) {
-    const double c[2] = {p.x, p.y}, wl = std::max(p.Wp, p.Lp);
-    for (int a = 0; a < 2; ++a) {
-      lo[a] = std::min(lo[a], std::floor((c[a] - wl) / d[a]) - 1.0);
-      hi[a] = std::max(hi[a], std::ceil((c[a] + wl) / d[a]) + 1.0);
-    }
-    hi[2] = std::max(hi[2], (std::fabs(p.z) + p.Lp) / m->desc.dx3);
-  }
-  F.zmax = hi[2] < 0.0 ? 0 : (int)std::min((double)m->g.h3, std::floor(hi[2]) + 2.0);
-  const int n[2] = {m->g.n1, m->g.n2};
-  int x0[2] = {0, 0}, nx[2] = {n[0], n[1]};
-  for (int a = 0; a < 2; ++a)
-    if (lo[a] >= -n[a] && hi[a] < n[a] && hi[a] - lo[a] + 1.0 < n[a]) {
-      x0[a] = ((int)lo[a] + 2 * n[a]) % n[a];
-      nx[a] = (int)(hi[a] - lo[a]) + 1;
-    }
-  F.x0 = x0[0]; F.nx = nx[0]; F.y0 = x0[1]; F.ny = nx[1];
+  band_box(m->R.fr, m->plane_dev_host.data(), np, m->g.n1, m->g.n2, m->g.h3, m->desc.dx1, m->desc.dx2, m->desc.dx3);
   m->md_dirty = true;
   return RELAX_OK;
 }

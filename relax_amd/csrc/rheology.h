@@ -69,7 +69,7 @@ __device__ __forceinline__ double d_my_sinh(double x) {
   return sinh(x);
 }
 // shiftedcoordinates, elastic3d.f90:4027-4048 (0-based index)
-__device__ __forceinline__ double d_shifted(int i, int n, double dx) {
+__host__ __device__ __forceinline__ double d_shifted(int i, int n, double dx) {
   return (double)(i < n / 2 ? i : i - n) * dx;
 }
 
@@ -188,7 +188,7 @@ __device__ __forceinline__ float friction_point(const RheoParams& R, const Plane
 constexpr double BAND = 7.02;
 
 // whether point (i1,i2,i3) lies in the band of a plane
-__device__ __forceinline__ bool in_band(const RheoParams& R, int i1, int i2, int i3) {
+__host__ __device__ __forceinline__ bool in_band(const RheoParams& R, int i1, int i2, int i3) {
 #pragma clang fp contract(off)
   if (i3 >= R.fr.zmax) return false;
   const double x1 = d_shifted(i1, R.n1, R.dx1), x2 = d_shifted(i2, R.n2, R.dx2), x3 = (double)i3 * R.dx3;
@@ -204,7 +204,7 @@ __device__ __forceinline__ bool in_band(const RheoParams& R, int i1, int i2, int
 
 // depths [lo, hi] between which the bands of all planes cross column (i1,i2)
 // (lo > hi: none)
-__device__ __forceinline__ void column_band(const RheoParams& R, int i1, int i2, int& lo, int& hi) {
+__host__ __device__ __forceinline__ void column_band(const RheoParams& R, int i1, int i2, int& lo, int& hi) {
 #pragma clang fp contract(off)
   lo = R.fr.zmax;
   hi = -1;
@@ -228,6 +228,38 @@ __device__ __forceinline__ void column_band(const RheoParams& R, int i1, int i2,
     lo = min(lo, max(0, (int)floor(fmin(za * r, 1e9) - 1e-3)));
     hi = max(hi, min(R.fr.zmax - 1, (int)ceil(zb * r + 1e-3)));
   }
+}
+
+// The box of all planes' bands, with a sample to spare: depths below zmax and
+// the samples along x1 and x2 (the whole axis where the box wraps or a plane's
+// geometry is not a number; a plane of negative extent reaches nothing).
+inline void band_box(FrictionTables& F, const PlaneDev* planes, int np, int n1, int n2, int h3, double dx1, double dx2,
+                     double dx3) {
+  const double far = 1e9;
+  double lo[2] = {far, far}, hi[2] = {-far, -far}, depth = -1.0;
+  for (int k = 0; k < np; ++k) {
+    const PlaneDev& P = planes[k];
+    const double x[2] = {P.x, P.y}, d[2] = {dx1, dx2}, wl = fmax(P.Wp, P.Lp);
+    double a[2], b[2];
+    for (int i = 0; i < 2; ++i) {
+      a[i] = floor((x[i] - wl) / d[i]) - 1.0;
+      b[i] = ceil((x[i] + wl) / d[i]) + 1.0;
+      if (!(a[i] > b[i] || a[i] <= b[i])) { a[i] = -far; b[i] = far; }
+    }
+    if (a[0] > b[0] || a[1] > b[1]) continue;
+    for (int i = 0; i < 2; ++i) { lo[i] = fmin(lo[i], a[i]); hi[i] = fmax(hi[i], b[i]); }
+    const double z = (fabs(P.z) + P.Lp) / dx3;
+    depth = z <= far ? fmax(depth, z) : far;  // not a number: the whole depth
+  }
+  F.zmax = depth < 0.0 ? 0 : (int)fmin((double)h3, floor(depth) + 2.0);
+  const int n[2] = {n1, n2};
+  int x0[2] = {0, 0}, nx[2] = {n1, n2};
+  for (int i = 0; i < 2; ++i)
+    if (lo[i] <= hi[i] && lo[i] >= -n[i] && hi[i] < n[i] && hi[i] - lo[i] + 1.0 < n[i]) {
+      x0[i] = ((int)lo[i] + 2 * n[i]) % n[i];
+      nx[i] = (int)(hi[i] - lo[i]) + 1;
+    }
+  F.x0 = x0[0]; F.nx = nx[0]; F.y0 = x0[1]; F.ny = nx[1];
 }
 
 // Moment-density rate of all mechanisms at one point (relax.f90:568-612).
