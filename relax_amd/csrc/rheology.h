@@ -182,10 +182,13 @@ __device__ __forceinline__ float friction_point(const RheoParams& R, const Plane
 }
 
 // The band of a creeping plane: every grid point where friction_point passes
-// its gates, and a little more (7.02 instead of 7.01 dx1).  Kernels with and
-// without the creep code share a model's points by these tests, so no
-// contraction: they round alike wherever they are inlined.
-constexpr double BAND = 7.02;
+// its gates, and a little more.  Kernels with and without the creep code share
+// a model's points by these tests, which round alike wherever they are inlined
+// (no contraction); friction_point's own gates may round apart from them, so
+// each gate is a hundredth of a sample wider here, far more than a coordinate's
+// rounding.  As there, a gate that is not a number does not shut.
+constexpr double BAND = 7.02;  // instead of 7.01 dx1
+constexpr double GATE = 0.01;  // samples
 
 // whether point (i1,i2,i3) lies in the band of a plane
 __host__ __device__ __forceinline__ bool in_band(const RheoParams& R, int i1, int i2, int i3) {
@@ -195,9 +198,10 @@ __host__ __device__ __forceinline__ bool in_band(const RheoParams& R, int i1, in
   bool in = false;
   for (int k = 0; k < R.fr.np; ++k) {
     const PlaneDev& P = R.fr.planes[k];
-    const double wl = fmax(P.Wp, P.Lp), c = P.cdip * (P.cstrike * x1 - P.sstrike * x2) - P.xr, d = P.sdip * x3;
-    in = in || (x3 <= fabs(P.z) + P.Lp && fabs(x1 - P.x) <= wl && fabs(x2 - P.y) <= wl &&
-                (fabs(c - d) <= BAND * R.dx1 || fabs(c + d) <= BAND * R.dx1));
+    const double wl = fmax(P.Wp, P.Lp), zl = P.Lp + GATE * R.dx3, w = BAND * R.dx1;
+    const double c = P.cdip * (P.cstrike * x1 - P.sstrike * x2) - P.xr, d = P.sdip * x3;
+    in = in || !((fabs(x3 - P.z) > zl && fabs(x3 + P.z) > zl) || fabs(x1 - P.x) > wl + GATE * R.dx1 ||
+                 fabs(x2 - P.y) > wl + GATE * R.dx2 || (fabs(c - d) > w && fabs(c + d) > w));
   }
   return in;
 }
@@ -212,9 +216,9 @@ __host__ __device__ __forceinline__ void column_band(const RheoParams& R, int i1
   for (int k = 0; k < R.fr.np; ++k) {
     const PlaneDev& P = R.fr.planes[k];
     const double wl = fmax(P.Wp, P.Lp);
-    if (!(fabs(x1 - P.x) <= wl && fabs(x2 - P.y) <= wl)) continue;
+    if (fabs(x1 - P.x) > wl + GATE * R.dx1 || fabs(x2 - P.y) > wl + GATE * R.dx2) continue;
     const double c = P.cdip * (P.cstrike * x1 - P.sstrike * x2) - P.xr, w = BAND * R.dx1, sd = fabs(P.sdip);
-    const double zlim = fabs(P.z) + P.Lp;
+    const double zl = fabs(P.z) + P.Lp + GATE * R.dx3, zlim = zl < 1e300 ? zl : 1e300;
     // |c| - w <= sd x3 <= |c| + w bounds both the plane and its image
     double za = 0.0, zb = zlim;
     if (sd * zlim > 1e-9 * R.dx1) {
@@ -226,7 +230,7 @@ __host__ __device__ __forceinline__ void column_band(const RheoParams& R, int i1
     if (za > zb + R.dx3) continue;
     const double r = 1.0 / R.dx3;
     lo = min(lo, max(0, (int)floor(fmin(za * r, 1e9) - 1e-3)));
-    hi = max(hi, min(R.fr.zmax - 1, (int)ceil(zb * r + 1e-3)));
+    hi = max(hi, (int)fmin((double)(R.fr.zmax - 1), ceil(fmin(zb * r, 1e9) + 1e-3)));
   }
 }
 

@@ -1,6 +1,8 @@
-"""The box of the creep bands (rheology.h: band_box, column_band), compiled for
-the host: it holds every column range and every point that passes the gates of
-frictioneigenstress, and no geometry makes a box that is not on the grid."""
+"""The points that the creep kernels take (rheology.h: in_band, column_band,
+band_box), compiled for the host: every point that passes the gates of
+frictioneigenstress lies in the band, its column's depth range and the box of
+the band launches, on the gates' very edges too, and no geometry makes a box
+that is not on the grid."""
 import ctypes
 import os
 import subprocess
@@ -62,3 +64,30 @@ def test_box_is_on_the_grid(native, geometry, pair):
     assert 0 <= zmax <= n[2] and 0 <= x0 < n[0] and 1 <= nx <= n[0] and 0 <= y0 < n[1] and 1 <= ny <= n[1]
     _, _, _, outside, columns = call(native.creep_sweep, p, n, (1.0, 1.0, 1.0), 5, np.int64)
     assert (outside, columns) == (0, 0)
+
+
+def edge_planes(rng, dx):
+    """Planes whose gates pass through grid points: centre and extent in whole
+    or half samples of decimal spacings, dips and strikes of round degrees."""
+    out = []
+    for _ in range(int(rng.integers(1, 3))):
+        half = lambda a, b: 0.5 * int(rng.integers(2 * a, 2 * b))
+        length, width = half(2, 20), half(2, 20)
+        # z + Lp, x + wl on whole samples: (1 + 2 beta)/2 = 0.7 of the extent
+        grow = rng.integers(2) * 0.7
+        z = half(0, 12) + (grow * length if rng.integers(2) else 0.0)
+        x, y = half(-16, 16) + grow * max(length, width), half(-8, 8) - grow * max(length, width)
+        strike, dip = np.deg2rad(15.0 * rng.integers(0, 24)), np.deg2rad(15.0 * rng.integers(-6, 13))
+        out.append(plane(x * dx[0], y * dx[1], z * dx[2], length * dx[2], width * dx[2], strike, dip))
+    return np.concatenate(out)
+
+
+@pytest.mark.parametrize("dx", [(0.1, 0.1, 0.1), (0.3, 0.7, 0.1), (1.0, 1.0, 1.0), (1e3 / 3, 1e3 / 3, 50.0), (0.05, 0.6, 0.9)])
+@pytest.mark.parametrize("n", [(64, 32, 16), (32, 32, 32)])
+def test_points_on_the_gates(native, n, dx):
+    rng = np.random.default_rng(11)
+    total = np.zeros(5, np.int64)
+    for _ in range(250):
+        total += call(native.creep_sweep, edge_planes(rng, dx), n, dx, 5, np.int64)
+    assert total[0] > 10000
+    assert (total[1:] == 0).all(), total
