@@ -22,6 +22,7 @@ namespace {
 
 struct ColumnConsts {
   float ratio1, ratio2p1;     // elasticresponse: (l+m)/(l+2m)/m/(2pi)^2, 1 + m/(l+m)
+  float ratio2;               // m/(l+m)
   float mu2pi, mod2pi, lam2pi, grav;  // traction: 2 pi mu, 2 pi (l+2m), 2 pi l, 2 mu alpha gamma
   float alpha, inv_alpha;
   float inv_n3dx3;
@@ -34,6 +35,7 @@ __host__ ColumnConsts make_consts(const GreenConst& gc) {
   const double alpha = (l + m) / (l + 2.0 * m);
   c.ratio1 = (float)((l + m) / (l + 2.0 * m) / m / (RELAX_PI2 * RELAX_PI2));
   c.ratio2p1 = (float)(1.0 + m / (l + m));
+  c.ratio2 = (float)(m / (l + m));
   c.mu2pi = (float)(RELAX_PI2 * m);
   c.mod2pi = (float)(RELAX_PI2 * (l + 2.0 * m));
   c.lam2pi = (float)(RELAX_PI2 * l);
@@ -590,9 +592,10 @@ __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu,
 //
 // 4 columns per workgroup, 30 KB of LDS, three waves: workgroups this small
 // wait for few others at each of the 15 barriers and four of them share a
-// compute unit.  512x512x512: 800 us (LDS form k_green_columns 1112; 8 columns
-// 1257, though its rows are 64 contiguous bytes; the vector instructions take
-// 605, the memory 320).  Four waves per SIMD instead of three: the same.
+// compute unit.  512x512x512: 823 us (LDS form k_green_columns 1112; 800 with
+// the traction summed as separate series; with those, 8 columns took 1257,
+// though its rows are 64 contiguous bytes, the vector instructions alone 605,
+// the memory 320).  Four waves per SIMD instead of three: the same.
 constexpr int DEEP_TX = 4;  // columns per workgroup
 __global__ __launch_bounds__(48 * DEEP_TX, 3) void k_green_deep(ColumnConsts C, double mu, double alpha, double gamma,
                                                                int n1, int n2, MPtr<float2> W_m, MPtr<float2> NQ_m,
@@ -604,7 +607,7 @@ __global__ __launch_bounds__(48 * DEEP_TX, 3) void k_green_deep(ColumnConsts C, 
   __shared__ float2 buf[3 * Q * RS];
   __shared__ float2 stw[H3];   // w_n3^z
   __shared__ float2 tws[256];  // w_H3^(j k1), row j
-  __shared__ float2 red[2][3][TX];
+  __shared__ float2 red[4][TX];
   __shared__ float2 pv[3][TX];
   __shared__ CerrutiCol ccs[TX];
   const int tid = threadIdx.x;
@@ -644,9 +647,16 @@ __global__ __launch_bounds__(48 * DEEP_TX, 3) void k_green_deep(ColumnConsts C, 
   };
   // this component's wavenumber is kx + kz k3
   const float kx = c == 0 ? k1w : c == 1 ? k2w : 0.f, kz = c == 2 ? 1.f : 0.f;
-  // this component's sums of k3 u and u over the frequencies
-  float2 Sk = make_float2(0.f, 0.f), Su = Sk;
+  // the sums over the frequencies of the traction (green.f90:357-359).  St:
+  // k3 u1, k3 u2 and, formed per frequency so that its two parts cancel before
+  // they are summed, 2 mu k3 u3 + l k.u, where k.u = m/(l+m) |k|^2 (k.c) denom;
+  // Su: u3.  Short partial sums: 8 frequencies, then the halves, then the
+  // lanes.  (One sum of 32 each of k3 u_c and u_c left the vertical surface
+  // displacement 6-12 % further from 64 bits than k_green_columns does.)
+  float2 St = make_float2(0.f, 0.f), Su = St;
+  const float m4pi = 2.f * C.mu2pi;
   auto forward = [&](bool odd, float2* X) {
+    float2 t[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)}, u[2] = {t[0], t[0]};
     if (odd) {
 #pragma unroll
       for (int m = 0; m < 16; ++m) x[m] = cmul(x[m], stw[Q * m + r]);
@@ -676,12 +686,22 @@ __global__ __launch_bounds__(48 * DEEP_TX, 3) void k_green_deep(ColumnConsts C, 
       const float2 d = make_float2(k1w * a1.x + k2w * a2.x + k3 * a3.x, k1w * a1.y + k2w * a2.y + k3 * a3.y);
       float2 a = make_float2((s * X[k2].x - kc * d.x) * denom, (s * X[k2].y - kc * d.y) * denom);
       // the k = 0 frequency is zeroed (green.f90:96-99)
-      if (!odd && k2 == 0 && A.k1i == 0 && A.k2i == 0 && r == 0) a = make_float2(0.f, 0.f);
+      const bool zero = !odd && k2 == 0 && A.k1i == 0 && A.k2i == 0 && r == 0;
+      if (zero) a = make_float2(0.f, 0.f);
       X[k2] = a;
-      Sk = make_float2(fmaf(k3, a.x, Sk.x), fmaf(k3, a.y, Sk.y));
-      Su = cadd(Su, a);
+      float2& tk = t[k2 & 1];
+      if (c == 2) {
+        const float g = zero ? 0.f : C.lam2pi * (C.ratio2 * r2 * denom);
+        const float2 d3 = zero ? make_float2(0.f, 0.f) : d;
+        tk = cadd(tk, make_float2(fmaf(m4pi * k3, a.x, g * d3.x), fmaf(m4pi * k3, a.y, g * d3.y)));
+        u[k2 & 1] = cadd(u[k2 & 1], a);
+      } else {
+        tk = make_float2(fmaf(k3, a.x, tk.x), fmaf(k3, a.y, tk.y));
+      }
       if (k2 % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // the other components' reads stay few in registers
     }
+    St = cadd(St, cadd(t[0], t[1]));
+    Su = cadd(Su, cadd(u[0], u[1]));
     __syncthreads();
   };
   float2 X0[Q], X1[Q];
@@ -691,10 +711,13 @@ __global__ __launch_bounds__(48 * DEEP_TX, 3) void k_green_deep(ColumnConsts C, 
   // a column's sums: lanes TX apart in the component's wave
 #pragma unroll
   for (int off = 32; off >= TX; off >>= 1) {
-    Sk.x += __shfl_xor(Sk.x, off); Sk.y += __shfl_xor(Sk.y, off);
+    St.x += __shfl_xor(St.x, off); St.y += __shfl_xor(St.y, off);
     Su.x += __shfl_xor(Su.x, off); Su.y += __shfl_xor(Su.y, off);
   }
-  if ((tid & 63) < TX) { red[0][c][col] = Sk; red[1][c][col] = Su; }
+  if ((tid & 63) < TX) {
+    red[c][col] = St;
+    if (c == 2) red[3][col] = Su;
+  }
   __syncthreads();
   if (tid < 3 * TX) {
     const int d = tid / TX, t = tid % TX;
@@ -702,18 +725,14 @@ __global__ __launch_bounds__(48 * DEEP_TX, 3) void k_green_deep(ColumnConsts C, 
     // sum_k3 of the traction summands (green.f90:357-359):
     //   i 2 pi mu (k3 u1 + k1 u3), i 2 pi mu (k3 u2 + k2 u3),
     //   i 2 pi ((l+2m) k3 u3 + l (k1 u1 + k2 u2)) - 2 mu alpha gamma u3
-    const float2 u3 = red[1][2][t];
+    const float2 sd = red[d][t], u3 = red[3][t];
     float2 acc;
     if (d < 2) {
       const float qc = d == 0 ? q1 : q2;
-      const float2 sk = red[0][d][t];
-      const float2 a = make_float2(sk.x + qc * u3.x, sk.y + qc * u3.y);
+      const float2 a = make_float2(sd.x + qc * u3.x, sd.y + qc * u3.y);
       acc = make_float2(-C.mu2pi * a.y, C.mu2pi * a.x);
     } else {
-      const float2 sk = red[0][2][t], u1 = red[1][0][t], u2 = red[1][1][t];
-      const float2 h = make_float2(q1 * u1.x + q2 * u2.x, q1 * u1.y + q2 * u2.y);
-      const float2 e = make_float2(C.mod2pi * sk.x + C.lam2pi * h.x, C.mod2pi * sk.y + C.lam2pi * h.y);
-      acc = make_float2(-e.y - C.grav * u3.x, e.x - C.grav * u3.y);
+      acc = make_float2(-sd.y - C.grav * u3.x, sd.x - C.grav * u3.y);
     }
     const float2 tt = gload(A.tbase + d * A.tcs + t);
     // p = t - p / (sx3 dx3)   (green.f90:373-375, :1082-1084)

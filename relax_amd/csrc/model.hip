@@ -312,7 +312,7 @@ static void tune_lookup(relax_model_t* m) {
 //    210).
 //  - Green column pass: the register form from 64-deep columns up (64x64x128:
 //    11.0 against 16.0, 256x256x128: 51.6 against 65.1, 512x512x256: 264
-//    against 419, 512x512x512: 800 against 1112); 32-deep columns radix 8
+//    against 419, 512x512x512: 823 against 1112); 32-deep columns radix 8
 //    (512x512x64: 87.8 against 94.9, the register form 128).  The forms round
 //    differently, and the slip of a creeping patch near the clamp of its
 //    friction law follows that rounding (5e-5 of the slip after 20 steps at
