@@ -335,8 +335,10 @@ int relax_model_synchronize(relax_model_t* m);
  * :2788-2873, with the model's taper); sig = -tau + C:eps(u).  A
  * tetrahedron's vertex index outside 1..nv is RELAX_ERR_ARG.  Tensile cracks and point sources reach
  * above the surface (their images), so such an event takes the full-depth
- * Green solve on temporary buffers; shear patches and loads alone take the
- * step's pruned solve.  Sources below the Nyquist size get no displacement
+ * Green solve, in the model's stress and work fields; shear patches and loads
+ * alone take the step's pruned solve.  An event that fails on the device
+ * after that solve was begun leaves sig = -tau + C:eps(u) of u and tau as
+ * they then are.  Sources below the Nyquist size get no displacement
  * (the reference adds Okada's solution for shear patches at t = 0 only,
  * relax.f90:357-360).  The event's surface loads stay with the model: the
  * following steps add the rate of the periodic ones to the surface traction

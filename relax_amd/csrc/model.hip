@@ -1912,6 +1912,11 @@ int relax_model_event(relax_model_t* m, const relax_event_t* ev, double nyquist)
   HIP_TRY(hipMemcpyAsync(&t, &m->sc->t, sizeof(double), hipMemcpyDeviceToHost, m->stream));
   HIP_TRY(hipStreamSynchronize(m->stream));
   const double dx1 = m->desc.dx1, dx2 = m->desc.dx2, dx3 = m->desc.dx3, lam = m->desc.lambda, mu = m->desc.mu;
+  // whatever fails while the solve holds sig, the model keeps a stress
+  struct SigLost {
+    relax_model_t* m = nullptr;
+    ~SigLost() { if (m) (void)model_stress_set(m); }
+  } sig_lost;
   if (nt == 0 && nm == 0) {
     // body forces in the top half only: the pruned Green solve of the step,
     // adding to u (relax.f90:362-371, :877-884)
@@ -1936,9 +1941,13 @@ int relax_model_event(relax_model_t* m, const relax_event_t* ev, double nyquist)
     // allocated and freed by each event: 386 us of 1180 at 256x256x128.)
     const long ld = g.n1 + 2, vs = ld * g.n2 * g.n3, ts = ld * g.n2;
     if (2 * vs > 6 * H || vs + 3 * ts > 3 * H) return RELAX_ERR_SIZE;
+    // an error that an earlier call left pending would fail the first launch:
+    // it is reported while the state stands
+    if (hipGetLastError() != hipSuccess) return RELAX_ERR_HIP;
     float* v[3] = {m->sig, m->sig + vs, m->W};
     float* tr[3] = {m->W + vs, m->W + vs + ts, m->W + vs + 2 * ts};
     const Field3 f{{v[0], v[1], v[2]}};
+    sig_lost.m = m;
     HIP_TRY(hipMemsetAsync(m->sig, 0, 2 * vs * 4, m->stream));
     HIP_TRY(hipMemsetAsync(m->W, 0, (vs + 3 * ts) * 4, m->stream));
     if (nbig && (rc = launch_source(m->shear_dev, m->shear_slip, nbig, mu, g.n1, g.n2, g.h3, dx1, dx2, dx3, f, ld,
@@ -1970,6 +1979,7 @@ int relax_model_event(relax_model_t* m, const relax_event_t* ev, double nyquist)
   Ctx c = single(m);
   c.prof = nullptr;
   if ((rc = launch_stress(STRESS_SET, g, m->S, c.md, c.one, 1, RHEO_VISCOUS, m->stream))) return rc;
+  sig_lost.m = nullptr;
   HIP_TRY(hipStreamSynchronize(m->stream));
   return RELAX_OK;
 }
