@@ -577,9 +577,20 @@ __device__ __forceinline__ void stress_block(const Grid& g, const RheoParams& R,
 // of its blocks (in address order: the sums keep one order), then takes them
 // 256 at a time: at 256x256x128 with a plane of 38x16 km 22 us (corrector)
 // beside 99 us for the other points, against 155 us for one kernel with the
-// creep code and 49 us for a band launch without the gathering.  Their sums are added to those that the launch over the other
-// points left in entry b0.
+// creep code and 49 us for a band launch without the gathering.  Their sums
+// are added to those that the launch over the other points left in entry b0.
 constexpr int SEGS = 16;
+// Blocks that a workgroup gathers: MIN_SEGS to SEGS, a power of two that divides
+// the grid's blocks (64 at least).  Between them 4096 groups, of which the
+// bands cross a few hundred: a step of 256x256x128 takes 704 us with groups of
+// 4, 709 with 8, 724 with 16; eight models of 64^3 in a batch 362 us with 4, 375
+// with 2, 381 with 1.  It hangs on the grid alone: the sums of power and C:E^i
+// are formed in one order whether a model is stepped by itself or in a batch.
+constexpr int MIN_SEGS = 4;
+__host__ __device__ __forceinline__ int band_segs(const Grid& g) {
+  const int s = (int)(g.H / 256 / 4096);
+  return s < MIN_SEGS ? MIN_SEGS : s > SEGS ? SEGS : s;
+}
 template <int MODE, bool EXT>
 __device__ __forceinline__ void stress_band(const Grid& g, const RheoParams& R, const StencilConst& S,
                                             const float* __restrict__ X, float* __restrict__ sig,
@@ -698,20 +709,19 @@ __global__ __launch_bounds__(256) void k_stress_list(const ModelDev* __restrict_
   }
 }
 
-// items in groups of SEGS, as many as belong to one model
+// MIN_SEGS items per workgroup, all of one model (its items are a multiple of
+// 64); a group of band_segs blocks goes to the workgroup that holds its first
 template <int MODE, bool EXT>
 __global__ __launch_bounds__(256) void k_stress_band_list(const ModelDev* __restrict__ md,
                                                           const WorkItem* __restrict__ wl, int nm) {
-  const long total = wl[nm].first, last = min(total, ((long)blockIdx.x + 1) * SEGS);
-  for (long item = (long)blockIdx.x * SEGS; item < last;) {
-    const int m = work_model(wl, nm, item);
-    const ModelDev& D = md[m];
-    const long end = min(last, wl[m + 1].first);
-    stress_band<MODE, EXT>(wl[m].g, D.R, wl[m].S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em,
-                           D.sc, D.partials, (int)(item - wl[m].first), (int)(end - wl[m].first));
-    __syncthreads();  // the lists in LDS are reused
-    item = end;
-  }
+  const long item = (long)blockIdx.x * MIN_SEGS;
+  if (item >= wl[nm].first) return;
+  const int m = work_model(wl, nm, item);
+  const int segs = band_segs(wl[m].g), b0 = (int)(item - wl[m].first);
+  if (b0 % segs) return;
+  const ModelDev& D = md[m];
+  stress_band<MODE, EXT>(wl[m].g, D.R, wl[m].S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em, D.sc,
+                         D.partials, b0, b0 + segs);
 }
 
 template <int TXB, int TYB, bool TM, bool RAW, bool EXT, int PART, int BTY, bool ZR>
@@ -879,10 +889,9 @@ int launch_stress(int mode, const Grid& g, const StencilConst& S, const ModelDev
   const ModelDev Dv = batch ? ModelDev{} : *one;
   if (rclass < RHEO_VISCOUS || rclass > RHEO_ALL) return RELAX_ERR_ARG;
   const dim3 grid((unsigned)stress_blocks(g), (unsigned)nm);
-  // the creep bands' part: no deeper than they reach, as many blocks per
-  // workgroup as leave two workgroups per CU (their registers admit two)
+  // the creep bands' part: no deeper than they reach
   const long nin = batch ? stress_blocks(g) : std::min(stress_blocks(g), ((long)g.n1 * g.n2 * Dv.R.fr.zmax + 255) / 256);
-  const int segs = (int)std::max(1L, std::min((long)SEGS, nin * nm / (2 * device_cus())));
+  const int segs = band_segs(g);
   const dim3 gin((unsigned)std::max(1L, (nin + segs - 1) / segs), (unsigned)nm);
 #define K(MODE, E, PART, GR)                                                     \
   {                                                                              \
@@ -981,7 +990,7 @@ int launch_stress_list(int mode, const WorkItem* wl, const ModelDev* md, int nm,
     if (!(rclass & RHEO_CREEP)) { K(MODE, E, PART_ALL) }       \
     else {                                                     \
       K(MODE, E, PART_OUT)                                     \
-      k_stress_band_list<MODE, E><<<(unsigned)((total + SEGS - 1) / SEGS), 256, 0, st>>>(md, wl, nm); \
+      k_stress_band_list<MODE, E><<<(unsigned)((total + MIN_SEGS - 1) / MIN_SEGS), 256, 0, st>>>(md, wl, nm); \
     }                                                          \
   }
 #define KM(MODE)                          \
