@@ -407,8 +407,9 @@ int relax_model_points(relax_model_t* m, const double* x, int n, double rot, dou
 /* Autotuner: times the launch-shape variants of the tunable kernels (columns
  * per workgroup of the y transform, columns/threads/radix of the Green
  * column pass, divergence tile and depth chunk) on this model's scratch buffers and keeps the
- * fastest for this device and grid; later models of the grid in the process
- * use the choice.  choice (3 ints, may be NULL) receives the variants;
+ * fastest for this device and grid; later models of the grid in the process,
+ * of any rheology, use the choice in place of the defaults of their grid and
+ * rheology class.  choice (3 ints, may be NULL) receives the variants;
  * ms (may be NULL) the average time of one launch of each variant in
  * milliseconds, 3 rows of RELAX_TUNE_VARIANTS (columns, Green, divergence),
  * with -1 for a variant that does not apply to the grid.  The model's state

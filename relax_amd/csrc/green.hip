@@ -592,7 +592,7 @@ __global__ __launch_bounds__(512, 4) void k_green_reg(ColumnConsts C, double mu,
 //
 // 4 columns per workgroup, 30 KB of LDS, three waves: workgroups this small
 // wait for few others at each of the 15 barriers and four of them share a
-// compute unit.  512x512x512: 823 us (LDS form k_green_columns 1112; 800 with
+// compute unit.  512x512x512: 842 us (LDS form k_green_columns 1112; 800 with
 // the traction summed as separate series; with those, 8 columns took 1257,
 // though its rows are 64 contiguous bytes, the vector instructions alone 605,
 // the memory 320).  Four waves per SIMD instead of three: the same.

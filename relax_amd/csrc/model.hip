@@ -312,12 +312,14 @@ static void tune_lookup(relax_model_t* m) {
 //    210).
 //  - Green column pass: the register form from 64-deep columns up (64x64x128:
 //    11.0 against 16.0, 256x256x128: 51.6 against 65.1, 512x512x256: 264
-//    against 419, 512x512x512: 823 against 1112); 32-deep columns radix 8
+//    against 419, 512x512x512: 842 against 1112); 32-deep columns radix 8
 //    (512x512x64: 87.8 against 94.9, the register form 128).  The forms round
 //    differently, and the slip of a creeping patch near the clamp of its
 //    friction law follows that rounding (5e-5 of the slip after 20 steps at
 //    256x256x128): models with creeping planes keep the radix-16 LDS form, in a
-//    batch too (green_launches).
+//    batch too (green_launches).  That is the untuned choice: one that
+//    relax_model_autotune made holds for every later model of its grid,
+//    creeping or not.
 //  - divergence: the register-window tiles wherever 64 divides n1, 64x8 on
 //    grids under 128^3 (64x64x64: 7.6 against 9.1 for 64x16 and 31 for the
 //    32x8 ring), else 64x16 (512x512x256: 247 against 268, ring 303).  The

@@ -575,7 +575,7 @@ __device__ __forceinline__ void stress_block(const Grid& g, const RheoParams& R,
 // a point with the creep code costs ten viscous ones and the bands hold a few
 // points of every block they cross, so the workgroup first gathers the points
 // of its blocks (in address order: the sums keep one order), then takes them
-// 256 at a time: at 256x256x128 with a plane of 38x16 km 22 us (corrector)
+// 256 at a time: at 256x256x128 with a plane of 38x16 km 21 us (corrector)
 // beside 99 us for the other points, against 155 us for one kernel with the
 // creep code and 49 us for a band launch without the gathering.  Their sums
 // are added to those that the launch over the other points left in entry b0.
@@ -823,11 +823,10 @@ static int tiles_of(int x0, int nx, int n, int T, int* t0) {
 // is some 20 planes deep and its points cost ten times a viscous one, so the
 // bands want many short chunks (2 planes, more where that made over 2048
 // workgroups), of the tiles in the bands' box only: at 256x256x128 with a
-// plane of 38x16 km the bands take 26 us beside 34 us (64x16) or 60 us (32x16)
-// for the rest, against 142 us for one kernel with the creep code over all
-// points.  The 64x16
-// tiles' bands go to 64x8 ones (at 1024 threads the creep code spills 40-137
-// registers).
+// plane of 38x16 km the bands take 22-23 us beside 47-49 us (64x16) or 60 us
+// (32x16) for the rest, against 142 us for one kernel with the creep code over
+// all points.  The 64x16 tiles' bands go to 64x8 ones (at 1024 threads the
+// creep code spills 40-137 registers).
 template <int TX, int TY, bool ZR, bool EXT>
 static void body_parts(const BodyLaunch& b, int rclass, int zc, int gz) {
   const TileBox all{0, b.g.n1 / TX, 0, b.g.n2 / TY};
