@@ -1331,7 +1331,7 @@ int relax_model_run(relax_model_t* m, int nsteps, const double* dt_override, rel
 // --------------------------------------------------- coseismic set-up ----
 // The source kernels add a list of sources, each of which reaches a small part
 // of the grid, point by point in the list's order.  A workgroup takes
-// SRC_POINTS points in address order (whole rows), gathers, still in order,
+// src_chunk points in address order (whole rows), gathers, still in order,
 // the sources whose gates along x2 and x3 the rows can pass, and visits the
 // samples along x1 that these reach, packed onto its threads; most workgroups
 // gather none and leave.  The FP64 tapers and Gaussians of the points visited
@@ -1339,7 +1339,27 @@ int relax_model_run(relax_model_t* m, int nsteps, const double* dt_override, rel
 // and 669 us (k_add_shear) with every point testing every source, 51 and 39 us
 // so, with 1024 points to a workgroup 87 and 67, with 8192 62 and 45.  A crack
 // and two point sources over 256x256x256: 139 and 133 us before, 29 and 23 now.
-constexpr int SRC_POINTS = 2048, SRC_LIST = 1024;
+constexpr int SRC_LIST = 1024;
+
+// Points per workgroup: 2048, fewer where that would leave less than 4096
+// workgroups and latency bound them (20 patches at 256x256x128: 28 and 18 us
+// with 1024, 40 and 26 with 2048).
+static int src_chunk(long n) {
+  int p = 256;
+  while (p < 2048 && n / (2 * p) >= 4096) p *= 2;
+  return p;
+}
+
+// Short lists on small grids are tested whole, by a thread for every point
+// (WHOLE): the sources reach much of such a grid, and the gathering's barriers
+// and loads in a row take longer than the tests they save.  k_source and
+// k_add_shear, whole / gathered / gathered with 2048 points to a workgroup, us:
+//   64x64x64,    4 patches  12, 8.4 / 16, 10 /  28,  18
+//   64x64x64,   60 patches  56,  36 / 69, 40 / 203, 134
+//   128x128x64, 40 patches  32,  23 / 37, 21 / 100,  64
+// From 128x128x128 on the gathering wins by 33 patches (40: 42, 31 / 27, 17),
+// at 128x128x64 by 65 (129: 84, 69 / 87, 48).
+static bool src_whole(long n, int np) { return n <= (1L << 20) && n * np <= (1L << 25); }
 
 struct SrcShared {
   unsigned short list[SRC_LIST];
@@ -1350,8 +1370,8 @@ struct SrcHit {
   bool hit;
   double cx, r;
 };
-// ranges of the shifted coordinates of points [o0, o0 + SRC_POINTS) of an
-// n1 x n2 x n3 grid along x2 and x3; full: x3 shifted as well (n3 planes)
+// ranges of the shifted coordinates of rows [r0, r1] of an n1 x n2 x n3 grid
+// along x2 and x3; full: x3 shifted as well (n3 planes)
 struct SrcBox {
   double ya, yb, za, zb;
   bool top;  // has points of plane 0
@@ -1377,12 +1397,18 @@ __device__ __forceinline__ bool src_reach(double a, double b, double c0, double 
 }
 // The points of this workgroup that the sources k < np may reach:
 // hit(box, k) gives a source's SrcHit, point(o, i1, i2, i3, k0, nl) adds the
-// sources k0 + list[0..nl) to the point at address o.  All 256 threads call.
-template <class H, class F>
-__device__ __forceinline__ void src_points(SrcShared& sh, int np, int n1, int n2, int n3, double dx1, double dx2,
-                                           double dx3, bool full, H hit, F point) {
+// sources k0 + list[0..nl) (WHOLE: 0..nl) to the point at address o.  All 256
+// threads call.
+template <bool WHOLE, class H, class F>
+__device__ __forceinline__ void src_points(SrcShared& sh, int pts, int np, int n1, int n2, int n3, double dx1,
+                                           double dx2, double dx3, bool full, H hit, F point) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const long o0 = (long)blockIdx.x * SRC_POINTS, o1 = min(o0 + SRC_POINTS, (long)n1 * n2 * n3);
+  if constexpr (WHOLE) {
+    const long o = blockIdx.x * 256L + tid, r = o / n1;
+    if (o < (long)n1 * n2 * n3) point(o, (int)(o % n1), (int)(r % n2), (int)(r / n2), 0, np);
+    return;
+  }
+  const long o0 = (long)blockIdx.x * pts, o1 = min(o0 + pts, (long)n1 * n2 * n3);
   const long r0 = o0 / n1, r1 = (o1 - 1) / n1;
   const SrcBox B = src_box(r0, r1, n2, n3, dx2, dx3, full);
   for (int k0 = 0; k0 < np; k0 += SRC_LIST) {
@@ -1424,12 +1450,26 @@ __device__ __forceinline__ void src_points(SrcShared& sh, int np, int n1, int n2
     }
   }
 }
-static unsigned src_blocks(long n) { return (unsigned)((n + SRC_POINTS - 1) / SRC_POINTS); }
+// source number l of a point's list (the same in every lane)
+template <bool WHOLE>
+__device__ __forceinline__ int src_at(const SrcShared& sh, int k0, int l) {
+  return WHOLE ? l : k0 + sh.list[l];
+}
+// K: a source kernel over n points for np sources, its arguments after the
+// points per workgroup
+#define SRC_LAUNCH(K, n, np, st, ...)                                                                    \
+  do {                                                                                                   \
+    const int pts_ = src_whole(n, np) ? 256 : src_chunk(n);                                              \
+    const unsigned nb_ = (unsigned)(((n) + pts_ - 1) / pts_);                                            \
+    if (src_whole(n, np)) K<true><<<nb_, 256, 0, st>>>(pts_, __VA_ARGS__);                               \
+    else K<false><<<nb_, 256, 0, st>>>(pts_, __VA_ARGS__);                                               \
+  } while (0)
 
 // momentdensityshear (elastic3d.f90:2661-2750) of a list of patches added to
 // tau, as dislocations does at each event (relax.f90:1199-1206)
-__global__ __launch_bounds__(256) void k_add_shear(const PlaneDev* __restrict__ P, const double* __restrict__ slip,
-                                                   int np, float rmu, Grid g, double dx1, double dx2, double dx3,
+template <bool WHOLE>
+__global__ __launch_bounds__(256) void k_add_shear(int pts, const PlaneDev* __restrict__ P,
+                                                   const double* __restrict__ slip, int np, float rmu, Grid g, double dx1, double dx2, double dx3,
                                                    float* tau) {
   __shared__ SrcShared sh;
   const long H = g.H;
@@ -1437,13 +1477,14 @@ __global__ __launch_bounds__(256) void k_add_shear(const PlaneDev* __restrict__ 
     const PlaneDev& p = P[k];
     return SrcHit{src_reach(B.za, B.zb, p.z, p.Lp) && src_reach(B.ya, B.yb, p.y, p.Wp), p.x, p.Wp};
   };
-  src_points(sh, np, g.n1, g.n2, g.h3, dx1, dx2, dx3, false, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+  src_points<WHOLE>(sh, pts, np, g.n1, g.n2, g.h3, dx1, dx2, dx3, false, hit,
+                    [&](long o, int i1, int i2, int i3, int k0, int nl) {
     const double x3 = (double)i3 * dx3;
     const double x1 = d_shifted(i1, g.n1, dx1), x2 = d_shifted(i2, g.n2, dx2);
     float acc[6] = {0, 0, 0, 0, 0, 0};
     bool any = false;
     for (int l = 0; l < nl; ++l) {
-      const int k = k0 + sh.list[l];
+      const int k = src_at<WHOLE>(sh, k0, l);
       const PlaneDev& p = P[k];
       if (fabs(x3 - p.z) > p.Lp) continue;
       if ((fabs(x1 - p.x) > p.Wp) || (fabs(x2 - p.y) > p.Wp)) continue;
@@ -1491,9 +1532,8 @@ static int stage_planes(relax_model_t* m, const double* slip) {
 // momentdensityshear of the staged patches [k0, k0+n) added to tau
 static int add_shear(relax_model_t* m, int k0, int n) {
   if (n == 0) return RELAX_OK;
-  k_add_shear<<<src_blocks(m->g.H), 256, 0, m->stream>>>(m->shear_dev + k0, m->shear_slip + k0, n,
-                                                      2.0f * (float)m->desc.mu, m->g, m->desc.dx1, m->desc.dx2,
-                                                      m->desc.dx3, m->tau);
+  SRC_LAUNCH(k_add_shear, m->g.H, n, m->stream, m->shear_dev + k0, m->shear_slip + k0, n, 2.0f * (float)m->desc.mu,
+             m->g, m->desc.dx1, m->desc.dx2, m->desc.dx3, m->tau);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 
@@ -1513,9 +1553,11 @@ int relax_model_add_shear(relax_model_t* m, const relax_plane_t* patches, const 
 // planes' contributions added in their order with the reference's
 // rounding (two FP32 roundings per plane and component); threads of the top
 // plane also add the surface traction (n sdyad mu s b) e3.
-__global__ __launch_bounds__(256) void k_source(const PlaneDev* __restrict__ P, const double* __restrict__ slip, int np,
-                                                double mu, int n1, int n2, int h3, double dx1, double dx2, double dx3,
-                                                Field3 f, long ld, float* t, long ts) {
+template <bool WHOLE>
+__global__ __launch_bounds__(256, WHOLE ? 4 : 1) void k_source(int pts, const PlaneDev* __restrict__ P,
+                                                               const double* __restrict__ slip, int np, double mu, int n1,
+                                                               int n2, int h3, double dx1, double dx2, double dx3,
+                                                               Field3 f, long ld, float* t, long ts) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
     // the surface traction has no gate in depth
@@ -1524,13 +1566,14 @@ __global__ __launch_bounds__(256) void k_source(const PlaneDev* __restrict__ P, 
                       (B.top || src_reach(B.za, B.zb, p.z, p.Lp) || src_reach(B.za, B.zb, -p.z, p.Lp)),
                   p.x, fmax(p.Lp, p.Wp)};
   };
-  src_points(sh, np, n1, n2, h3, dx1, dx2, dx3, false, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+  src_points<WHOLE>(sh, pts, np, n1, n2, h3, dx1, dx2, dx3, false, hit,
+                    [&](long o, int i1, int i2, int i3, int k0, int nl) {
     const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
     const long of = i1 + ld * (i2 + (long)n2 * i3), ot = i1 + ld * i2;
     float f1, f2, f3, t1, t2, t3;
     bool any = false;
     for (int l = 0; l < nl; ++l) {
-      const int k = k0 + sh.list[l];
+      const int k = src_at<WHOLE>(sh, k0, l);
       const PlaneDev& p = P[k];
       const double wl = fmax(p.Lp, p.Wp);
       if ((fabs(x1 - p.x) > wl) || (fabs(x2 - p.y) > wl)) continue;
@@ -1591,7 +1634,7 @@ __global__ __launch_bounds__(256) void k_source(const PlaneDev* __restrict__ P, 
 int launch_source(const PlaneDev* P, const double* slip, int np, double mu, int n1, int n2, int h3, double dx1,
                   double dx2, double dx3, Field3 f, long ld, float* t, long ts, hipStream_t st) {
   const long N = (long)n1 * n2 * h3;
-  k_source<<<src_blocks(N), 256, 0, st>>>(P, slip, np, mu, n1, n2, h3, dx1, dx2, dx3, f, ld, t, ts);
+  SRC_LAUNCH(k_source, N, np, st, P, slip, np, mu, n1, n2, h3, dx1, dx2, dx3, f, ld, t, ts);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 
@@ -1599,7 +1642,8 @@ int launch_source(const PlaneDev* P, const double* slip, int np, double mu, int 
 // depth (x3 from the shifted coordinates, so that the images above the
 // surface land in the lower half of the grid), the cracks added in their
 // order with one rounding each
-__global__ __launch_bounds__(256) void k_tensile_source(const PlaneDev* __restrict__ P,
+template <bool WHOLE>
+__global__ __launch_bounds__(256) void k_tensile_source(int pts, const PlaneDev* __restrict__ P,
                                                         const double* __restrict__ opening, int np, double lambda,
                                                         double mu, int n1, int n2, int n3, double dx1, double dx2,
                                                         double dx3, Field3 f, long ld) {
@@ -1610,13 +1654,14 @@ __global__ __launch_bounds__(256) void k_tensile_source(const PlaneDev* __restri
                       (src_reach(B.za, B.zb, p.z, p.Lp) || src_reach(B.za, B.zb, -p.z, p.Lp)),
                   p.x, p.Wp};
   };
-  src_points(sh, np, n1, n2, n3, dx1, dx2, dx3, true, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+  src_points<WHOLE>(sh, pts, np, n1, n2, n3, dx1, dx2, dx3, true, hit,
+                    [&](long o, int i1, int i2, int i3, int k0, int nl) {
     const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = d_shifted(i3, n3, dx3);
     const long of = i1 + ld * (i2 + (long)n2 * i3);
     float f1, f2, f3;
     bool any = false;
     for (int l = 0; l < nl; ++l) {
-      const int k = k0 + sh.list[l];
+      const int k = src_at<WHOLE>(sh, k0, l);
       const PlaneDev& p = P[k];
       if ((fabs(x3 - p.z) > p.Lp) && (fabs(x3 + p.z) > p.Lp)) continue;
       if ((fabs(x1 - p.x) > p.Wp) || (fabs(x2 - p.y) > p.Wp)) continue;
@@ -1649,8 +1694,9 @@ __global__ __launch_bounds__(256) void k_tensile_source(const PlaneDev* __restri
 
 // mogisource, elastic3d.f90:2458-2509: point dilatation sources (volume
 // change in slip) and their images over the full depth
-__global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __restrict__ M, int nm, double lambda,
-                                                     double mu, int n1, int n2, int n3, double dx1, double dx2,
+template <bool WHOLE>
+__global__ __launch_bounds__(256) void k_mogi_source(int pts, const relax_source_t* __restrict__ M, int nm,
+                                                     double lambda, double mu, int n1, int n2, int n3, double dx1, double dx2,
                                                      double dx3, Field3 f, long ld) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
@@ -1660,7 +1706,8 @@ __global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __res
                       (src_reach(B.za, B.zb, s.z, r) || src_reach(B.za, B.zb, -s.z, r)),
                   s.x, r};
   };
-  src_points(sh, nm, n1, n2, n3, dx1, dx2, dx3, true, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+  src_points<WHOLE>(sh, pts, nm, n1, n2, n3, dx1, dx2, dx3, true, hit,
+                    [&](long o, int i1, int i2, int i3, int k0, int nl) {
     // a source at the surface and its image cancel exactly in f3
 #pragma clang fp contract(off)
     const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = d_shifted(i3, n3, dx3);
@@ -1669,7 +1716,7 @@ __global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __res
     float f1, f2, f3;
     bool any = false;
     for (int l = 0; l < nl; ++l) {
-      const int k = k0 + sh.list[l];
+      const int k = src_at<WHOLE>(sh, k0, l);
       const relax_source_t& s = M[k];
       if ((fabs(x3 - s.z) > Lp) && (fabs(x3 + s.z) > Lp)) continue;
       if ((fabs(x1 - s.x) > Wp) || (fabs(x2 - s.y) > Wp)) continue;
@@ -1693,7 +1740,8 @@ __global__ __launch_bounds__(256) void k_mogi_source(const relax_source_t* __res
 
 // momentdensitytensile, elastic3d.f90:3137-3215: Hooke's law of
 // n sdyad (opening n), n carrying the aperture; each crack adds in turn
-__global__ __launch_bounds__(256) void k_add_tensile(const PlaneDev* __restrict__ P,
+template <bool WHOLE>
+__global__ __launch_bounds__(256) void k_add_tensile(int pts, const PlaneDev* __restrict__ P,
                                                      const double* __restrict__ opening, int np, double lambda,
                                                      double mu, int n1, int n2, int h3, double dx1, double dx2,
                                                      double dx3, float* sig, long H) {
@@ -1702,13 +1750,14 @@ __global__ __launch_bounds__(256) void k_add_tensile(const PlaneDev* __restrict_
     const PlaneDev& p = P[k];
     return SrcHit{src_reach(B.ya, B.yb, p.y, p.Wp) && src_reach(B.za, B.zb, p.z, p.Lp), p.x, p.Wp};
   };
-  src_points(sh, np, n1, n2, h3, dx1, dx2, dx3, false, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+  src_points<WHOLE>(sh, pts, np, n1, n2, h3, dx1, dx2, dx3, false, hit,
+                    [&](long o, int i1, int i2, int i3, int k0, int nl) {
     const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
     const float m2 = (float)(2.0 * mu);
     float acc[6];
     bool any = false;
     for (int l = 0; l < nl; ++l) {
-      const int k = k0 + sh.list[l];
+      const int k = src_at<WHOLE>(sh, k0, l);
       const PlaneDev& p = P[k];
       if (fabs(x3 - p.z) > p.Lp) continue;
       if ((fabs(x1 - p.x) > p.Wp) || (fabs(x2 - p.y) > p.Wp)) continue;
@@ -1742,8 +1791,9 @@ __global__ __launch_bounds__(256) void k_add_tensile(const PlaneDev* __restrict_
 }
 
 // momentdensitymogi, elastic3d.f90:3240-3286: kappa o G on the diagonal
-__global__ __launch_bounds__(256) void k_add_mogi(const relax_source_t* __restrict__ M, int nm, double lambda, double mu,
-                                                  int n1, int n2, int h3, double dx1, double dx2, double dx3,
+template <bool WHOLE>
+__global__ __launch_bounds__(256) void k_add_mogi(int pts, const relax_source_t* __restrict__ M, int nm, double lambda,
+                                                  double mu, int n1, int n2, int h3, double dx1, double dx2, double dx3,
                                                   float* sig, long H) {
   __shared__ SrcShared sh;
   const auto hit = [&](const SrcBox& B, int k) {
@@ -1751,14 +1801,15 @@ __global__ __launch_bounds__(256) void k_add_mogi(const relax_source_t* __restri
     const double r = 6.0 * fmax(dx1, fmax(dx2, dx3));
     return SrcHit{src_reach(B.ya, B.yb, s.y, r) && src_reach(B.za, B.zb, s.z, r), s.x, r};
   };
-  src_points(sh, nm, n1, n2, h3, dx1, dx2, dx3, false, hit, [&](long o, int i1, int i2, int i3, int k0, int nl) {
+  src_points<WHOLE>(sh, pts, nm, n1, n2, h3, dx1, dx2, dx3, false, hit,
+                    [&](long o, int i1, int i2, int i3, int k0, int nl) {
     const double x1 = d_shifted(i1, n1, dx1), x2 = d_shifted(i2, n2, dx2), x3 = (double)i3 * dx3;
     const double kappa = lambda + 2.0 / 3.0 * mu;
     const double Wp = 6.0 * fmax(dx1, fmax(dx2, dx3)), Lp = Wp;
     float a11 = 0.f, a22 = 0.f, a33 = 0.f;
     bool any = false;
     for (int l = 0; l < nl; ++l) {
-      const int k = k0 + sh.list[l];
+      const int k = src_at<WHOLE>(sh, k0, l);
       const relax_source_t& s = M[k];
       if (fabs(x3 - s.z) > Lp) continue;
       if ((fabs(x1 - s.x) > Wp) || (fabs(x2 - s.y) > Wp)) continue;
@@ -1775,24 +1826,24 @@ __global__ __launch_bounds__(256) void k_add_mogi(const relax_source_t* __restri
 
 int launch_tensile_source(const PlaneDev* P, const double* opening, int np, double lambda, double mu, int n1, int n2,
                           int n3, double dx1, double dx2, double dx3, Field3 f, long ld, hipStream_t st) {
-  k_tensile_source<<<src_blocks((long)n1 * n2 * n3), 256, 0, st>>>(P, opening, np, lambda, mu, n1, n2, n3, dx1, dx2,
-                                                                  dx3, f, ld);
+  SRC_LAUNCH(k_tensile_source, (long)n1 * n2 * n3, np, st, P, opening, np, lambda, mu, n1, n2, n3, dx1, dx2, dx3, f,
+             ld);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 int launch_mogi_source(const relax_source_t* M, int nm, double lambda, double mu, int n1, int n2, int n3,
                        double dx1, double dx2, double dx3, Field3 f, long ld, hipStream_t st) {
-  k_mogi_source<<<src_blocks((long)n1 * n2 * n3), 256, 0, st>>>(M, nm, lambda, mu, n1, n2, n3, dx1, dx2, dx3, f, ld);
+  SRC_LAUNCH(k_mogi_source, (long)n1 * n2 * n3, nm, st, M, nm, lambda, mu, n1, n2, n3, dx1, dx2, dx3, f, ld);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 int launch_add_tensile(const PlaneDev* P, const double* opening, int np, double lambda, double mu, int n1, int n2,
                        int h3, double dx1, double dx2, double dx3, float* sig, long H, hipStream_t st) {
-  k_add_tensile<<<src_blocks((long)n1 * n2 * h3), 256, 0, st>>>(P, opening, np, lambda, mu, n1, n2, h3, dx1, dx2, dx3,
-                                                               sig, H);
+  SRC_LAUNCH(k_add_tensile, (long)n1 * n2 * h3, np, st, P, opening, np, lambda, mu, n1, n2, h3, dx1, dx2, dx3, sig,
+             H);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 int launch_add_mogi(const relax_source_t* M, int nm, double lambda, double mu, int n1, int n2, int h3, double dx1,
                     double dx2, double dx3, float* sig, long H, hipStream_t st) {
-  k_add_mogi<<<src_blocks((long)n1 * n2 * h3), 256, 0, st>>>(M, nm, lambda, mu, n1, n2, h3, dx1, dx2, dx3, sig, H);
+  SRC_LAUNCH(k_add_mogi, (long)n1 * n2 * h3, nm, st, M, nm, lambda, mu, n1, n2, h3, dx1, dx2, dx3, sig, H);
   return hipGetLastError() == hipSuccess ? RELAX_OK : RELAX_ERR_HIP;
 }
 
@@ -2025,8 +2076,8 @@ int relax_model_set_interseismic(relax_model_t* m, const relax_event_t* ev) {
   if ((rc = stage_planes(m, amp.data()))) return rc;
   const double dx1 = m->desc.dx1, dx2 = m->desc.dx2, dx3 = m->desc.dx3;
   if (ns) {
-    k_add_shear<<<src_blocks(H), 256, 0, m->stream>>>(m->shear_dev, m->shear_slip, ns, 2.0f * (float)m->desc.mu, g,
-                                                   dx1, dx2, dx3, m->mi);
+    SRC_LAUNCH(k_add_shear, H, ns, m->stream, m->shear_dev, m->shear_slip, ns, 2.0f * (float)m->desc.mu, g, dx1, dx2,
+               dx3, m->mi);
     if (hipGetLastError() != hipSuccess) return RELAX_ERR_HIP;
   }
   if (nt && (rc = launch_add_tensile(m->shear_dev + ns, m->shear_slip + ns, nt, m->desc.lambda, m->desc.mu, g.n1,
