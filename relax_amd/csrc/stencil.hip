@@ -571,40 +571,41 @@ __device__ __forceinline__ void stress_block(const Grid& g, const RheoParams& R,
   if (status) atomicMax(&sc->status, status);
 }
 
-// The points in the creep bands among blocks [b0, b1) (at most SEGS) of 256:
-// a point with the creep code costs ten viscous ones and the bands hold a few
+// The points in the creep bands among the SEGS blocks of 256 from b0: a point
+// with the creep code costs ten viscous ones and the bands often hold a few
 // points of every block they cross, so the workgroup first gathers the points
 // of its blocks (in address order: the sums keep one order), then takes them
-// 256 at a time: at 256x256x128 with a plane of 38x16 km 21 us (corrector)
-// beside 99 us for the other points, against 155 us for one kernel with the
+// 256 at a time.  At 256x256x128 with a plane of 38x16 km 22 us (corrector)
+// beside 100 us for the other points, against 155 us for one kernel with the
 // creep code and 49 us for a band launch without the gathering.  Their sums
 // are added to those that the launch over the other points left in entry b0.
-constexpr int SEGS = 16;
-// Blocks that a workgroup gathers: MIN_SEGS to SEGS, a power of two that divides
-// the grid's blocks (64 at least).  Between them 4096 groups, of which the
-// bands cross a few hundred: a step of 256x256x128 takes 704 us with groups of
-// 4, 709 with 8, 724 with 16; eight models of 64^3 in a batch 362 us with 4, 375
-// with 2, 381 with 1.  It hangs on the grid alone: the sums of power and C:E^i
-// are formed in one order whether a model is stepped by itself or in a batch.
-constexpr int MIN_SEGS = 4;
-__host__ __device__ __forceinline__ int band_segs(const Grid& g) {
-  const int s = (int)(g.H / 256 / 4096);
-  return s < MIN_SEGS ? MIN_SEGS : s > SEGS ? SEGS : s;
+// The number of blocks is one for all launches, so power and C:E^i are summed
+// in one order whether a model is stepped by itself or in a batch.  Two: with
+// planes along x1, whose blocks lie in the band whole, larger groups leave
+// most of the chip idle (a vertical plane through 256x256x256, step: 1.39 ms,
+// 4 blocks 1.72), with one block small batches lose (8 x 64^3: 367 us, 381).
+constexpr int SEGS = 2;
+// Group i of a launch, rotated by one per plane of the grid: the rows of a
+// plane that a band crosses lie together and in the same place for a vertical
+// fault, and workgroups go to the eight XCDs in turn; rotated, every XCD gets
+// its share (a vertical plane through 128x128x256, step: 638 -> 550 us).
+__device__ __forceinline__ int band_group(int i, const Grid& g) {
+  const int P = g.n1 * g.n2 / (256 * SEGS), p = i / P;
+  return p * P + (i + p) % P;
 }
 template <int MODE, bool EXT>
 __device__ __forceinline__ void stress_band(const Grid& g, const RheoParams& R, const StencilConst& S,
                                             const float* __restrict__ X, float* __restrict__ sig,
                                             float* __restrict__ tau, float* __restrict__ gam, float* __restrict__ E,
                                             float* __restrict__ Em, StepScalars* sc, double2* __restrict__ partials,
-                                            int b0, int b1) {
+                                            int b0) {
   __shared__ unsigned short q[SEGS * 256];
   __shared__ unsigned long long mask[SEGS * 4];
-  __shared__ int base[SEGS * 4 + 1];
+  __shared__ int base[65];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l1 = __builtin_ctz((unsigned)g.n1), l2 = __builtin_ctz((unsigned)g.n2);
   if (!R.fr.active || (((long)b0 * 256) >> (l1 + l2)) >= R.fr.zmax) return;
-  const int ns = b1 - b0;
-  for (int s = 0; s < ns; ++s) {
+  for (int s = 0; s < SEGS; ++s) {
     const long o = (long)(b0 + s) * 256 + tid;
     const bool in = in_band(R, (int)(o & (g.n1 - 1)), (int)((o >> l1) & (g.n2 - 1)), (int)(o >> (l1 + l2)));
     const unsigned long long m = __ballot(in);
@@ -612,7 +613,7 @@ __device__ __forceinline__ void stress_band(const Grid& g, const RheoParams& R, 
   }
   __syncthreads();
   if (wave == 0) {
-    int c = lane < 4 * ns ? __popcll(mask[lane]) : 0, t = c;
+    int c = lane < 4 * SEGS ? __popcll(mask[lane]) : 0, t = c;
     for (int off = 1; off < 64; off <<= 1) {
       const int v = __shfl_up(t, off);
       if (lane >= off) t += v;
@@ -623,7 +624,7 @@ __device__ __forceinline__ void stress_band(const Grid& g, const RheoParams& R, 
   __syncthreads();
   const int n = base[64];
   if (n == 0) return;
-  for (int s = 0; s < ns; ++s) {
+  for (int s = 0; s < SEGS; ++s) {
     const unsigned long long m = mask[4 * s + wave];
     if ((m >> lane) & 1)
       q[base[4 * s + wave] + __popcll(m & ((1ull << lane) - 1))] = (unsigned short)(256 * s + tid);
@@ -666,15 +667,13 @@ __global__ __launch_bounds__(256) void k_stress(Grid g, ModelDev Dv, const Model
                          D.partials, blk);
 }
 
-// segs blocks of 256 points per workgroup
+// SEGS blocks of 256 points per workgroup
 template <int MODE, bool EXT, bool BATCH>
 __global__ __launch_bounds__(256) void k_stress_band(Grid g, ModelDev Dv, const ModelDev* __restrict__ md,
-                                                    StencilConst S, int segs) {
+                                                    StencilConst S) {
   const ModelDev& D = BATCH ? md[blockIdx.y] : Dv;
-  const int b0 = blockIdx.x * segs, nb = (int)(g.H / 256);
-  if (b0 >= nb) return;
   stress_band<MODE, EXT>(g, D.R, S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em, D.sc, D.partials,
-                         b0, min(b0 + segs, nb));
+                         SEGS * band_group(blockIdx.x, g));
 }
 
 // ---------------------------------------------- models of uneven grids ----
@@ -709,19 +708,15 @@ __global__ __launch_bounds__(256) void k_stress_list(const ModelDev* __restrict_
   }
 }
 
-// MIN_SEGS items per workgroup, all of one model (its items are a multiple of
-// 64); a group of band_segs blocks goes to the workgroup that holds its first
+// SEGS items per workgroup, all of one model (its items are a multiple of 64)
 template <int MODE, bool EXT>
 __global__ __launch_bounds__(256) void k_stress_band_list(const ModelDev* __restrict__ md,
                                                           const WorkItem* __restrict__ wl, int nm) {
-  const long item = (long)blockIdx.x * MIN_SEGS;
-  if (item >= wl[nm].first) return;
+  const long item = (long)blockIdx.x * SEGS;
   const int m = work_model(wl, nm, item);
-  const int segs = band_segs(wl[m].g), b0 = (int)(item - wl[m].first);
-  if (b0 % segs) return;
   const ModelDev& D = md[m];
   stress_band<MODE, EXT>(wl[m].g, D.R, wl[m].S, MODE == STRESS_PRED ? D.W : D.u, D.sig, D.tau, D.gam, D.E, D.Em, D.sc,
-                         D.partials, b0, b0 + segs);
+                         D.partials, SEGS * band_group((int)(item - wl[m].first) / SEGS, wl[m].g));
 }
 
 template <int TXB, int TYB, bool TM, bool RAW, bool EXT, int PART, int BTY, bool ZR>
@@ -819,13 +814,15 @@ static int tiles_of(int x0, int nx, int n, int T, int* t0) {
   return std::min(c, nt);
 }
 // Creeping planes: the points outside the bands on the tiles of the variant;
-// then the bands, on the same tiles in chunks of a few planes.  A tile's band
-// is some 20 planes deep and its points cost ten times a viscous one, so the
-// bands want many short chunks (2 planes, more where that made over 2048
-// workgroups), of the tiles in the bands' box only: at 256x256x128 with a
-// plane of 38x16 km the bands take 22-23 us beside 47-49 us (64x16) or 60 us
-// (32x16) for the rest, against 142 us for one kernel with the creep code over
-// all points.  The 64x16 tiles' bands go to 64x8 ones (at 1024 threads the
+// then the bands, on the same tiles in chunks of a few planes, of the tiles in
+// the bands' box only.  A tile's band is often some 20 planes deep and its
+// points cost ten times a viscous one, so the bands want many short chunks:
+// from 2 planes, up to 8 while that makes over 1024 workgroups, deeper over
+// 2048 (four planes across 128x128x256, step: 1.07 ms, 1.20 with chunks of 2;
+// a flat plane under 512x512x64 1.55, 1.73 with chunks of 16).  At 256x256x128
+// with a plane of 38x16 km the bands take 22-23 us beside 47-49 us (64x16) or
+// 60 us (32x16) for the rest, against 142 us for one kernel with the creep code
+// over all points.  The 64x16 tiles' bands go to 64x8 ones (at 1024 threads the
 // creep code spills 40-137 registers).
 template <int TX, int TY, bool ZR, bool EXT>
 static void body_parts(const BodyLaunch& b, int rclass, int zc, int gz) {
@@ -848,7 +845,7 @@ static void body_parts(const BodyLaunch& b, int rclass, int zc, int gz) {
   }
   const long tiles = (long)box.nx * box.ny * b.nm;
   int zi = 2;
-  while (zi < b.g.h3 && tiles * ((depth + zi - 1) / zi) > 2048) zi *= 2;
+  while (zi < b.g.h3 && tiles * ((depth + zi - 1) / zi) > (zi < 8 ? 1024 : 2048)) zi *= 2;
   body_mode<TX, IY, ZR, EXT, PART_IN, TY>(b, zi, (depth + zi - 1) / zi, box);
 }
 
@@ -888,10 +885,10 @@ int launch_stress(int mode, const Grid& g, const StencilConst& S, const ModelDev
   const ModelDev Dv = batch ? ModelDev{} : *one;
   if (rclass < RHEO_VISCOUS || rclass > RHEO_ALL) return RELAX_ERR_ARG;
   const dim3 grid((unsigned)stress_blocks(g), (unsigned)nm);
-  // the creep bands' part: no deeper than they reach
-  const long nin = batch ? stress_blocks(g) : std::min(stress_blocks(g), ((long)g.n1 * g.n2 * Dv.R.fr.zmax + 255) / 256);
-  const int segs = band_segs(g);
-  const dim3 gin((unsigned)std::max(1L, (nin + segs - 1) / segs), (unsigned)nm);
+  // the creep bands' part: no deeper than they reach (whole planes, of at
+  // least four blocks each)
+  const long planes = batch ? g.h3 : Dv.R.fr.zmax;
+  const dim3 gin((unsigned)std::max(1L, planes * (g.n1 * g.n2 / (256 * SEGS))), (unsigned)nm);
 #define K(MODE, E, PART, GR)                                                     \
   {                                                                              \
     if (batch) k_stress<MODE, E, PART, true><<<GR, 256, 0, st>>>(g, Dv, md, S);  \
@@ -902,8 +899,8 @@ int launch_stress(int mode, const Grid& g, const StencilConst& S, const ModelDev
     if (!(rclass & RHEO_CREEP)) K(MODE, E, PART_ALL, grid)                   \
     else {                                                                   \
       K(MODE, E, PART_OUT, grid)                                             \
-      if (batch) k_stress_band<MODE, E, true><<<gin, 256, 0, st>>>(g, Dv, md, S, segs); \
-      else k_stress_band<MODE, E, false><<<gin, 256, 0, st>>>(g, Dv, md, S, segs);      \
+      if (batch) k_stress_band<MODE, E, true><<<gin, 256, 0, st>>>(g, Dv, md, S); \
+      else k_stress_band<MODE, E, false><<<gin, 256, 0, st>>>(g, Dv, md, S);      \
     }                                                                        \
   }
 #define KM(MODE)                          \
@@ -989,7 +986,7 @@ int launch_stress_list(int mode, const WorkItem* wl, const ModelDev* md, int nm,
     if (!(rclass & RHEO_CREEP)) { K(MODE, E, PART_ALL) }       \
     else {                                                     \
       K(MODE, E, PART_OUT)                                     \
-      k_stress_band_list<MODE, E><<<(unsigned)((total + MIN_SEGS - 1) / MIN_SEGS), 256, 0, st>>>(md, wl, nm); \
+      k_stress_band_list<MODE, E><<<(unsigned)(total / SEGS), 256, 0, st>>>(md, wl, nm); \
     }                                                          \
   }
 #define KM(MODE)                          \
